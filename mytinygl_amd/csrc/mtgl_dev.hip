@@ -4006,29 +4006,59 @@ __global__ void __launch_bounds__(256) k_clear_span(uint32_t *color, float *dept
     }
 }
 
-// glReadPixels packing (reference src/gl_api.c:1180-1229), one thread per
-// output pixel of the band of window rows [r0, r0 + nrows): window row r is
-// framebuffer row fb_h - 1 - (y + r); rows outside the framebuffer are zero
-// bytes, columns outside it in rows that exist read as (0, 0, 0, 255).  bpp 4
-// stores the packed pixel (its bytes are r, g, b, a in memory), bpp 3 the
-// first three bytes.
+// Readback packing (glReadPixels, reference src/gl_api.c:1180-1229, and
+// present): output pixel i of a w-pixel-wide window is window row r0 + i / w,
+// column i % w, tightly packed.  flip: window rows count up from the bottom
+// row (framebuffer row fb_h - 1 - (y + r)); else they are framebuffer rows.
+// Rows outside the framebuffer are zero bytes, columns outside it in rows
+// that exist read as (0, 0, 0, 255).  A thread takes four consecutive pixels
+// and stores 16 bytes (BPP 4) or 12 (BPP 3), so that a wave stores whole
+// cache lines (out is 16-byte aligned for BPP 4, 4-byte for BPP 3): out is
+// device memory, or the caller's own pinned memory over PCIe, which bounds
+// the kernel then.  poison (null: not wanted) receives the Exec's poison in
+// pinned host memory, so that the wait for the pixels also tells the host
+// whether the queued work took effect; no pixel is stored when it did not.
+template <int BPP>
 __global__ void __launch_bounds__(256) k_read_pixels(const uint32_t *color, int32_t fb_w, int32_t fb_h, int32_t x,
-                                                     int32_t y, int32_t w, int32_t r0, int32_t nrows, int32_t bpp,
-                                                     uint8_t *out)
+                                                     int32_t y, int32_t flip, uint32_t w, int32_t r0, uint64_t n,
+                                                     uint8_t *out, const Counters *ctr, uint32_t *poison)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)w * (uint64_t)nrows) return;
-    const int64_t r = r0 + (int64_t)(i / (uint64_t)w), col = (int64_t)(i % (uint64_t)w);
-    const int64_t fy = (int64_t)fb_h - 1 - ((int64_t)y + r), sx = (int64_t)x + col;
-    uint32_t p = 0u;
-    if (fy >= 0 && fy < fb_h) p = (sx >= 0 && sx < fb_w) ? color[fy * fb_w + sx] : 0xFF000000u;
-    if (bpp == 4) {
-        reinterpret_cast<uint32_t *>(out)[i] = p;
-    } else {
-        out[3 * i + 0] = (uint8_t)(p & 0xFFu);
-        out[3 * i + 1] = (uint8_t)((p >> 8) & 0xFFu);
-        out[3 * i + 2] = (uint8_t)((p >> 16) & 0xFFu);
+    static_assert(BPP == 3 || BPP == 4, "GL_RGB or GL_RGBA");
+    if (poison) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *poison = ctr->poison;
+        if (exec_poisoned(ctr)) return;
     }
+    const uint64_t i = 4ull * ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= n) return;
+    uint64_t row = n <= 0xFFFFFFFFull ? (uint64_t)((uint32_t)i / w) : i / w;
+    uint32_t col = (uint32_t)(i - row * w);
+    uint32_t p[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int64_t r = (int64_t)y + r0 + (int64_t)row, fy = flip ? (int64_t)fb_h - 1 - r : r;
+        const int64_t sx = (int64_t)x + col;
+        p[k] = 0u;
+        if (i + k < n && fy >= 0 && fy < fb_h) p[k] = (sx >= 0 && sx < fb_w) ? color[fy * fb_w + sx] : 0xFF000000u;
+        if (++col == w) {
+            col = 0;
+            row++;
+        }
+    }
+    if (i + 4 <= n) {
+        if (BPP == 4) {
+            *reinterpret_cast<uint4 *>(out + 4 * i) = make_uint4(p[0], p[1], p[2], p[3]);
+        } else {
+            uint32_t *o = reinterpret_cast<uint32_t *>(out + 3 * i);
+            o[0] = (p[0] & 0xFFFFFFu) | (p[1] << 24);
+            o[1] = ((p[1] >> 8) & 0xFFFFu) | (p[2] << 16);
+            o[2] = ((p[2] >> 16) & 0xFFu) | (p[3] << 8);
+        }
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        if (i + k < n)
+            for (int c = 0; c < BPP; c++) out[BPP * (i + k) + c] = (uint8_t)(p[k] >> (8 * c));
 }
 
 __global__ void __launch_bounds__(256) k_mip1(const uint32_t *src, int32_t w, uint32_t *dst, int32_t mw, int32_t mh)
@@ -4476,6 +4506,7 @@ struct Exec {
     uint32_t resident[8] = {256, 256, 256, 256, 256, 256, 256, 256};
     Counters *ctr = nullptr;                       // device
     Counters *ctr_host = nullptr;                  // pinned mirror for readback
+    uint32_t *report = nullptr;                    // pinned: the poison the latest read reported
     uint8_t *pinned = nullptr;                     // staging for uploads that wait for their copy
     size_t pinned_cap = 0;
     // staging of launch tables and staged arrays: blocks taken in order and
@@ -4819,6 +4850,8 @@ int exec_init(Exec &x, int device)
     HIPC(hipMalloc((void **)&x.ctr, sizeof(Counters)));
     HIPC(hipMalloc((void **)&x.stat_slots, 2 * STAT_SLOTS * sizeof(unsigned long long)));
     HIPC(hipHostMalloc((void **)&x.ctr_host, sizeof(Counters), hipHostMallocDefault));
+    HIPC(hipHostMalloc((void **)&x.report, 256, hipHostMallocDefault));
+    *x.report = 0u;
     HIPC(hipEventCreateWithFlags(&x.upload_done, hipEventDisableTiming));
     HIPC(hipMemsetAsync(x.stat_slots, 0, 2 * STAT_SLOTS * sizeof(unsigned long long), x.stream));
     HIPC(hipMemsetAsync(x.ctr, 0, sizeof(Counters), x.stream));
@@ -4843,6 +4876,7 @@ void exec_free(Exec &x)
     if (x.ctr) (void)hipFree(x.ctr);
     if (x.stat_slots) (void)hipFree(x.stat_slots);
     if (x.ctr_host) (void)hipHostFree(x.ctr_host);
+    if (x.report) (void)hipHostFree(x.report);
     if (x.pinned) (void)hipHostFree(x.pinned);
     for (auto &b : x.ring) (void)hipHostFree(b.first);
     x.ring.clear();
@@ -4852,6 +4886,7 @@ void exec_free(Exec &x)
     x.ctr = nullptr;
     x.stat_slots = nullptr;
     x.ctr_host = nullptr;
+    x.report = nullptr;
     x.pinned = nullptr;
     x.upload_done = nullptr;
     x.stream = nullptr;
@@ -5732,7 +5767,12 @@ void invalidate_batches(mtgl_dev *d)
 int dev_join(mtgl_dev *d)
 {
     if (d->pending) {
-        HIPC(hipStreamWaitEvent(d->ex.stream, d->pending->done, 0));
+        // (a launch that has ended needs no wait on the stream: reads of many
+        // contexts after one launch then cost no barrier each)
+        if (hipEventQuery(d->pending->done) != hipSuccess) {
+            (void)hipGetLastError();
+            HIPC(hipStreamWaitEvent(d->ex.stream, d->pending->done, 0));
+        }
         d->pending = nullptr;
     }
     return MTGL_OK;
@@ -6204,9 +6244,74 @@ MTGL_API int mtgl_dev_read(mtgl_dev *d, uint32_t which, int32_t x, int32_t y, in
     return MTGL_OK;
 }
 
-// Packed on the device in bands of rows that fit READBACK_BAND bytes (one row
-// at least), each copied to the caller's memory as soon as it is packed.
+// The device's address of host memory [p, p + bytes) when all of it is
+// pinned and mapped for the current device (hipHostMalloc or registered by
+// the caller), else null: a kernel can then write it.
+static uint8_t *mapped_host(void *p, size_t bytes)
+{
+    hipPointerAttribute_t a, b;
+    uint8_t *const last = (uint8_t *)p + bytes - 1;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipPointerGetAttributes(&b, last) != hipSuccess) {
+        (void)hipGetLastError();   // (memory the runtime does not know)
+        return nullptr;
+    }
+    if (a.type != hipMemoryTypeHost || b.type != hipMemoryTypeHost || !a.devicePointer || !b.devicePointer) return nullptr;
+    if ((uint8_t *)b.devicePointer - (uint8_t *)a.devicePointer != (ptrdiff_t)(bytes - 1)) return nullptr;
+    return (uint8_t *)a.devicePointer;
+}
+
+// A tightly packed window of the colour plane to host memory (k_read_pixels'
+// arguments), after the queued work.  Pinned memory (16-byte aligned for
+// RGBA, 4 for RGB) is written by the kernel itself, queued behind that work:
+// one launch and one wait for the counters, the packing and the copy, which
+// took three operations and two waits (a 640x480 frame 144 to 111 us, a
+// 1080p one 345 to 322; a copy queued after the packing kernel instead gave
+// 128 and 346, its engine waiting for the kernel's).  When the kernel reports
+// that a queued launch overflowed, the log runs again (confirm) and the
+// window is read once more.  Other memory gets the packed pixels in bands of
+// rows that fit READBACK_BAND bytes (one row at least), each copied as soon
+// as it is packed.
 constexpr size_t READBACK_BAND = 64u << 20;
+
+static int read_window(mtgl_dev *d, int32_t x, int32_t y, int32_t flip, int32_t width, int32_t height, int bpp,
+                       void *dst)
+{
+    Exec &ex = d->ex;
+    int rc = dev_join(d);
+    if (rc) return rc;
+    const size_t row_bytes = (size_t)width * (size_t)bpp;
+    auto launch = [&](int32_t r0, uint64_t n, uint8_t *out, uint32_t *poison) {
+        hipLaunchKernelGGL(bpp == 4 ? k_read_pixels<4> : k_read_pixels<3>, dim3((uint32_t)blocks_for((n + 3) / 4, 256)),
+                           dim3(256), 0, ex.stream, d->color, d->w, d->h, x, y, flip, (uint32_t)width, r0, n, out,
+                           (const Counters *)ex.ctr, poison);
+        return hipGetLastError();
+    };
+    uint8_t *const host = row_bytes <= SIZE_MAX / (size_t)height ? mapped_host(dst, row_bytes * (size_t)height) : nullptr;
+    if (host && ((uintptr_t)host & (bpp == 4 ? 15u : 3u)) == 0) {
+        for (;;) {
+            const bool queued = !d->ops.empty();
+            HIPC(launch(0, (uint64_t)width * (uint64_t)height, host, queued ? ex.report : nullptr));
+            HIPC(hipStreamSynchronize(ex.stream));
+            if (!queued) return MTGL_OK;
+            if (*(volatile uint32_t *)ex.report == 0u) break;
+            if ((rc = confirm(d))) return rc;
+        }
+        d->ops.clear();   // every queued op took effect
+        ring_release(ex);
+        return MTGL_OK;
+    }
+    if ((rc = confirm(d))) return rc;
+    const int32_t band = (int32_t)std::max<size_t>(1, std::min<size_t>((size_t)height, READBACK_BAND / row_bytes));
+    if ((rc = arena_reserve(ex, d->readback, row_bytes * (size_t)band))) return rc;
+    for (int32_t r0 = 0; r0 < height; r0 += band) {
+        const int32_t nr = std::min(band, height - r0);
+        HIPC(launch(r0, (uint64_t)width * (uint64_t)nr, as<uint8_t>(d->readback), nullptr));
+        HIPC(hipMemcpyAsync((uint8_t *)dst + (size_t)r0 * row_bytes, d->readback.ptr, row_bytes * (size_t)nr,
+                            hipMemcpyDeviceToHost, ex.stream));
+    }
+    HIPC(hipStreamSynchronize(ex.stream));
+    return MTGL_OK;
+}
 
 MTGL_API int mtgl_dev_read_pixels(mtgl_dev *d, int32_t x, int32_t y, int32_t width, int32_t height, uint32_t format,
                                   void *dst)
@@ -6214,29 +6319,14 @@ MTGL_API int mtgl_dev_read_pixels(mtgl_dev *d, int32_t x, int32_t y, int32_t wid
     if (!d || !dst) return MTGL_ERR_INVALID;
     const int32_t bpp = format == GL_RGBA ? 4 : (format == GL_RGB ? 3 : 0);
     if (width <= 0 || height <= 0 || bpp == 0) return MTGL_OK;
-    int rc = dev_join(d);
-    if (rc) return rc;
-    if ((rc = confirm(d))) return rc;
-    const size_t row_bytes = (size_t)width * (size_t)bpp;
-    const int32_t band = (int32_t)std::max<size_t>(1, std::min<size_t>((size_t)height, READBACK_BAND / row_bytes));
-    if ((rc = arena_reserve(d->ex, d->readback, row_bytes * (size_t)band))) return rc;
-    uint8_t *out = (uint8_t *)dst;
-    for (int32_t r0 = 0; r0 < height; r0 += band) {
-        const int32_t nr = std::min(band, height - r0);
-        const uint64_t n = (uint64_t)width * (uint64_t)nr;
-        hipLaunchKernelGGL(k_read_pixels, dim3((uint32_t)blocks_for(n, 256)), dim3(256), 0, d->ex.stream, d->color,
-                           d->w, d->h, x, y, width, r0, nr, bpp, as<uint8_t>(d->readback));
-        HIPC(hipGetLastError());
-        HIPC(hipMemcpyAsync(out + (size_t)r0 * row_bytes, d->readback.ptr, row_bytes * (size_t)nr,
-                            hipMemcpyDeviceToHost, d->ex.stream));
-    }
-    HIPC(hipStreamSynchronize(d->ex.stream));
-    return MTGL_OK;
+    return read_window(d, x, y, 1, width, height, bpp, dst);
 }
 
 MTGL_API int mtgl_dev_present(mtgl_dev *d, void *dst, int64_t pitch)
 {
     if (!d || !dst || pitch < (int64_t)d->w * 4) return MTGL_ERR_INVALID;
+    if (pitch == (int64_t)d->w * 4 && ((uintptr_t)dst & 15u) == 0 && mapped_host(dst, (size_t)d->w * 4 * (size_t)d->h))
+        return read_window(d, 0, 0, 0, d->w, d->h, 4, dst);
     int rc = dev_join(d);
     if (rc) return rc;
     if ((rc = confirm(d))) return rc;
