@@ -10,10 +10,11 @@
 //                 screen mapping, cull, bounding box, area, per-triangle LOD
 //                 (src/raster.c:451-529, :729-958).  Writes up to 7 fan
 //                 triangles per input triangle, ordered by (triangle, fan j).
-//   K3 binner     scan of per-triangle tile counts, load-balanced expansion to
-//                 (tile, triangle) pairs in submission order, stable LSD radix
-//                 sort by tile (LDS digit histograms, wavefront ballot ranks),
-//                 segment list of non-empty tiles.
+//   K3 binner     every tile's records in submission order and the work list
+//                 of non-empty tiles: k_bin, a workgroup per square of tiles;
+//                 or, for launches it does not suit (use_bins), load-balanced
+//                 expansion to (tile, record) pairs and a stable sort by tile
+//                 (LDS digit counts, wavefront ballot ranks).
 //   K4 k_raster   persistent waves; one 8x8 tile per wave, one pixel per lane;
 //                 the pixel's colour, depth and stencil stay in registers while
 //                 the wave walks the tile's bin in submission order, applying
@@ -142,8 +143,6 @@ struct __align__(16) RCold {
 // by the launch's first kernel; the second persists across launches.
 struct Counters {
     unsigned long long npairs;    // (tile, record) pairs of the launch (the pair-count scan or k_expand)
-    unsigned int nheavy;          // work items at the front of the tile list: heavy-tile parts, medium tiles
-    unsigned int nlight;          // the other non-empty tiles (with nheavy: one 64-bit word for the list atomics)
     unsigned int unsupported;
     unsigned int noverflow;       // overflow slots requested by clipped triangles
     unsigned int overflow_full;   // bit 0: the clip pool was too small; bit 1: the pair arrays were
@@ -155,13 +154,23 @@ struct Counters {
                                   // later framebuffer write of this Exec is skipped until the host clears it
     unsigned long long poison_pairs;   // pairs that launch needed
     unsigned int poison_flags;    // its overflow_full
-    unsigned int pad1;
+    unsigned int meets;           // the latest launch's (set-up block, square it meets) pairs, capped at 2^32 - 1
     unsigned long long acc_tri_raster; // fan triangles and pairs of every launch that did not overflow
     unsigned long long acc_bin_pairs;
 };
 
-static_assert(offsetof(Counters, nheavy) % 8 == 0 && offsetof(Counters, nlight) == offsetof(Counters, nheavy) + 4,
-              "nheavy and nlight form one 64-bit word");
+// A launch's work list lies in BIN_REGIONS regions of the list's memory, each
+// with counters of its own a cache line apart: atomics on one address take 9
+// ns each, one after the other, and k_bin makes two per square (the 2,040
+// squares of a 1080p frame whose triangles lie everywhere would queue for 37
+// us).  The tile sort uses region 0 alone.
+constexpr uint32_t BIN_REGIONS = 16;
+struct __align__(128) RegionCounters {
+    unsigned int nheavy;          // work items at the front of the region: heavy-tile parts, medium tiles
+    unsigned int nlight;          // the other non-empty tiles, at its back (with nheavy: one 64-bit word for the atomics)
+    unsigned long long pairs;     // records k_bin's squares of the region have listed for their tiles
+};
+static_assert(sizeof(RegionCounters) == 128 && offsetof(RegionCounters, nlight) == 4, "RegionCounters layout");
 
 // attribute stream resolved to a device pointer
 struct DArr {
@@ -217,6 +226,8 @@ struct SetupParams {
     uint32_t *rec_base;           // first global record slot per input triangle
     unsigned long long *tri_tiles;  // (tile, record) pairs per input triangle
     uint32_t overflow_cap;        // slots of the overflow pool
+    uint2 *tbox;                  // tile bounds per input triangle (launches binned by k_bin), else null
+    uint32_t bin_side, bin_cols;  // k_bin's squares of the scene: tiles per side, squares per row
     Counters *ctr;
 };
 
@@ -255,8 +266,10 @@ struct RasterParams {
     const uint32_t *vals;          // per bin, in submission order: record slot
     const uint4 *list;             // work items (tile | part << 28, e0, e1, scene): nheavy from the front, nlight from the back
     uint32_t ntiles;
-    uint32_t list_cap;             // items the list holds (HEAVY_SPLIT per tile)
-    uint32_t part;                 // list items of this launch: 0 all, 1 the heavy ones, 2 the others
+    uint32_t list_cap;             // items one region of the list holds (HEAVY_SPLIT per tile)
+    const RegionCounters *regions;
+    uint32_t *kept, *meets;        // k_setup's 64 partial counts, for the first kernel of the stage (kept: only after
+                                   // k_bin), else null
     unsigned long long *stats;     // per block: fragments, algorithmic bytes (summed when read)
     Counters *ctr;
 };
@@ -480,12 +493,12 @@ __device__ __forceinline__ uint32_t scene_of(const uint32_t *map, uint32_t nscen
 
 // The three maps of a multi-scene launch, one block per scene: vertex block,
 // setup block and tile -> scene.
-__global__ void __launch_bounds__(256) k_scene_maps(const uint32_t *vblock_pre, const uint32_t *sblock_pre,
-                                                    const uint32_t *tile_pre, uint32_t *vmap, uint32_t *smap,
+__global__ void __launch_bounds__(256) k_scene_maps(const uint32_t *bin_pre, const uint32_t *sblock_pre,
+                                                    const uint32_t *tile_pre, uint32_t *bmap, uint32_t *smap,
                                                     uint32_t *tmap)
 {
     const uint32_t s = blockIdx.x;
-    for (uint32_t i = vblock_pre[s] + threadIdx.x; i < vblock_pre[s + 1]; i += blockDim.x) vmap[i] = s;
+    for (uint32_t i = bin_pre[s] + threadIdx.x; i < bin_pre[s + 1]; i += blockDim.x) bmap[i] = s;
     for (uint32_t i = sblock_pre[s] + threadIdx.x; i < sblock_pre[s + 1]; i += blockDim.x) smap[i] = s;
     for (uint32_t i = tile_pre[s] + threadIdx.x; i < tile_pre[s + 1]; i += blockDim.x) tmap[i] = s;
 }
@@ -819,8 +832,6 @@ __device__ __forceinline__ void perspective_divide(CV &v)
     v.x *= iw; v.y *= iw; v.z *= iw; v.w = iw;
 }
 
-// one fan triangle (c[0], c[j], c[j+1]) after the divide; returns 1 when a
-// record was written
 // The rasteriser set-up of one filled fan triangle (src/raster.c:458-529):
 // the box clamped to viewport and scissor, the area, the drop below half a
 // pixel and the per-triangle LOD, into record r; box gets the box clamped to
@@ -911,8 +922,7 @@ __device__ __forceinline__ void cold_record(const CV &A, const CV &B, const CV &
 __device__ __forceinline__ unsigned long long box_tile_mask(const int32_t *X, const int32_t *Y, float area,
                                                             int32_t minX, int32_t minY, int32_t maxX, int32_t maxY,
                                                             int32_t tx0, int32_t ty0, int32_t tw, int32_t th,
-                                                            int32_t fb_w, int32_t fb_h, int32_t lo = 0,
-                                                            int32_t hi = 64)
+                                                            int32_t fb_w, int32_t fb_h)
 {
     const float fx0 = (float)X[0], fy0 = (float)Y[0], fx1 = (float)X[1], fy1 = (float)Y[1];
     const float fx2 = (float)X[2], fy2 = (float)Y[2];
@@ -936,15 +946,14 @@ __device__ __forceinline__ unsigned long long box_tile_mask(const int32_t *X, co
         for (int e = 0; e < 3; e++) b[e] = ((dx[e] >= 0.0f ? ya : yb) - ey[e]) * dx[e];
     };
     // the box holds at most 64 tiles, so its shorter side at most 8: those
-    // terms are formed once, the longer side's once per step (the steps
-    // [lo, hi) of it)
+    // terms are formed once, the longer side's once per step
     unsigned long long m = 0ull;
     if (th <= tw) {
         float b[8][3];
 #pragma unroll
         for (int j = 0; j < 8; j++)
             if (j < th) row_b(j, b[j]);
-        for (int32_t i = lo; i < min(tw, hi); i++) {
+        for (int32_t i = 0; i < tw; i++) {
             float a[3];
             col_a(i, a);
 #pragma unroll
@@ -958,7 +967,7 @@ __device__ __forceinline__ unsigned long long box_tile_mask(const int32_t *X, co
 #pragma unroll
         for (int i = 0; i < 8; i++)
             if (i < tw) col_a(i, a[i]);
-        for (int32_t j = lo; j < min(th, hi); j++) {
+        for (int32_t j = 0; j < th; j++) {
             float b[3];
             row_b(j, b);
 #pragma unroll
@@ -971,19 +980,22 @@ __device__ __forceinline__ unsigned long long box_tile_mask(const int32_t *X, co
     return m;
 }
 
-// What box_tile_mask needs of one record, handed from the set-up wave to
-// the waves that form the mask when set-up defers it (want: a box of at
-// most BOX_MASK_TILES tiles)
-struct MaskIn {
-    int32_t X[3], Y[3];
-    float area;
-    int32_t minX, minY, maxX, maxY;
-    int32_t tx0, ty0, tw, th;
-    int32_t want;
+// Tile bounds of a triangle (or of a set-up block's triangles) for k_bin: x
+// holds the first tile column and row, y the last, 16 bits each; TBOX_LIST
+// marks a triangle whose records are rec_base .. + n_rt (a clipped one),
+// else its record is its own slot.  No records: TBOX_NONE.
+constexpr uint32_t TBOX_LIST = 0x8000u;          // (tile coordinates are below 2048)
+constexpr uint32_t TBOX_NONE_X = 0xFFFFFFFFu, TBOX_NONE_Y = 0u;
+
+struct TileBounds {
+    int32_t x0, y0, x1, y1;
 };
 
+// one fan triangle (c[0], c[j], c[j+1]) after the divide; returns 1 when a
+// record was written, with its tiles in tb (and, for launches binned by the
+// tile sort, its box in boxp and its pairs in tiles_out)
 __device__ int setup_fan(const SetupParams &P, const mtgl_raster_state *rs, const CV &A, const CV &B, const CV &C,
-                         bool cold, RTri *outp, RCold *coldp, RBox *boxp, int *tiles_out, MaskIn *defer = nullptr)
+                         bool cold, RTri *outp, RCold *coldp, TileBounds &tb, RBox *boxp, int *tiles_out)
 {
     const int32_t vx = rs->viewport[0], vy = rs->viewport[1], vw = rs->viewport[2], vh = rs->viewport[3];
     const CV *v[3] = {&A, &B, &C};
@@ -1006,47 +1018,35 @@ __device__ int setup_fan(const SetupParams &P, const mtgl_raster_state *rs, cons
     int32_t bb[4];
     if (!fan_record(rs, P.fb_w, P.fb_h, P.tex_w, P.tex_h, A, B, C, X, Y, back, r, bb)) return 0;
     *outp = r;
-    const int32_t tx0 = bb[0] / TILE, ty0 = bb[1] / TILE, tx1 = bb[2] / TILE, ty1 = bb[3] / TILE;
-    RBox bx;
-    bx.key0 = P.tile_off + (uint32_t)(ty0 * P.tiles_x + tx0);
-    bx.tw = (uint32_t)(tx1 - tx0 + 1);
-    bx.ntiles = bx.tw * (uint32_t)(ty1 - ty0 + 1);
-    bx.tiles_x = (uint32_t)P.tiles_x;
-    bx.mask = 0ull;
-    bx.masked = 0u;
-    bx.pad = 0u;
-    if (defer) {
-        // the caller has the mask formed elsewhere and completes the box
-        MaskIn &d = *defer;
-        for (int k = 0; k < 3; k++) {
-            d.X[k] = X[k];
-            d.Y[k] = Y[k];
+    tb.x0 = bb[0] / TILE;
+    tb.y0 = bb[1] / TILE;
+    tb.x1 = bb[2] / TILE;
+    tb.y1 = bb[3] / TILE;
+    if (boxp) {
+        RBox bx;
+        bx.key0 = P.tile_off + (uint32_t)(tb.y0 * P.tiles_x + tb.x0);
+        bx.tw = (uint32_t)(tb.x1 - tb.x0 + 1);
+        bx.ntiles = bx.tw * (uint32_t)(tb.y1 - tb.y0 + 1);
+        bx.tiles_x = (uint32_t)P.tiles_x;
+        bx.mask = 0ull;
+        bx.masked = 0u;
+        bx.pad = 0u;
+        if (bx.ntiles <= BOX_MASK_TILES) {
+            // the tiles of a small box the record can cover: only those get pairs
+            const unsigned long long m = box_tile_mask(X, Y, r.area, r.minX, r.minY, r.maxX, r.maxY, tb.x0, tb.y0,
+                                                       (int32_t)bx.tw, tb.y1 - tb.y0 + 1, P.fb_w, P.fb_h);
+            bx.mask = m;
+            bx.masked = 1u;
+            bx.ntiles = (uint32_t)__popcll(m);
         }
-        d.area = r.area;
-        d.minX = r.minX;
-        d.minY = r.minY;
-        d.maxX = r.maxX;
-        d.maxY = r.maxY;
-        d.tx0 = tx0;
-        d.ty0 = ty0;
-        d.tw = (int32_t)bx.tw;
-        d.th = ty1 - ty0 + 1;
-        d.want = bx.ntiles <= BOX_MASK_TILES ? 1 : 0;
-    } else if (bx.ntiles <= BOX_MASK_TILES) {
-        // the tiles of a small box the record can cover: only those get pairs
-        const unsigned long long m = box_tile_mask(X, Y, r.area, r.minX, r.minY, r.maxX, r.maxY, tx0, ty0,
-                                                   (int32_t)bx.tw, ty1 - ty0 + 1, P.fb_w, P.fb_h);
-        bx.mask = m;
-        bx.masked = 1u;
-        bx.ntiles = (uint32_t)__popcll(m);
+        *boxp = bx;
+        *tiles_out = (int)bx.ntiles;
     }
-    *boxp = bx;
     if (cold) {
         RCold q;
         cold_record(A, B, C, q);
         *coldp = q;
     }
-    *tiles_out = (int)bx.ntiles;
     return 1;
 }
 
@@ -1054,10 +1054,11 @@ __device__ int setup_fan(const SetupParams &P, const mtgl_raster_state *rs, cons
 // left, right, bottom, top; src/clipping.h:106-126), divide, fan split of
 // input triangle t into slots of the shared overflow pool.  Out of line: a
 // few triangles of a draw take it, and its vertex arrays live in scratch.
-// Returns the fan triangles kept; base gets the first slot, tiles their
-// (tile, record) pairs.
+// Returns the fan triangles kept; base gets the first slot, tb the union of
+// their tiles (when any was kept), tiles their (tile, record) pairs where the
+// tile sort bins the launch.
 __device__ __noinline__ uint32_t setup_clipped(const SetupParams &P, const mtgl_raster_state *rs, const CV &A,
-                                               const CV &B, const CV &C, bool cold, uint32_t &base,
+                                               const CV &B, const CV &C, bool cold, uint32_t &base, TileBounds &tb,
                                                unsigned long long &tiles)
 {
     CV a[MAX_CLIP], b[MAX_CLIP];
@@ -1081,12 +1082,20 @@ __device__ __noinline__ uint32_t setup_clipped(const SetupParams &P, const mtgl_
     uint32_t nout = 0;
     RTri *out = P.rt_over + base;
     RCold *cout = cold ? P.rcold_over + base : nullptr;
+    const bool boxes = P.tbox == nullptr;
     for (int k = 0; k < n; k++) perspective_divide(b[k]);
     for (int j = 1; j + 1 < n; j++) {
         int nt = 0;
         RBox q;
-        if (setup_fan(P, rs, b[0], b[j], b[j + 1], cold, out + nout, cout ? cout + nout : nullptr, &q, &nt)) {
-            P.box_over[base + nout] = q;
+        TileBounds t;
+        if (setup_fan(P, rs, b[0], b[j], b[j + 1], cold, out + nout, cout ? cout + nout : nullptr, t,
+                      boxes ? &q : nullptr, &nt)) {
+            if (boxes) P.box_over[base + nout] = q;
+            if (nout == 0) tb = t;
+            tb.x0 = min(tb.x0, t.x0);
+            tb.y0 = min(tb.y0, t.y0);
+            tb.x1 = max(tb.x1, t.x1);
+            tb.y1 = max(tb.y1, t.y1);
             nout++;
             tiles += (unsigned long long)nt;
         }
@@ -1112,29 +1121,58 @@ __device__ __forceinline__ void stage_words(void *dst, const void *src, uint32_t
     for (uint32_t k = threadIdx.x; k < bytes / 4u; k += blockDim.x) d[k] = q[k];
 }
 
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// Minimum (MAX false) or maximum of each 16-bit half over the 64 lanes, in
+// lane 63: the DPP pattern of dpp_incl_scan with the identity for lanes
+// without a source.
+template <bool MAX>
+__device__ __forceinline__ uint32_t dpp_wave_minmax_u16x2(uint32_t v)
+{
+    const int id = MAX ? 0 : -1;
+#define MINMAX16_STEP(ctrl, rm, bm)                                                                     \
+    {                                                                                                   \
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(id, (int)v, ctrl, rm, bm, false);      \
+        const u16x2 a = __builtin_bit_cast(u16x2, v), b = __builtin_bit_cast(u16x2, o);                 \
+        v = __builtin_bit_cast(uint32_t, MAX ? __builtin_elementwise_max(a, b) : __builtin_elementwise_min(a, b)); \
+    }
+    MINMAX16_STEP(0x111, 0xf, 0xf)   // row_shr:1
+    MINMAX16_STEP(0x112, 0xf, 0xf)   // row_shr:2
+    MINMAX16_STEP(0x114, 0xf, 0xe)   // row_shr:4, lanes 4..15
+    MINMAX16_STEP(0x118, 0xf, 0xc)   // row_shr:8, lanes 8..15
+    MINMAX16_STEP(0x142, 0xa, 0xf)   // row_bcast:15 into rows 1, 3
+    MINMAX16_STEP(0x143, 0xc, 0xf)   // row_bcast:31 into rows 2, 3
+#undef MINMAX16_STEP
+    return v;
+}
+
 // Set-up of every input triangle, one thread each: triangles inside every
 // frustum plane pass through the clipper unchanged (each plane re-emits the
 // vertices in order), so they are set up directly into slot t; the others go
-// through setup_clipped.  Every kept record's tiles are counted into the
-// bins.  A block takes SETUP_BLOCK triangles.  With NW = 3 waves (launches
-// of few blocks, which leave SIMDs idle) wave c runs the vertex pipeline of
-// every triangle's corner c into LDS, three SIMDs at once, then wave 0 sets
-// the triangles up; with NW = 1 (launches that fill the GPU) the one wave
-// runs all three corners itself.  MULTI draws switch vertex states per
-// vertex and read them from HBM.
-template <bool MULTI, int NW>
+// through setup_clipped.  A block takes SETUP_BLOCK triangles.  With NW = 3
+// waves (launches of few blocks, which leave SIMDs idle) wave c runs the
+// vertex pipeline of every triangle's corner c into LDS, three SIMDs at once,
+// then wave 0 sets the triangles up; with NW = 1 (launches that fill the GPU)
+// the one wave runs all three corners itself.  MULTI draws switch vertex
+// states per vertex and read them from HBM.  BIN: k_bin follows, which reads
+// each triangle's tile bounds (tbox) and their union per block (blk_box); the
+// tile masks are then k_bin's, and only the launches of the tile sort write a
+// box and a pair count per triangle and the counts per block.  sums: 64
+// partial counts of the kept fan triangles (BIN), then 64 of the squares of
+// bin_side tiles that the blocks' bounds meet, which tell the host how far a
+// block's triangles lie apart (use_bins).
+template <bool MULTI, int NW, bool BIN>
 __global__ void __launch_bounds__(NW * SETUP_BLOCK) k_setup(const SetupParams *Ss, const VertexParams *Vs,
                                                             const uint32_t *block_pre, const uint32_t *block_scene,
                                                             uint32_t nscenes, uint32_t *blk_kept,
-                                                            unsigned long long *blk_pairs,
+                                                            unsigned long long *blk_pairs, uint2 *blk_box,
+                                                            uint32_t *sums, RegionCounters *regions,
                                                             const mtgl_raster_state *rs1,
                                                             const mtgl_vertex_state *vs1)
 {
     static_assert(NW == 1 || NW == 3, "one wave, or one per corner");
     __shared__ SetupStage st;
     __shared__ CV s_corner[NW == 3 ? 3 : 1][NW == 3 ? SETUP_BLOCK : 1];
-    __shared__ MaskIn s_mi[NW == 3 ? SETUP_BLOCK : 1];                       // records whose mask waves 1, 2 form
-    __shared__ unsigned long long s_mpart[NW == 3 ? 2 : 1][NW == 3 ? SETUP_BLOCK : 1];   // ... their halves
     const uint32_t sc = scene_of(block_scene, nscenes, blockIdx.x);
     // the scene's tables and the states they point to: one round of loads
     // when the launch passes the states of its one scene (rs1, vs1), else two
@@ -1154,10 +1192,12 @@ __global__ void __launch_bounds__(NW * SETUP_BLOCK) k_setup(const SetupParams *S
     const VertexParams &V = st.vp;
     const mtgl_vertex_state *vs0 = MULTI ? V.vstates : &st.vs;
     // the counters later kernels of the launch accumulate start at zero
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        P.ctr->nheavy = 0u;
-        P.ctr->nlight = 0u;
-        P.ctr->nbig = 0u;
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < BIN_REGIONS) regions[threadIdx.x] = {0u, 0u, 0ull};
+        if (threadIdx.x == 0) {
+            P.ctr->npairs = 0ull;
+            P.ctr->nbig = 0u;
+        }
     }
     const uint32_t l = threadIdx.x % SETUP_BLOCK, corner = threadIdx.x / SETUP_BLOCK;
     const uint32_t t = (blockIdx.x - block_pre[sc]) * SETUP_BLOCK + l;
@@ -1173,17 +1213,14 @@ __global__ void __launch_bounds__(NW * SETUP_BLOCK) k_setup(const SetupParams *S
             s_corner[NW == 3 ? corner : 0u][NW == 3 ? l : 0u] = o;
         }
         __syncthreads();
+        if (corner != 0u) return;   // (whole waves)
     }
     const mtgl_raster_state *rs = &st.rs;
     uint32_t nout = 0, rb = 0;
     unsigned long long tiles = 0;
-    // NW = 3: the set-up wave leaves the tile masks of its unclipped records
-    // to waves 1 and 2 (half of each box's longer side each) and completes
-    // those boxes afterwards
-    MaskIn mi;
-    mi.want = 0;
-    RBox bxd;
-    if (corner == 0u && act) {
+    TileBounds tb = {0, 0, 0, 0};
+    bool list = false;   // the records are a run of the overflow pool
+    if (act) {
         CV v[3];
         if (NW == 3) {
             for (int k = 0; k < 3; k++) v[k] = s_corner[NW == 3 ? k : 0][NW == 3 ? l : 0u];
@@ -1207,48 +1244,43 @@ __global__ void __launch_bounds__(NW * SETUP_BLOCK) k_setup(const SetupParams *S
             for (int k = 0; k < 3; k++) perspective_divide(v[k]);
             int nt = 0;
             RBox bx;
-            if (setup_fan(P, rs, v[0], v[1], v[2], cold, P.rt + t, cold ? P.rcold + t : nullptr, &bx, &nt,
-                          NW == 3 ? &mi : nullptr)) {
+            if (setup_fan(P, rs, v[0], v[1], v[2], cold, P.rt + t, cold ? P.rcold + t : nullptr, tb,
+                          BIN ? nullptr : &bx, &nt)) {
                 nout = 1;
                 tiles = (unsigned long long)nt;
-                if (mi.want) bxd = bx;
-                else P.box[t] = bx;
-            } else {
-                mi.want = 0;
+                if (!BIN) P.box[t] = bx;
             }
         } else {
             uint32_t base;
-            nout = setup_clipped(P, rs, v[0], v[1], v[2], cold, base, tiles);
+            nout = setup_clipped(P, rs, v[0], v[1], v[2], cold, base, tb, tiles);
             rb = P.over_base + base;
+            list = true;
         }
     }
-    if (NW == 3) {
-        if (corner == 0u) {
-            if (mi.want) s_mi[l] = mi;
-            else s_mi[l].want = 0;
-        }
-        __syncthreads();
-        if (corner != 0u) {
-            const MaskIn &d = s_mi[l];
-            unsigned long long m = 0ull;
-            if (d.want) {
-                const int32_t half = (max(d.tw, d.th) + 1) / 2;
-                const int32_t lo = corner == 1u ? 0 : half, hi = corner == 1u ? half : 64;
-                m = box_tile_mask(d.X, d.Y, d.area, d.minX, d.minY, d.maxX, d.maxY, d.tx0, d.ty0, d.tw, d.th,
-                                  P.fb_w, P.fb_h, lo, hi);
+    const uint32_t kept = (uint32_t)__builtin_amdgcn_readlane((int)dpp_incl_scan(nout), 63);
+    {
+        const uint32_t lo = nout ? (uint32_t)tb.x0 | ((uint32_t)tb.y0 << 16) : TBOX_NONE_X;
+        const uint32_t hi = nout ? (uint32_t)tb.x1 | ((uint32_t)tb.y1 << 16) : TBOX_NONE_Y;
+        if (BIN && act) {
+            P.tbox[t] = make_uint2(lo, hi | (nout && list ? TBOX_LIST : 0u));
+            if (nout && list) {
+                P.n_rt[t] = nout;
+                P.rec_base[t] = rb;
             }
-            s_mpart[corner - 1u][l] = m;
         }
-        __syncthreads();
-        if (corner != 0u) return;   // (whole waves)
-        if (mi.want) {
-            const unsigned long long m = s_mpart[0][l] | s_mpart[1][l];
-            bxd.mask = m;
-            bxd.masked = 1u;
-            bxd.ntiles = (uint32_t)__popcll(m);
-            P.box[t] = bxd;
-            tiles = bxd.ntiles;
+        const uint32_t blo = dpp_wave_minmax_u16x2<false>(lo), bhi = dpp_wave_minmax_u16x2<true>(hi);
+        if (threadIdx.x == 63) {
+            if (BIN) blk_box[blockIdx.x] = make_uint2(blo, bhi);
+            if (kept) {
+                // (64 addresses: no long queue at any of them)
+                const uint32_t side = P.bin_side;
+                const uint32_t cols = (bhi & 0xFFFFu) / side - (blo & 0xFFFFu) / side + 1u;
+                const uint32_t rows = (bhi >> 16) / side - (blo >> 16) / side + 1u;
+                atomicAdd(sums + 64u + (blockIdx.x & 63u), cols * rows);
+                if (BIN) atomicAdd(sums + (blockIdx.x & 63u), kept);
+            }
         }
+        if (BIN) return;
     }
     if (act) {
         P.n_rt[t] = nout;
@@ -1257,7 +1289,6 @@ __global__ void __launch_bounds__(NW * SETUP_BLOCK) k_setup(const SetupParams *S
     }
     // the block's kept fan triangles and pairs into its own slots (the pair
     // offsets of the launch are a scan of the block sums)
-    const uint32_t kept = (uint32_t)__builtin_amdgcn_readlane((int)dpp_incl_scan(nout), 63);
     const unsigned long long pairs = wave_inclusive_scan(tiles);
     if (threadIdx.x == 63) {
         blk_kept[blockIdx.x] = kept;
@@ -1749,7 +1780,7 @@ __global__ void __launch_bounds__(256) k_tile_list(const uint32_t *tile_start, c
                                                    const uint32_t *tile_gen, uint32_t gen, uint32_t ntiles,
                                                    uint32_t heavy_bin, const uint32_t *tile_scene,
                                                    const uint32_t *tile_pre, uint32_t nscenes, uint4 *list,
-                                                   uint32_t list_cap, Counters *ctr)
+                                                   uint32_t list_cap, Counters *ctr, RegionCounters *regions)
 {
     __shared__ uint32_t s_waves[4];
     __shared__ uint32_t s_base[2];
@@ -1775,7 +1806,7 @@ __global__ void __launch_bounds__(256) k_tile_list(const uint32_t *tile_start, c
     if (threadIdx.x == 0) {
         const uint32_t th = tot & 0xFFFFu, tl = tot >> 16;
         const unsigned long long hl =
-            th | tl ? atomicAdd(reinterpret_cast<unsigned long long *>(&ctr->nheavy),
+            th | tl ? atomicAdd(reinterpret_cast<unsigned long long *>(&regions->nheavy),
                                 ((unsigned long long)tl << 32) | th)
                     : 0ull;
         s_base[0] = (uint32_t)hl;
@@ -1955,7 +1986,7 @@ __global__ void __launch_bounds__(BINS_THREADS) k_tile_bins(const uint32_t *keys
                                                             uint32_t *vals_out, uint32_t *tile_gen, uint32_t gen,
                                                             uint32_t heavy_bin, const uint32_t *tile_scene,
                                                             const uint32_t *tile_pre, uint32_t nscenes, uint4 *list,
-                                                            uint32_t list_cap, Counters *ctr)
+                                                            uint32_t list_cap, Counters *ctr, RegionCounters *regions)
 {
     __shared__ uint32_t cur[BINS_WAVES][1 << BINS_MAX_SHIFT];   // per wave and tile: count, then cursor
     __shared__ uint32_t seg_v[BINS_MAX_SEGS + 1];   // runs of the bucket: first position in bucket order
@@ -2077,7 +2108,7 @@ __global__ void __launch_bounds__(BINS_THREADS) k_tile_bins(const uint32_t *keys
             tl += x1;
         }
         const unsigned long long hl =
-            th | tl ? atomicAdd(reinterpret_cast<unsigned long long *>(&ctr->nheavy),
+            th | tl ? atomicAdd(reinterpret_cast<unsigned long long *>(&regions->nheavy),
                                 ((unsigned long long)tl << 32) | th)
                     : 0ull;
         hb = (uint32_t)hl;
@@ -2113,6 +2144,328 @@ __global__ void __launch_bounds__(BINS_THREADS) k_tile_bins(const uint32_t *keys
 
 
 // ---------------------------------------------------------------------------
+// K3 in one launch: bins without a global sort
+// ---------------------------------------------------------------------------
+
+// One workgroup per square of a scene, BIN_T tiles a side (32 pixels) or, in
+// scenes with many triangles per tile, fewer (bin_side).  It walks the scene's set-up blocks in order, then
+// the triangles of those whose tile bounds meet the square, and lists the
+// records that do (s_list, in submission order).  Per 64 listed records a
+// wave, one record per lane, tests the 64 tiles exactly (box_tile_mask's
+// argument: a tile whose best corner fails an edge holds no covered pixel)
+// and leaves, per tile, the mask of the records it can hold; the masks'
+// running counts place each tile's records, in order, in one range of vals
+// reserved with one atomic.  The tiles' work items follow as in k_tile_bins.
+// More than BIN_LIST records in one square are taken in windows of the list
+// order, twice: to count, and to write.
+//
+// Against the expansion to pairs and the two-level sort by tile, which this
+// replaces where it applies (use_bins), the pairs, their keys and the
+// per-triangle boxes and masks never reach memory, and three launches go:
+// those kernels are bound by their chains of dependent loads, not by
+// bandwidth, and so is this one.  For the 32,768-triangle sphere at 1080p it
+// takes 23 us (the four kernels 31, and set-up 4 more for the masks), for a
+// draw of 1,280 triangles 10.7 (18.1).  Squares of 8 tiles a side took 42 and
+// 16 us, of 2 tiles 13 on the small draw; 16 waves 31 and 13, 4 waves 30 and
+// 12.
+constexpr int BIN_T = 4;
+constexpr uint32_t BIN_TILES = BIN_T * BIN_T, BIN_PARTS = 64 / BIN_TILES;
+constexpr int BIN_WAVES = 8;
+constexpr int BIN_THREADS = 64 * BIN_WAVES;
+constexpr uint32_t BIN_LIST = 4096;
+constexpr uint32_t BIN_GROUPS = BIN_LIST / 64;
+constexpr int BIN_U = 4;               // set-up blocks a wave's lanes hold per step of the walk
+
+struct BinParams {
+    const SetupParams *scenes;         // several scenes: their tables
+    const uint32_t *bin_pre, *bin_scene, *sblock_pre;
+    uint32_t nscenes;
+    uint32_t ntri;                     // one scene: its triangles and framebuffer
+    int32_t fb_w, fb_h, tiles_x, side;
+    uint32_t cols;
+    const uint2 *tbox, *blk_box;       // per triangle and set-up block of the launch
+    const uint32_t *n_rt, *rec_base;
+    const RTri *rt;
+    uint32_t cap;                      // records one region of vals holds
+    uint32_t *vals, *tile_gen;
+    uint32_t gen, heavy_bin, list_cap, seq;
+    uint4 *list;
+    RegionCounters *regions;
+    Counters *ctr;
+};
+
+struct BinArea {
+    uint32_t lo, hi;                   // first and last tile column | row << 16 (TBox layout)
+};
+
+__device__ __forceinline__ bool bin_meets(const BinArea &a, uint2 q)
+{
+    return (q.x & 0xFFFFu) <= (a.hi & 0xFFFFu) && (q.x >> 16) <= (a.hi >> 16) &&
+           (q.y & (TBOX_LIST - 1u)) >= (a.lo & 0xFFFFu) && (q.y >> 16) >= (a.lo >> 16);
+}
+
+// The sum of v over the waves before this one, and over all (s: one word per
+// wave); every thread of the workgroup calls it with its wave's value.
+__device__ __forceinline__ uint32_t bin_wave_offset(uint32_t v, uint32_t *s, uint32_t &all)
+{
+    const uint32_t w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63u) == 0u) s[w] = v;
+    __syncthreads();
+    uint32_t before = 0;
+    all = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)BIN_WAVES; k++) {
+        const uint32_t x = s[k];
+        before += k < w ? x : 0u;
+        all += x;
+    }
+    return before;
+}
+
+__global__ void __launch_bounds__(BIN_THREADS) k_bin(BinParams P)
+{
+    __shared__ uint32_t s_list[BIN_LIST];
+    __shared__ uint64_t s_mask[BIN_GROUPS][BIN_TILES];
+    __shared__ uint32_t s_pre[BIN_GROUPS][BIN_TILES];
+    __shared__ uint32_t s_start[BIN_TILES];
+    __shared__ uint32_t s_blk[BIN_THREADS];
+    __shared__ uint32_t s_w[2][BIN_WAVES];
+    __shared__ uint32_t s_over;
+    // (looked at after the walk, whose loads they overlap)
+    const uint32_t poison = P.ctr->poison, clip_full = P.ctr->overflow_full;
+    uint32_t sc = 0, ntri = P.ntri, blk0 = 0, tri0 = 0, tile0 = 0, bin = blockIdx.x;
+    int32_t fb_w = P.fb_w, fb_h = P.fb_h, tiles_x = P.tiles_x, side = P.side;
+    uint32_t cols = P.cols;
+    if (P.nscenes > 1u) {
+        sc = __builtin_amdgcn_readfirstlane(P.bin_scene[blockIdx.x]);
+        const SetupParams &S = P.scenes[sc];
+        bin -= P.bin_pre[sc];
+        ntri = S.ntri;
+        blk0 = P.sblock_pre[sc];
+        tri0 = S.tri_off;
+        tile0 = S.tile_off;
+        fb_w = S.fb_w;
+        fb_h = S.fb_h;
+        tiles_x = S.tiles_x;
+        side = (int32_t)S.bin_side;
+        cols = S.bin_cols;
+    }
+    const int32_t tx0 = (int32_t)(bin % cols) * side, ty0 = (int32_t)(bin / cols) * side;
+    const BinArea area = {(uint32_t)tx0 | ((uint32_t)ty0 << 16),
+                          (uint32_t)(tx0 + side - 1) | ((uint32_t)(ty0 + side - 1) << 16)};
+    const uint32_t nblk = (ntri + SETUP_BLOCK - 1) / SETUP_BLOCK;
+    const uint32_t lane = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t lt = (1ull << lane) - 1ull;
+
+    // records [win, win + BIN_LIST) of the square's list into s_list; returns
+    // the length of the whole list
+    auto walk = [&](uint32_t win) -> uint32_t {
+        uint32_t total = 0;
+        for (uint32_t b0 = 0; b0 < nblk; b0 += BIN_THREADS) {
+            const uint32_t b = b0 + threadIdx.x;
+            const bool hit = b < nblk && bin_meets(area, P.blk_box[blk0 + b]);
+            const uint64_t bal = __ballot(hit);
+            uint32_t nl;
+            const uint32_t off = bin_wave_offset((uint32_t)__popcll(bal), s_w[0], nl);
+            if (hit) s_blk[off + (uint32_t)__popcll(bal & lt)] = b;
+            __syncthreads();
+            for (uint32_t i0 = 0; i0 < nl; i0 += BIN_WAVES * BIN_U) {   // (uniform)
+                uint32_t tl[BIN_U], cnt[BIN_U], inc[BIN_U], sum = 0;
+                uint2 q[BIN_U];
+#pragma unroll
+                for (int u = 0; u < BIN_U; u++) {
+                    const uint32_t i = i0 + w * BIN_U + (uint32_t)u;
+                    tl[u] = i < nl ? s_blk[i] * SETUP_BLOCK + lane : ntri;
+                    q[u] = tl[u] < ntri ? P.tbox[tri0 + tl[u]] : make_uint2(TBOX_NONE_X, TBOX_NONE_Y);
+                }
+#pragma unroll
+                for (int u = 0; u < BIN_U; u++) {
+                    const bool own = bin_meets(area, q[u]);
+                    cnt[u] = own ? 1u : 0u;
+                    if (own && (q[u].y & TBOX_LIST)) cnt[u] = P.n_rt[tri0 + tl[u]];
+                    inc[u] = dpp_incl_scan(cnt[u]);
+                    sum += (uint32_t)__builtin_amdgcn_readlane((int)inc[u], 63);
+                }
+                uint32_t all;
+                uint32_t base = total + bin_wave_offset(sum, s_w[1], all);
+#pragma unroll
+                for (int u = 0; u < BIN_U; u++) {
+                    const uint32_t at = base + inc[u] - cnt[u] - win;
+                    if (cnt[u]) {
+                        if (q[u].y & TBOX_LIST) {
+                            const uint32_t rb = P.rec_base[tri0 + tl[u]];
+                            for (uint32_t j = 0; j < cnt[u]; j++)
+                                if (at + j < BIN_LIST) s_list[at + j] = rb + j;
+                        } else if (at < BIN_LIST) {
+                            s_list[at] = tri0 + tl[u];
+                        }
+                    }
+                    base += (uint32_t)__builtin_amdgcn_readlane((int)inc[u], 63);
+                }
+                total += all;
+                __syncthreads();   // s_w and s_list are written before the next step, or read
+            }
+        }
+        return total;
+    };
+
+    // per 64 records of the window and tile of the square: the mask of the
+    // records whose covered pixels may lie in the tile
+    auto masks = [&](uint32_t n) {
+        for (uint32_t g = w; g * 64u < n; g += BIN_WAVES) {
+            const bool valid = g * 64u + lane < n;
+            const uint32_t rec = valid ? s_list[g * 64u + lane] : 0u;
+            float4 q[3];
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                q[k] = valid ? reinterpret_cast<const float4 *>(P.rt + rec)[k] : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float fx0 = (float)__float_as_int(q[0].x), fy0 = (float)__float_as_int(q[0].y);
+            const float fx1 = (float)__float_as_int(q[0].z), fy1 = (float)__float_as_int(q[0].w);
+            const float fx2 = (float)__float_as_int(q[1].x), fy2 = (float)__float_as_int(q[1].y);
+            const int32_t xl = max(__float_as_int(q[1].z), 0), yl = max(__float_as_int(q[1].w), 0);
+            const int32_t xh = min(__float_as_int(q[2].x), fb_w - 1), yh = min(__float_as_int(q[2].y), fb_h - 1);
+            const float sg = q[2].z > 0.0f ? 1.0f : -1.0f;
+            const float dy0 = sg * (fy2 - fy1), dy1 = sg * (fy0 - fy2), dy2 = sg * (fy1 - fy0);
+            const float dx0 = sg * (fx2 - fx1), dx1 = sg * (fx0 - fx2), dx2 = sg * (fx1 - fx0);
+            float a0[BIN_T], a1[BIN_T], a2[BIN_T], b0[BIN_T], b1[BIN_T], b2[BIN_T];
+#pragma unroll
+            for (int i = 0; i < BIN_T; i++) {
+                const int32_t px = (tx0 + i) * TILE, py = (ty0 + i) * TILE;
+                const int32_t xa = max(px, xl), xb = min(px + TILE - 1, xh);
+                const int32_t ya = max(py, yl), yb = min(py + TILE - 1, yh);
+                a0[i] = ((float)(dy0 >= 0.0f ? xb : xa) - fx1) * dy0;
+                a1[i] = ((float)(dy1 >= 0.0f ? xb : xa) - fx2) * dy1;
+                a2[i] = ((float)(dy2 >= 0.0f ? xb : xa) - fx0) * dy2;
+                b0[i] = ((float)(dx0 >= 0.0f ? ya : yb) - fy1) * dx0;
+                b1[i] = ((float)(dx1 >= 0.0f ? ya : yb) - fy2) * dx1;
+                b2[i] = ((float)(dx2 >= 0.0f ? ya : yb) - fy0) * dx2;
+                if (!valid || xa > xb || i >= side) a0[i] = -__builtin_inff();
+                if (ya > yb || i >= side) b0[i] = __builtin_inff();
+            }
+#pragma unroll
+            for (int j = 0; j < BIN_T; j++)
+#pragma unroll
+                for (int i = 0; i < BIN_T; i++) {
+                    const uint64_t bal = __builtin_amdgcn_ballot_w64(a0[i] >= b0[j]) &
+                                         __builtin_amdgcn_ballot_w64(a1[i] >= b1[j]) &
+                                         __builtin_amdgcn_ballot_w64(a2[i] >= b2[j]);
+                    if (lane == 0) s_mask[g][j * BIN_T + i] = bal;
+                }
+        }
+    };
+
+    // (the lanes below BIN_TILES of one wave) each tile's records before
+    // every group of 64, from run on
+    auto prefix = [&](uint32_t n, uint32_t run) -> uint32_t {
+        if (lane < BIN_TILES) {
+#pragma unroll 4
+            for (uint32_t g = 0; g < (n + 63u) / 64u; g++) {
+                s_pre[g][lane] = run;
+                run += (uint32_t)__popcll(s_mask[g][lane]);
+            }
+        }
+        return run;
+    };
+
+    const uint32_t total = walk(0u);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && clip_full != 0u) {
+        // set-up's clip pool was too small: the launch runs again
+        const uint32_t was = atomicCAS(&P.ctr->poison, 0u, P.seq);
+        if (was == 0u || was == P.seq) atomicOr(&P.ctr->poison_flags, clip_full);
+        atomicOr(&P.ctr->sticky, clip_full);
+    }
+    // (poisoned by an earlier launch: this one runs again)
+    if (total == 0u || (poison != 0u && poison != P.seq)) return;
+    const bool one = total <= BIN_LIST;
+    uint32_t run = 0;
+    for (uint32_t win = 0; win < total; win += BIN_LIST) {   // (uniform)
+        const uint32_t n = min(BIN_LIST, total - win);
+        if (win) walk(win);
+        masks(n);
+        __syncthreads();
+        if (w == 0u) run = prefix(n, run);
+        if (!one) __syncthreads();
+    }
+    uint32_t start = 0;
+    if (w == 0u) {
+        // the square's range of vals and its items' places in the work list,
+        // in its region of both
+        const uint32_t region = blockIdx.x % BIN_REGIONS;
+        const uint32_t inc = dpp_incl_scan(run);
+        const uint32_t sum = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+        const bool hv = run > P.heavy_bin, md = !hv && run > MED_BIN, ltl = !hv && !md && run != 0u;
+        const uint64_t bh = __ballot(hv), bm = __ballot(md), bl = __ballot(ltl);
+        unsigned long long at = 0, hl = 0;
+        if (lane == 0u && sum != 0u) {
+            at = atomicAdd(&P.regions[region].pairs, (unsigned long long)sum);
+            hl = atomicAdd(reinterpret_cast<unsigned long long *>(&P.regions[region].nheavy),
+                           ((unsigned long long)(uint32_t)__popcll(bl) << 32) |
+                               (HEAVY_SPLIT * (uint32_t)__popcll(bh) + (uint32_t)__popcll(bm)));
+            const bool over = at + sum > P.cap;
+            if (over) {
+                // more records than the region of vals holds: the launch
+                // poisons the Exec, with the pairs that BIN_REGIONS regions of
+                // this one's need would hold (the last square of the fullest
+                // region to reserve its range has the largest)
+                const uint32_t was = atomicCAS(&P.ctr->poison, 0u, P.seq);
+                if (was == 0u || was == P.seq) {
+                    atomicOr(&P.ctr->poison_flags, 2u);
+                    atomicMax(&P.ctr->poison_pairs, (at + sum) * BIN_REGIONS);
+                }
+                atomicOr(&P.ctr->sticky, 2u);
+            }
+            s_over = over ? 1u : 0u;
+        }
+        if (lane == 0u && sum == 0u) s_over = 0u;
+        const uint32_t base = region * P.cap + (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
+        uint4 *const list = P.list + (size_t)region * P.list_cap;
+        const uint32_t hb = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)hl);
+        const uint32_t lb = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(hl >> 32));
+        start = base + inc - run;
+        const uint32_t tile = (uint32_t)((ty0 + (int32_t)(lane / BIN_T)) * tiles_x + tx0 + (int32_t)(lane % BIN_T));
+        if (run != 0u) {
+            P.tile_gen[tile0 + tile] = P.gen;
+            const uint4 item = make_uint4(tile, start, start + run, sc);
+            const uint32_t of = hb + HEAVY_SPLIT * (uint32_t)__popcll(bh & lt) + (uint32_t)__popcll(bm & lt);
+            if (hv) {
+                for (uint32_t k = 0; k < HEAVY_SPLIT; k++)
+                    if (of + k < P.list_cap)
+                        list[of + k] = make_uint4(item.x | ((k + 1u) << ITEM_TILE_BITS), item.y, item.z, item.w);
+            }
+            if (md && of < P.list_cap) list[of] = item;
+            if (ltl) {
+                const uint32_t o = lb + (uint32_t)__popcll(bl & lt);
+                if (o < P.list_cap) list[P.list_cap - 1u - o] = item;
+            }
+        }
+        if (lane < BIN_TILES) s_start[lane] = start;
+    }
+    __syncthreads();
+    if (s_over != 0u) return;
+    // a tile per lane, the group's records in BIN_PARTS parts
+    const uint32_t tl = lane % BIN_TILES, part = lane / BIN_TILES, per = 64u / BIN_PARTS;
+    const uint32_t tstart = s_start[tl];
+    run = 0;
+    for (uint32_t win = 0; win < total; win += BIN_LIST) {   // (uniform)
+        const uint32_t n = min(BIN_LIST, total - win);
+        if (!one) {
+            __syncthreads();   // the previous window is written
+            walk(win);
+            masks(n);
+            __syncthreads();
+            if (w == 0u) run = prefix(n, run);
+            __syncthreads();
+        }
+        for (uint32_t g = w; g * 64u < n; g += BIN_WAVES) {
+            const uint64_t mg = s_mask[g][tl];
+            uint32_t at = tstart + s_pre[g][tl] + (uint32_t)__popcll(mg & ((1ull << (part * per)) - 1ull));
+            for (uint32_t m = (uint32_t)(mg >> (part * per)) & ((1u << per) - 1u); m; m &= m - 1u)
+                P.vals[at++] = s_list[g * 64u + part * per + (uint32_t)__builtin_ctz(m)];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // K4: fine raster and per-fragment pipeline
 // ---------------------------------------------------------------------------
 
@@ -2123,8 +2476,6 @@ __global__ void __launch_bounds__(BINS_THREADS) k_tile_bins(const uint32_t *keys
 __device__ __forceinline__ void reset_counters(Counters *ctr)
 {
     ctr->npairs = 0;
-    ctr->nheavy = 0;
-    ctr->nlight = 0;
     ctr->unsupported = 0;
     ctr->noverflow = 0;
     ctr->nbig = 0;
@@ -2840,14 +3191,21 @@ __device__ __forceinline__ uint64_t depth_pass(const RasterConsts &K, const RCov
 // items last the dispatcher hands
 // each freed slot the next block: a slot busy with a long item takes no
 // other.
-__device__ __forceinline__ void list_counts(const RasterParams &P, uint32_t &nh, uint32_t &it0, uint32_t &nt)
+struct ListIndex {
+    uint32_t nh, nt;     // items at the fronts of the regions, and in all
+    uint32_t fr, bk;     // lane r: front and back items of regions 0 .. r
+};
+
+__device__ __forceinline__ void list_counts(const RasterParams &P, ListIndex &X)
 {
-    nh = __builtin_amdgcn_readfirstlane(*(volatile uint32_t *)&P.ctr->nheavy);
-    nt = nh + __builtin_amdgcn_readfirstlane(*(volatile uint32_t *)&P.ctr->nlight);
-    nt = min(nt, P.list_cap);
-    nh = min(nh, nt);
-    it0 = P.part == 2u ? nh : 0u;
-    if (P.part == 1u) nt = nh;
+    unsigned long long v = 0;
+    if (threadIdx.x < BIN_REGIONS)
+        v = *(const volatile unsigned long long *)&P.regions[threadIdx.x].nheavy;
+    const uint32_t h = min((uint32_t)v, P.list_cap), l = min((uint32_t)(v >> 32), P.list_cap - h);
+    X.fr = dpp_incl_scan(h);
+    X.bk = dpp_incl_scan(l);
+    X.nh = (uint32_t)__builtin_amdgcn_readlane((int)X.fr, 63);
+    X.nt = X.nh + (uint32_t)__builtin_amdgcn_readlane((int)X.bk, 63);
 }
 
 // The dispatcher deals consecutive blocks of a grid to the 8 XCDs in turn,
@@ -2867,18 +3225,25 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t G)
     return ((i / XCD_RUN) * NXCD + x) * XCD_RUN + i % XCD_RUN;
 }
 
-__device__ __forceinline__ uint32_t list_item(uint32_t it0, uint32_t k, uint32_t b, uint32_t G)
+__device__ __forceinline__ uint32_t list_item(uint32_t k, uint32_t b, uint32_t G)
 {
     const uint32_t v = xcd_block(b, G);
-    return it0 + k * G + ((k & 1u) ? G - 1u - v : v);
+    return k * G + ((k & 1u) ? G - 1u - v : v);
 }
 
 
 // list item -> scene, the scene-local tile, the part (0 whole tile, q = 1..HEAVY_SPLIT
 // pixel rows [(q - 1) * PART_ROWS, q * PART_ROWS)) and the tile's bin [e0, e1)
-__device__ __forceinline__ uint4 load_item(const RasterParams &P, uint32_t it, uint32_t nh)
+__device__ __forceinline__ uint4 load_item(const RasterParams &P, uint32_t it, const ListIndex &X)
 {
-    return P.list[it < nh ? it : P.list_cap - 1u - (it - nh)];
+    // (it is uniform) the region that holds the item: the first whose running
+    // count passes it
+    const bool front = it < X.nh;
+    const uint32_t i = front ? it : it - X.nh, run = front ? X.fr : X.bk;
+    const uint32_t r = (uint32_t)__popcll(__ballot(run <= i));
+    const uint32_t before = r ? (uint32_t)__builtin_amdgcn_readlane((int)run, (int)r - 1) : 0u;
+    const uint32_t k = i - before;
+    return P.list[(size_t)r * P.list_cap + (front ? k : P.list_cap - 1u - k)];
 }
 
 __device__ __forceinline__ void decode_item(uint4 v, uint32_t &sc, uint32_t &tile, uint32_t &e0, uint32_t &e1,
@@ -2901,10 +3266,10 @@ __device__ __forceinline__ void item_priority(uint32_t it, uint32_t nh)
     else __builtin_amdgcn_s_setprio(0);
 }
 
-__device__ __forceinline__ void item_tile(const RasterParams &P, uint32_t it, uint32_t nh, uint32_t &sc, uint32_t &tile,
-                                          uint32_t &e0, uint32_t &e1, uint32_t &quarter)
+__device__ __forceinline__ void item_tile(const RasterParams &P, uint32_t it, const ListIndex &X, uint32_t &sc,
+                                          uint32_t &tile, uint32_t &e0, uint32_t &e1, uint32_t &quarter)
 {
-    decode_item(load_item(P, it, nh), sc, tile, e0, e1, quarter);
+    decode_item(load_item(P, it, X), sc, tile, e0, e1, quarter);
 }
 
 __device__ __forceinline__ void raster_consts(const SceneRaster &P, RasterConsts &K)
@@ -2967,6 +3332,33 @@ __device__ __forceinline__ void raster_consts(const SceneRaster &P, RasterConsts
     else K.depth_mode = DEPTH_IND;
 }
 
+// The first raster kernel of a launch (its block 0) takes set-up's count of
+// met squares and, after k_bin, ends its and set-up's use of the per-launch
+// counters: a launch that did not overflow adds its kept fan triangles and
+// its pairs to the running counts, and the clip pool, its overflow bits and
+// the unsupported flags start the next launch at zero.
+__device__ __forceinline__ void end_binning(const RasterParams &P)
+{
+    Counters *c = P.ctr;
+    const unsigned long long met = wave_inclusive_scan((unsigned long long)P.meets[threadIdx.x]);
+    P.meets[threadIdx.x] = 0u;
+    if (threadIdx.x == 63) c->meets = (uint32_t)min(met, 0xFFFFFFFFull);
+    if (!P.kept) return;
+    const uint32_t k = P.kept[threadIdx.x];
+    P.kept[threadIdx.x] = 0u;
+    const uint32_t kept = dpp_wave_sum(k);
+    const uint32_t pairs = dpp_wave_sum(threadIdx.x < BIN_REGIONS ? (uint32_t)P.regions[threadIdx.x].pairs : 0u);
+    if (threadIdx.x == 0) {
+        if (c->poison == 0u) {
+            c->acc_tri_raster += kept;
+            c->acc_bin_pairs += pairs;   // (a launch that fits has fewer than 2^31)
+        }
+        c->overflow_full = 0u;
+        c->noverflow = 0u;
+        c->unsupported = 0u;
+    }
+}
+
 // Per-lane counts summed over the wave (bytes as two 32-bit halves) and
 // added to this block's own slot: no two blocks of a launch share a slot and
 // launches on the stream are ordered, so plain adds suffice (thousands of
@@ -3012,19 +3404,21 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
     __shared__ float s_dep[DCAP_W];
     __shared__ uint16_t s_slot[DCAP_W];   // taps << 12 | entry << 6 | pixel
 
+    if (blockIdx.x == 0 && P.meets) end_binning(P);
     if (exec_poisoned(P.ctr)) return;   // the launch runs again once its arrays have grown
     RasterConsts K;
     const int lane = threadIdx.x;
-    uint32_t nh, it0, nt;
-    list_counts(P, nh, it0, nt);
+    ListIndex X;
+    list_counts(P, X);
+    const uint32_t nh = X.nh, nt = X.nt;
     uint32_t frag_count = 0;
     unsigned long long frag_bytes = 0;
     // the next item's header is loaded while the current item is processed
-    uint32_t it = list_item(it0, 0u, blockIdx.x, gridDim.x);
-    uint4 hdr = it < nt ? load_item(P, it, nh) : make_uint4(0u, 0u, 0u, 0u);
+    uint32_t it = list_item(0u, blockIdx.x, gridDim.x);
+    uint4 hdr = it < nt ? load_item(P, it, X) : make_uint4(0u, 0u, 0u, 0u);
     for (uint32_t pass = 0; it < nt; pass++) {
-    const uint32_t it_next = list_item(it0, pass + 1u, blockIdx.x, gridDim.x);
-    const uint4 hdr_next = it_next < nt ? load_item(P, it_next, nh) : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t it_next = list_item(pass + 1u, blockIdx.x, gridDim.x);
+    const uint4 hdr_next = it_next < nt ? load_item(P, it_next, X) : make_uint4(0u, 0u, 0u, 0u);
     uint32_t sc, tile, e0, e1, quarter;
     decode_item(hdr, sc, tile, e0, e1, quarter);
     item_priority(it, nh);
@@ -3316,16 +3710,18 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PLAIN ?
     __shared__ uint16_t s_slot[FCAP];
     __shared__ uint8_t s_meta[FCAP];
 
+    if (blockIdx.x == 0 && P.meets) end_binning(P);
     if (exec_poisoned(P.ctr)) return;   // the launch runs again once its arrays have grown
     const int lane = threadIdx.x;
-    uint32_t nh, it0, nt;
-    list_counts(P, nh, it0, nt);
+    ListIndex X;
+    list_counts(P, X);
+    const uint32_t nh = X.nh, nt = X.nt;
     unsigned long long frag_count = 0, frag_bytes = 0;
     for (uint32_t pass = 0;; pass++) {
-    const uint32_t it = list_item(it0, pass, blockIdx.x, gridDim.x);
+    const uint32_t it = list_item(pass, blockIdx.x, gridDim.x);
     if (it >= nt) break;
     uint32_t sc, tile, e0, e1, quarter;
-    item_tile(P, it, nh, sc, tile, e0, e1, quarter);
+    item_tile(P, it, X, sc, tile, e0, e1, quarter);
     item_priority(it, nh);
     const SceneRaster &S = P.scenes[sc];
     const uint32_t kind = __builtin_amdgcn_readfirstlane(S.kind);
@@ -4015,8 +4411,8 @@ __global__ void __launch_bounds__(256) k_clear_span(uint32_t *color, float *dept
 // and stores 16 bytes (BPP 4) or 12 (BPP 3), so that a wave stores whole
 // cache lines (out is 16-byte aligned for BPP 4, 4-byte for BPP 3): out is
 // device memory, or the caller's own pinned memory over PCIe, which bounds
-// the kernel then.  poison (null: not wanted) receives the Exec's poison in
-// pinned host memory, so that the wait for the pixels also tells the host
+// the kernel then.  poison (null: not wanted) receives the Exec's poison, and
+// the latest launch's count of met squares after it, in pinned host memory, so that the wait for the pixels also tells the host
 // whether the queued work took effect; no pixel is stored when it did not.
 template <int BPP>
 __global__ void __launch_bounds__(256) k_read_pixels(const uint32_t *color, int32_t fb_w, int32_t fb_h, int32_t x,
@@ -4025,7 +4421,10 @@ __global__ void __launch_bounds__(256) k_read_pixels(const uint32_t *color, int3
 {
     static_assert(BPP == 3 || BPP == 4, "GL_RGB or GL_RGBA");
     if (poison) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) *poison = ctr->poison;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            poison[0] = ctr->poison;
+            poison[1] = ctr->meets;
+        }
         if (exec_poisoned(ctr)) return;
     }
     const uint64_t i = 4ull * ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x);
@@ -4517,7 +4916,12 @@ struct Exec {
     size_t ring_blk = 0, ring_off = 0, ring_used = 0;
     hipEvent_t upload_done = nullptr;
     Arena vhot, vcold, rt, rcold, box, n_rt, rec_base, tri_tiles, pair_base, scan_tmp, big_list;
-    Arena blk_kept, blk_pairs, blk_off;   // per set-up block: kept fan triangles, pairs, first pair
+    Arena blk_kept, blk_pairs, blk_off;   // per set-up block: kept fan triangles, pairs, first pair (the tile sort)
+    Arena tbox, blk_box;                  // tile bounds per triangle and per set-up block (k_bin)
+    RegionCounters *regions = nullptr;    // BIN_REGIONS: the work list's and vals' regions
+    uint32_t *sums = nullptr;             // k_setup's partial counts: 64 of kept fan triangles, 64 of met squares
+    double spread = -1.0;                 // of the latest launch seen to end: the part of the (set-up block, square)
+    uint64_t last_work = 0;               // pairs that meet, of last_work in all (-1: none seen yet)
     uint32_t overflow_cap = 0;
     Arena keys[2], vals[2], sort_tmp, tile_list;   // (tile, record) pairs and their sort
     Arena tile_start, tile_end, tile_gen;          // per launch-wide tile: bin range, generation of the range
@@ -4544,7 +4948,14 @@ struct Launch {
     uint8_t *host_rs = nullptr, *host_vs = nullptr, *host_st = nullptr;   // staged bytes
     uint32_t ns = 0;               // scenes with triangles
     uint32_t tri_total = 0, tiles_total = 0;
-    uint32_t vblocks = 0, sblocks = 0;
+    uint32_t sblocks = 0;
+    uint32_t nbins = 0;            // k_bin's squares
+    uint32_t region_items = 0;     // items a region of the work list may hold then
+    uint64_t work = 0;             // (set-up block, square) pairs
+    bool bins = false;             // binned by k_bin (else by the tile sort)
+    uint32_t ntri1 = 0;            // one scene: its triangles and framebuffer
+    int32_t fb_w1 = 0, fb_h1 = 0, tiles_x1 = 0, side1 = 0;
+    uint32_t cols1 = 0;
     bool any_cold = false;
     bool multi_vs = false;         // some scene switches vertex states per vertex
     bool unsupported = false;
@@ -4553,7 +4964,7 @@ struct Launch {
     bool simple = true;            // no scene for the depth kernel lights per fragment or samples the full chain
     uint64_t pairs_cap = 0;        // pairs of the sizing run (frozen replays use it)
     const VertexParams *vp = nullptr;
-    const uint32_t *vblock_pre = nullptr;
+    const uint32_t *bin_pre = nullptr;
     const SetupParams *sp = nullptr;
     const uint32_t *sblock_pre = nullptr;
     const uint32_t *tri_pre = nullptr;
@@ -4564,7 +4975,7 @@ struct Launch {
     const mtgl_raster_state *rs1 = nullptr;
     const mtgl_vertex_state *vs1 = nullptr;
     Arena maps;                    // block/tile -> scene maps of a launch with several scenes
-    const uint32_t *vmap = nullptr, *smap = nullptr, *tmap = nullptr;
+    const uint32_t *bmap = nullptr, *smap = nullptr, *tmap = nullptr;
     // the bytes the device copy of `params` holds (blocks up to PARAM_SHADOW_MAX):
     // a launch whose prepared bytes equal them does not upload them again
     std::vector<uint8_t> shadow;
@@ -4849,6 +5260,10 @@ int exec_init(Exec &x, int device)
     HIPC(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
     HIPC(hipMalloc((void **)&x.ctr, sizeof(Counters)));
     HIPC(hipMalloc((void **)&x.stat_slots, 2 * STAT_SLOTS * sizeof(unsigned long long)));
+    HIPC(hipMalloc((void **)&x.regions, BIN_REGIONS * sizeof(RegionCounters)));
+    HIPC(hipMemsetAsync(x.regions, 0, BIN_REGIONS * sizeof(RegionCounters), x.stream));
+    HIPC(hipMalloc((void **)&x.sums, 128 * sizeof(uint32_t)));
+    HIPC(hipMemsetAsync(x.sums, 0, 128 * sizeof(uint32_t), x.stream));
     HIPC(hipHostMalloc((void **)&x.ctr_host, sizeof(Counters), hipHostMallocDefault));
     HIPC(hipHostMalloc((void **)&x.report, 256, hipHostMallocDefault));
     *x.report = 0u;
@@ -4863,7 +5278,7 @@ void exec_free(Exec &x)
 {
     if (x.stream) (void)hipStreamSynchronize(x.stream);
     Arena *arenas[] = {&x.vhot, &x.vcold, &x.rt, &x.rcold, &x.box, &x.n_rt, &x.rec_base, &x.tri_tiles, &x.pair_base,
-                       &x.scan_tmp, &x.big_list, &x.blk_kept, &x.blk_pairs, &x.blk_off, &x.keys[0], &x.keys[1], &x.vals[0], &x.vals[1], &x.sort_tmp,
+                       &x.scan_tmp, &x.big_list, &x.blk_kept, &x.blk_pairs, &x.blk_off, &x.tbox, &x.blk_box, &x.keys[0], &x.keys[1], &x.vals[0], &x.vals[1], &x.sort_tmp,
                        &x.tile_list, &x.tile_start, &x.tile_end, &x.tile_gen};
     for (Arena *a : arenas) arena_free(*a);
     for (auto &pr : x.pending_events) {
@@ -4875,6 +5290,8 @@ void exec_free(Exec &x)
     x.free_events.clear();
     if (x.ctr) (void)hipFree(x.ctr);
     if (x.stat_slots) (void)hipFree(x.stat_slots);
+    if (x.sums) (void)hipFree(x.sums);
+    if (x.regions) (void)hipFree(x.regions);
     if (x.ctr_host) (void)hipHostFree(x.ctr_host);
     if (x.report) (void)hipHostFree(x.report);
     if (x.pinned) (void)hipHostFree(x.pinned);
@@ -4885,6 +5302,8 @@ void exec_free(Exec &x)
     if (x.stream) (void)hipStreamDestroy(x.stream);
     x.ctr = nullptr;
     x.stat_slots = nullptr;
+    x.sums = nullptr;
+    x.regions = nullptr;
     x.ctr_host = nullptr;
     x.report = nullptr;
     x.pinned = nullptr;
@@ -5007,8 +5426,61 @@ VSlots vertex_slots(const mtgl_dev *d, const mtgl_draw *dr)
 struct Sizes {
     uint64_t tri = 0, tiles = 0;
     uint64_t sblocks = 0;          // set-up blocks (each scene starts a block of its own)
+    uint64_t bins = 0;             // k_bin's squares
+    uint64_t work = 0, work_sum = 0;   // (set-up block, square) pairs of the largest scene and of all
+    uint64_t items = 0;            // work list items of one region after k_bin
+    bool crowded = false;          // a scene of over BIN_LARGE triangles, over BIN_LARGE_DENSE per tile
     bool cold = false;
 };
+
+// Which launches k_bin takes, the others going through the tile sort.  Every
+// square reads the bounds of its scene's set-up blocks, and of the triangles
+// of those that meet it: little where a block's triangles lie together, as a
+// mesh's do (a 1080p frame's 32,768-triangle sphere, of whose 1.04M (block,
+// square) pairs 1% meet, takes 88 us so and 104 sorted), all of them where
+// they lie anywhere (10,000 triangles scattered over 1080p, 0.32M pairs
+// nearly all of which meet: 117 and 105; 40,000: 247 and 163; 2,000, 0.06M
+// pairs: 72 and 71).  The set-up counts the pairs that meet, and the host
+// takes the part of them in the latest launch it has seen end for the next
+// one's; before it has seen any, launches of at most BIN_UNSEEN pairs.  Two
+// more go through the sort: meshes so large and dense that many squares list
+// more than a window holds (204,800 triangles of a sphere take 459 us at
+// 1080p and 353 sorted, 100,352 181 and 187; at 4K, 439 and 818), and
+// launches of so many squares that they wait for the chip in turn (the 512
+// scenes of the batched workload 2.37 ms and 2.22).  The choice changes no
+// pixel.
+constexpr double BIN_MEETS = 200e3;
+constexpr uint64_t BIN_UNSEEN = 1'500'000;
+constexpr uint64_t BIN_MAX = 16384;      // squares of a launch
+constexpr uint64_t BIN_LARGE = 128u << 10, BIN_LARGE_DENSE = 4;   // triangles of a scene, and per tile of it
+constexpr uint32_t BIN_DENSE = 24;       // triangles per tile above which squares shrink
+
+bool use_bins(const Exec &x, const Sizes &z)
+{
+    if (z.bins > BIN_MAX || z.crowded) return false;
+    return x.spread < 0.0 ? z.work <= BIN_UNSEEN : x.spread * (double)z.work <= BIN_MEETS;
+}
+
+// the met squares of the launch the host has just seen end
+void saw_meets(Exec &x, uint32_t meets)
+{
+    if (x.last_work) x.spread = (double)meets / (double)x.last_work;
+}
+
+// Tiles per side of k_bin's squares: BIN_T while the scene has few triangles
+// per tile, fewer where a square's list would grow past its window (a mesh
+// that fills a small framebuffer).
+uint32_t bin_side(const mtgl_dev *d, uint32_t ntri)
+{
+    const uint64_t tiles = (uint64_t)d->tiles_x * (uint64_t)d->tiles_y;
+    return ntri <= BIN_DENSE * tiles ? (uint32_t)BIN_T : ntri <= 8u * BIN_DENSE * tiles ? 2u : 1u;
+}
+
+uint32_t scene_bins(const mtgl_dev *d, uint32_t ntri)
+{
+    const int32_t t = (int32_t)bin_side(d, ntri);
+    return (uint32_t)((d->tiles_x + t - 1) / t) * (uint32_t)((d->tiles_y + t - 1) / t);
+}
 
 Sizes scene_sizes(const SceneIn *in, uint32_t n)
 {
@@ -5020,6 +5492,12 @@ Sizes scene_sizes(const SceneIn *in, uint32_t n)
         if (ntri == 0) continue;
         z.tri += ntri;
         z.sblocks += blocks_for(ntri, SETUP_BLOCK);
+        const uint64_t bins = scene_bins(in[i].dev, ntri), side = bin_side(in[i].dev, ntri);
+        z.bins += bins;
+        z.crowded |= ntri > BIN_LARGE && ntri > BIN_LARGE_DENSE * (uint64_t)in[i].dev->tiles_x * (uint64_t)in[i].dev->tiles_y;
+        z.work = std::max<uint64_t>(z.work, bins * blocks_for(ntri, SETUP_BLOCK));
+        z.work_sum += bins * blocks_for(ntri, SETUP_BLOCK);
+        z.items += HEAVY_SPLIT * side * side * ((bins + BIN_REGIONS - 1) / BIN_REGIONS);
         z.tiles += (uint64_t)in[i].dev->tiles_x * (uint64_t)in[i].dev->tiles_y;
         z.cold |= needs_cold(dr->raster);
     }
@@ -5035,11 +5513,15 @@ int reserve_scene_buffers(Exec &x, const Sizes &z)
     x.overflow_cap = std::max<uint32_t>(x.overflow_cap, std::min<uint32_t>((uint32_t)(z.tri / 8u), 1u << 24));
     if ((rc = arena_reserve(x, x.rt, (t + x.overflow_cap) * sizeof(RTri)))) return rc;
     if (z.cold && (rc = arena_reserve(x, x.rcold, (t + x.overflow_cap) * sizeof(RCold)))) return rc;
-    if ((rc = arena_reserve(x, x.box, (t + x.overflow_cap) * sizeof(RBox)))) return rc;
     if ((rc = arena_reserve(x, x.n_rt, t * sizeof(uint32_t)))) return rc;
     if ((rc = arena_reserve(x, x.rec_base, t * sizeof(uint32_t)))) return rc;
-    if ((rc = arena_reserve(x, x.big_list, t * sizeof(uint32_t)))) return rc;
     const size_t sb = (size_t)std::max<uint64_t>(z.sblocks, 1u);
+    if (use_bins(x, z)) {
+        if ((rc = arena_reserve(x, x.tbox, t * sizeof(uint2)))) return rc;
+        return arena_reserve(x, x.blk_box, sb * sizeof(uint2));
+    }
+    if ((rc = arena_reserve(x, x.box, (t + x.overflow_cap) * sizeof(RBox)))) return rc;
+    if ((rc = arena_reserve(x, x.big_list, t * sizeof(uint32_t)))) return rc;
     if ((rc = arena_reserve(x, x.blk_kept, sb * sizeof(uint32_t)))) return rc;
     if ((rc = arena_reserve(x, x.blk_pairs, sb * sizeof(unsigned long long)))) return rc;
     if ((rc = arena_reserve(x, x.blk_off, sb * sizeof(unsigned long long)))) return rc;
@@ -5113,8 +5595,11 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
     if (z.tri > 0x0FFFFFFFull || z.tiles >= (1ull << ITEM_TILE_BITS) / HEAVY_SPLIT) return MTGL_ERR_OUT_OF_MEMORY;
     L.tri_total = (uint32_t)z.tri;
     L.tiles_total = (uint32_t)z.tiles;
-    L.vblocks = 0;
     L.sblocks = (uint32_t)sb;
+    L.bins = use_bins(x, z);
+    L.nbins = L.bins ? (uint32_t)z.bins : 0u;
+    L.region_items = L.bins ? (uint32_t)z.items : 0u;
+    L.work = z.work_sum;
     L.any_cold = z.cold;
     L.plain = true;
     L.simple = true;
@@ -5143,8 +5628,8 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
     SetupParams *sp = reinterpret_cast<SetupParams *>(host + off_sp);
     SceneRaster *sr = reinterpret_cast<SceneRaster *>(host + off_sr);
     uint32_t *pre = reinterpret_cast<uint32_t *>(host + off_pre);
-    uint32_t *vbp = pre, *sbp = pre + (ns + 1), *tp = pre + 2 * (ns + 1), *tlp = pre + 3 * (ns + 1);
-    uint32_t toff = 0, tileoff = 0, sbo = 0;
+    uint32_t *bnp = pre, *sbp = pre + (ns + 1), *tp = pre + 2 * (ns + 1), *tlp = pre + 3 * (ns + 1);
+    uint32_t toff = 0, tileoff = 0, sbo = 0, bno = 0;
     for (uint32_t s = 0; s < ns; s++) {
         const Plan &p = plan[s];
         mtgl_dev *d = p.s->dev;
@@ -5197,17 +5682,26 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
         if (s == 0) {
             L.rs1 = rs_dev;
             L.vs1 = v.vstates;
+            L.ntri1 = p.ntri;
+            L.fb_w1 = d->w;
+            L.fb_h1 = d->h;
+            L.tiles_x1 = d->tiles_x;
+            L.side1 = (int32_t)bin_side(d, p.ntri);
+            L.cols1 = (uint32_t)((d->tiles_x + L.side1 - 1) / L.side1);
         }
         q.rt = as<RTri>(x.rt) + toff;
         q.rcold = L.any_cold ? as<RCold>(x.rcold) + toff : nullptr;
-        q.box = as<RBox>(x.box) + toff;
+        q.box = L.bins ? nullptr : as<RBox>(x.box) + toff;
         q.rt_over = as<RTri>(x.rt) + ttot;
         q.rcold_over = L.any_cold ? as<RCold>(x.rcold) + ttot : nullptr;
-        q.box_over = as<RBox>(x.box) + ttot;
+        q.box_over = L.bins ? nullptr : as<RBox>(x.box) + ttot;
         q.over_base = ttot;
         q.n_rt = as<uint32_t>(x.n_rt) + toff;
         q.rec_base = as<uint32_t>(x.rec_base) + toff;
-        q.tri_tiles = as<unsigned long long>(x.tri_tiles) + toff;
+        q.tri_tiles = L.bins ? nullptr : as<unsigned long long>(x.tri_tiles) + toff;
+        q.tbox = L.bins ? as<uint2>(x.tbox) + toff : nullptr;
+        q.bin_side = bin_side(d, p.ntri);
+        q.bin_cols = ((uint32_t)d->tiles_x + q.bin_side - 1u) / q.bin_side;
         q.overflow_cap = x.overflow_cap;
         q.ctr = x.ctr;
         sp[s] = q;
@@ -5237,15 +5731,16 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
         if (!(r.kind & KIND_LAST_WRITER) && (r.tex != nullptr || needs_cold(dr->raster))) L.plain = false;
         if ((r.kind & KIND_LAST_WRITER) && (needs_cold(dr->raster) || r.lod_mode == MTGL_LOD_FULL_CHAIN)) L.simple = false;
 
-        vbp[s] = 0;
+        bnp[s] = bno;
         sbp[s] = sbo;
         tp[s] = toff;
         tlp[s] = tileoff;
         toff += p.ntri;
         tileoff += (uint32_t)(d->tiles_x * d->tiles_y);
         sbo += blocks_for(p.ntri, SETUP_BLOCK);
+        if (L.bins) bno += scene_bins(d, p.ntri);
     }
-    vbp[ns] = 0;
+    bnp[ns] = bno;
     sbp[ns] = sbo;
     tp[ns] = toff;
     tlp[ns] = tileoff;
@@ -5260,104 +5755,51 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
     L.sp = (const SetupParams *)(dev + off_sp);
     L.sr = (const SceneRaster *)(dev + off_sr);
     const uint32_t *pre_dev = (const uint32_t *)(dev + off_pre);
-    L.vblock_pre = pre_dev;
+    L.bin_pre = pre_dev;
     L.sblock_pre = pre_dev + (ns + 1);
     L.tri_pre = pre_dev + 2 * (ns + 1);
     L.tile_pre = pre_dev + 3 * (ns + 1);
     if (ns > 1) {
-        const size_t nmap = (size_t)L.vblocks + L.sblocks + L.tiles_total;
+        const size_t nb = L.bins ? L.nbins : 0;
+        const size_t nmap = nb + L.sblocks + L.tiles_total;
         if ((rc = arena_reserve(x, L.maps, nmap * 4))) return rc;
         uint32_t *m = as<uint32_t>(L.maps);
-        L.vmap = m;
-        L.smap = m + L.vblocks;
-        L.tmap = m + L.vblocks + L.sblocks;
-        hipLaunchKernelGGL(k_scene_maps, dim3(ns), dim3(256), 0, x.stream, L.vblock_pre, L.sblock_pre, L.tile_pre,
-                           m, m + L.vblocks, m + L.vblocks + L.sblocks);
+        L.bmap = m;
+        L.smap = m + nb;
+        L.tmap = m + nb + L.sblocks;
+        hipLaunchKernelGGL(k_scene_maps, dim3(ns), dim3(256), 0, x.stream, L.bin_pre, L.sblock_pre, L.tile_pre,
+                           m, m + nb, m + nb + L.sblocks);
         HIPC(hipGetLastError());
     }
     return MTGL_OK;
 }
 
-// The pipeline over the scenes of L, queued on x.stream without waiting for
-// the GPU.  The pair arrays are sized from x.pair_ratio (a frozen run, a
-// replay or one being captured into a graph, allocates nothing and uses the
-// capacity of its sizing run); a launch that needs more pairs, or more clip
-// slots than the pool holds, poisons the Exec with seq (k_bin_scatter) and
-// writes nothing: the host learns of it when it next waits for the stream and
-// runs the launch again with larger arrays.
-int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
+// pairs the arrays of x hold for a launch binned by k_bin or by the tile sort
+uint64_t pairs_room(const Exec &x, bool bins)
 {
-    if (L.ns == 0) return L.unsupported ? MTGL_ERR_UNSUPPORTED : MTGL_OK;
+    size_t c = x.vals[0].cap;
+    if (!bins) c = std::min(std::min(c, x.vals[1].cap), std::min(x.keys[0].cap, x.keys[1].cap));
+    return std::min<uint64_t>(c / 4, 0x7FFFFFFFull);
+}
+
+// K3 of launches k_bin does not take: pair offsets and total (read on the
+// device: the host never waits), expansion in submission order, stable sort
+// by tile, tile ranges and the work list.  vals: the sorted records.
+int tile_sort(Exec &x, Launch &L, bool frozen, uint32_t seq, uint32_t cap, uint32_t list_cap, uint32_t nblocks,
+              uint32_t nlocal, uint32_t *&vals)
+{
     int rc;
     const uint32_t ttot = L.tri_total, ntiles = L.tiles_total;
-    if (!frozen) {
-        const double want = std::min(2147483647.0, (double)x.pair_ratio * (double)ttot + 4096.0);
-        for (int k = 0; k < 2; k++) {
-            if ((rc = arena_reserve(x, x.keys[k], (size_t)want * 4))) return rc;
-            if ((rc = arena_reserve(x, x.vals[k], (size_t)want * 4))) return rc;
-        }
-        size_t c = x.keys[0].cap;
-        for (int k = 0; k < 2; k++) c = std::min(c, std::min(x.keys[k].cap, x.vals[k].cap));
-        // the estimate, not the arenas' power-of-two size, bounds the launch
-        // (the sort's grid and histograms scale with it)
-        L.pairs_cap = std::min<uint64_t>(std::min<uint64_t>(c / 4, (uint64_t)want), 0x7FFFFFFFull);
-    }
-    const uint32_t cap = (uint32_t)L.pairs_cap;
-    if ((rc = arena_reserve(x, x.tile_start, (size_t)ntiles * 4, frozen))) return rc;
-    if ((rc = arena_reserve(x, x.tile_end, (size_t)ntiles * 4, frozen))) return rc;
-    const uint32_t list_cap = HEAVY_SPLIT * ntiles;   // up to HEAVY_SPLIT items per tile
-    if ((rc = arena_reserve(x, x.tile_list, (size_t)list_cap * sizeof(uint4), frozen))) return rc;
-    const uint32_t nblocks = (cap + SORT_TILE - 1) / SORT_TILE;
-    const uint32_t nlocal = (cap + LOCAL_TILE - 1) / LOCAL_TILE;
-    // digit counts, or the local sort's bucket counts and runs' starts
-    if ((rc = arena_reserve(x, x.sort_tmp, (size_t)2 * RADIX * std::max(nblocks, nlocal) * 4, frozen))) return rc;
-    if (!frozen) {
-        if (x.tile_gen.cap < (size_t)ntiles * 4 || x.gen == 0xFFFFFFFFu) {
-            if ((rc = arena_reserve(x, x.tile_gen, (size_t)ntiles * 4))) return rc;
-            HIPC(hipMemsetAsync(x.tile_gen.ptr, 0, x.tile_gen.cap, x.stream));
-            x.gen = 0;
-        }
-        x.gen++;
-    } else {
-        // replays of different rounds share one generation: clear the stamps
-        if ((rc = arena_reserve(x, x.tile_gen, (size_t)ntiles * 4, true))) return rc;
-        hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(ntiles, 256)), dim3(256), 0, x.stream, as<uint32_t>(x.tile_gen),
-                           ntiles, 0u);
-    }
-
-    // ---- K2: set-up, with the vertex transform
     unsigned long long *tri_tiles = as<unsigned long long>(x.tri_tiles);
     unsigned long long *blk_pairs = as<unsigned long long>(x.blk_pairs);
-    // k_setup and k_expand reset the per-launch counters as they go; a
-    // launch that stopped between them leaves them to k_launch_begin
-    if (!x.ctr_clean) hipLaunchKernelGGL(k_launch_begin, dim3(1), dim3(64), 0, x.stream, x.ctr);
-    x.ctr_clean = false;
-    // a wave per corner while the blocks leave SIMDs idle
-    const bool split = L.sblocks <= SETUP_SPLIT_CU * x.cu_count;
-    auto setup_kernel = [&](auto kern, int nw) {
-        hipLaunchKernelGGL(kern, dim3(L.sblocks), dim3(nw * SETUP_BLOCK), 0, x.stream, L.sp, L.vp, L.sblock_pre,
-                           L.smap, L.ns, as<uint32_t>(x.blk_kept), blk_pairs, L.ns == 1u ? L.rs1 : nullptr,
-                           L.ns == 1u ? L.vs1 : nullptr);
-    };
-    if (L.multi_vs) {
-        if (split) setup_kernel(k_setup<true, 3>, 3);
-        else setup_kernel(k_setup<true, 1>, 1);
-    } else {
-        if (split) setup_kernel(k_setup<false, 3>, 3);
-        else setup_kernel(k_setup<false, 1>, 1);
-    }
-    HIPC(hipGetLastError());
-
-    // ---- K3: pair offsets and total (read on the device: the host never
-    // waits), expansion in submission order, stable sort by tile, tile
-    // ranges and the work list
     unsigned long long *pair_base = as<unsigned long long>(x.pair_base);
     unsigned long long *blk_off = as<unsigned long long>(x.blk_off);
     const bool fold = L.sblocks <= EXPAND_FOLD;
     if (!fold && (rc = device_scan<unsigned long long>(x, blk_pairs, blk_off, L.sblocks, frozen, &x.ctr->npairs)))
         return rc;
     const unsigned long long *np = &x.ctr->npairs;
-    uint32_t *keys = as<uint32_t>(x.keys[0]), *vals = as<uint32_t>(x.vals[0]);
+    uint32_t *keys = as<uint32_t>(x.keys[0]);
+    vals = as<uint32_t>(x.vals[0]);
     uint32_t *keys2 = as<uint32_t>(x.keys[1]), *vals2 = as<uint32_t>(x.vals[1]);
     hipLaunchKernelGGL(k_expand, dim3(L.sblocks), dim3(SETUP_BLOCK), 0, x.stream, L.sp, L.sblock_pre, L.smap, L.ns,
                        fold ? nullptr : (const unsigned long long *)blk_off, (const unsigned long long *)blk_pairs,
@@ -5365,7 +5807,6 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
                        (const uint32_t *)as<uint32_t>(x.n_rt), (const uint32_t *)as<uint32_t>(x.rec_base),
                        (const RBox *)as<RBox>(x.box), (uint64_t)cap, keys, vals, as<uint32_t>(x.big_list), x.ctr, seq,
                        (const uint32_t *)as<uint32_t>(x.blk_kept), L.sblocks, ttot);
-    x.ctr_clean = true;
     // (the queue holds only triangles of over EXPAND_WAVE pairs: few waves)
     hipLaunchKernelGGL(k_expand_big, dim3(std::min<uint32_t>(std::max<uint32_t>(ttot, 1u), 256u)), dim3(64), 0,
                        x.stream, (const unsigned long long *)pair_base, (const uint32_t *)as<uint32_t>(x.n_rt),
@@ -5386,7 +5827,7 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
         hipLaunchKernelGGL(k_tile_bins, dim3(((ntiles - 1u) >> shift) + 1u), dim3(BINS_THREADS), 0, x.stream,
                            (const uint32_t *)keys2, (const uint32_t *)vals2, cap, np, shift, nlocal, nullptr,
                            (const uint32_t *)counts, (const uint32_t *)loc, ntiles, vals, as<uint32_t>(x.tile_gen),
-                           x.gen, x.heavy_bin, L.tmap, L.tile_pre, L.ns, as<uint4>(x.tile_list), list_cap, x.ctr);
+                           x.gen, x.heavy_bin, L.tmap, L.tile_pre, L.ns, as<uint4>(x.tile_list), list_cap, x.ctr, x.regions);
     } else if (ntiles > 0u && shift <= BINS_MAX_SHIFT) {
         hipLaunchKernelGGL(k_sort_hist, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys, cap, np,
                            shift, nblocks, counts);
@@ -5396,7 +5837,7 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
         hipLaunchKernelGGL(k_tile_bins, dim3(((ntiles - 1u) >> shift) + 1u), dim3(BINS_THREADS), 0, x.stream,
                            (const uint32_t *)keys2, (const uint32_t *)vals2, cap, np, shift, nblocks,
                            (const uint32_t *)counts, nullptr, nullptr, ntiles, vals, as<uint32_t>(x.tile_gen), x.gen,
-                           x.heavy_bin, L.tmap, L.tile_pre, L.ns, as<uint4>(x.tile_list), list_cap, x.ctr);
+                           x.heavy_bin, L.tmap, L.tile_pre, L.ns, as<uint4>(x.tile_list), list_cap, x.ctr, x.regions);
     } else {
         // stable LSD radix sort by tile: pairs keep submission order within a tile
         int key_bits = 1;
@@ -5416,11 +5857,127 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
         hipLaunchKernelGGL(k_tile_list, dim3(blocks_for(ntiles, 256 * TILE_LIST_PER)), dim3(256), 0, x.stream,
                            (const uint32_t *)as<uint32_t>(x.tile_start), (const uint32_t *)as<uint32_t>(x.tile_end),
                            (const uint32_t *)as<uint32_t>(x.tile_gen), x.gen, ntiles, x.heavy_bin, L.tmap, L.tile_pre,
-                           L.ns, as<uint4>(x.tile_list), list_cap, x.ctr);
+                           L.ns, as<uint4>(x.tile_list), list_cap, x.ctr, x.regions);
+    }
+    HIPC(hipGetLastError());
+    return MTGL_OK;
+}
+
+// The pipeline over the scenes of L, queued on x.stream without waiting for
+// the GPU.  The pair arrays are sized from x.pair_ratio (a frozen run, a
+// replay or one being captured into a graph, allocates nothing and uses the
+// capacity of its sizing run); a launch that needs more pairs, or more clip
+// slots than the pool holds, poisons the Exec with seq (k_bin_scatter) and
+// writes nothing: the host learns of it when it next waits for the stream and
+// runs the launch again with larger arrays.
+int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
+{
+    if (L.ns == 0) return L.unsupported ? MTGL_ERR_UNSUPPORTED : MTGL_OK;
+    int rc;
+    const uint32_t ttot = L.tri_total, ntiles = L.tiles_total;
+    const double est_pairs = (double)x.pair_ratio * (double)ttot;
+    if (!frozen) {
+        // k_bin keeps 4 bytes per pair: room for many more pairs than most
+        // draws have, so that a context's first draws seldom run twice
+        const double want = L.bins ? std::min(2147483647.0, std::max(est_pairs, 32.0 * ttot) + 4.0 * ntiles + 65536.0)
+                                   : std::min(2147483647.0, est_pairs + 4096.0);
+        for (int k = 0; k < (L.bins ? 1 : 2); k++) {
+            if (!L.bins && (rc = arena_reserve(x, x.keys[k], (size_t)want * 4))) return rc;
+            if ((rc = arena_reserve(x, x.vals[k], (size_t)want * 4))) return rc;
+        }
+        // the estimate, not the arenas' power-of-two size, bounds the tile
+        // sort (its grid and histograms scale with it)
+        L.pairs_cap = std::min<uint64_t>(pairs_room(x, L.bins), (uint64_t)want);
+    }
+    const uint32_t cap = (uint32_t)L.pairs_cap;
+    // up to HEAVY_SPLIT items per tile, in one region or in each one's squares
+    const uint32_t list_cap = L.bins ? L.region_items : HEAVY_SPLIT * ntiles;
+    if ((rc = arena_reserve(x, x.tile_list, (size_t)list_cap * (L.bins ? BIN_REGIONS : 1u) * sizeof(uint4), frozen)))
+        return rc;
+    const uint32_t nblocks = (cap + SORT_TILE - 1) / SORT_TILE;
+    const uint32_t nlocal = (cap + LOCAL_TILE - 1) / LOCAL_TILE;
+    if (!L.bins) {
+        if ((rc = arena_reserve(x, x.tile_start, (size_t)ntiles * 4, frozen))) return rc;
+        if ((rc = arena_reserve(x, x.tile_end, (size_t)ntiles * 4, frozen))) return rc;
+        // digit counts, or the local sort's bucket counts and runs' starts
+        if ((rc = arena_reserve(x, x.sort_tmp, (size_t)2 * RADIX * std::max(nblocks, nlocal) * 4, frozen))) return rc;
+    }
+    if (!frozen) {
+        if (x.tile_gen.cap < (size_t)ntiles * 4 || x.gen == 0xFFFFFFFFu) {
+            if ((rc = arena_reserve(x, x.tile_gen, (size_t)ntiles * 4))) return rc;
+            HIPC(hipMemsetAsync(x.tile_gen.ptr, 0, x.tile_gen.cap, x.stream));
+            x.gen = 0;
+        }
+        x.gen++;
+    } else {
+        // replays of different rounds share one generation: clear the stamps
+        if ((rc = arena_reserve(x, x.tile_gen, (size_t)ntiles * 4, true))) return rc;
+        hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(ntiles, 256)), dim3(256), 0, x.stream, as<uint32_t>(x.tile_gen),
+                           ntiles, 0u);
+    }
+
+    // ---- K2: set-up, with the vertex transform
+    unsigned long long *blk_pairs = as<unsigned long long>(x.blk_pairs);
+    // k_setup and k_expand reset the per-launch counters as they go; a
+    // launch that stopped between them leaves them to k_launch_begin
+    if (!x.ctr_clean) hipLaunchKernelGGL(k_launch_begin, dim3(1), dim3(64), 0, x.stream, x.ctr);
+    x.ctr_clean = false;
+    // a wave per corner while the blocks leave SIMDs idle
+    const bool split = L.sblocks <= SETUP_SPLIT_CU * x.cu_count;
+    auto setup_kernel = [&](auto kern, int nw) {
+        hipLaunchKernelGGL(kern, dim3(L.sblocks), dim3(nw * SETUP_BLOCK), 0, x.stream, L.sp, L.vp, L.sblock_pre,
+                           L.smap, L.ns, as<uint32_t>(x.blk_kept), blk_pairs, as<uint2>(x.blk_box), x.sums, x.regions,
+                           L.ns == 1u ? L.rs1 : nullptr, L.ns == 1u ? L.vs1 : nullptr);
+    };
+    if (!L.bins) {
+        if (L.multi_vs) setup_kernel(k_setup<true, 1, false>, 1);
+        else setup_kernel(k_setup<false, 1, false>, 1);
+    } else if (L.multi_vs) {
+        if (split) setup_kernel(k_setup<true, 3, true>, 3);
+        else setup_kernel(k_setup<true, 1, true>, 1);
+    } else {
+        if (split) setup_kernel(k_setup<false, 3, true>, 3);
+        else setup_kernel(k_setup<false, 1, true>, 1);
+    }
+    HIPC(hipGetLastError());
+
+    // ---- K3: every tile's records in submission order and the work list
+    uint32_t *vals = as<uint32_t>(x.vals[0]);
+    if (L.bins) {
+        BinParams bp = {};
+        bp.scenes = L.sp;
+        bp.bin_pre = L.bin_pre;
+        bp.bin_scene = L.bmap;
+        bp.sblock_pre = L.sblock_pre;
+        bp.nscenes = L.ns;
+        bp.ntri = L.ntri1;
+        bp.fb_w = L.fb_w1;
+        bp.fb_h = L.fb_h1;
+        bp.tiles_x = L.tiles_x1;
+        bp.side = L.side1;
+        bp.cols = L.cols1;
+        bp.tbox = as<uint2>(x.tbox);
+        bp.blk_box = as<uint2>(x.blk_box);
+        bp.n_rt = as<uint32_t>(x.n_rt);
+        bp.rec_base = as<uint32_t>(x.rec_base);
+        bp.rt = as<RTri>(x.rt);
+        bp.cap = cap / BIN_REGIONS;
+        bp.regions = x.regions;
+        bp.vals = vals;
+        bp.tile_gen = as<uint32_t>(x.tile_gen);
+        bp.gen = x.gen;
+        bp.heavy_bin = x.heavy_bin;
+        bp.list_cap = list_cap;
+        bp.seq = seq;
+        bp.list = as<uint4>(x.tile_list);
+        bp.ctr = x.ctr;
+        hipLaunchKernelGGL(k_bin, dim3(L.nbins), dim3(BIN_THREADS), 0, x.stream, bp);
+    } else if ((rc = tile_sort(x, L, frozen, seq, cap, list_cap, nblocks, nlocal, vals))) {
+        return rc;
     }
     HIPC(hipGetLastError());
     // raster grids: no more blocks than items, which the estimated pairs bound
-    const uint64_t est_items = std::min<uint64_t>(cap, (uint64_t)((double)x.pair_ratio * (double)ttot) + 64u);
+    const uint64_t est_items = std::min<uint64_t>(cap, (uint64_t)est_pairs + 64u);
 
     // ---- K4
     RasterParams rp = {};
@@ -5434,8 +5991,10 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
     rp.list = as<uint4>(x.tile_list);
     rp.ntiles = ntiles;
     rp.list_cap = list_cap;
-    rp.part = 0;
+    rp.regions = x.regions;
     rp.ctr = x.ctr;
+    rp.kept = L.bins ? x.sums : nullptr;
+    rp.meets = x.sums + 64;
     rp.stats = x.stat_slots;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     if (x.timing && !frozen && x.timing_count++ % x.timing_every == 0u) (void)take_event_pair(x, ev0, ev1);
@@ -5478,21 +6037,26 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
         fns[nl] = L.plain ? (const void *)k_raster<true> : (const void *)k_raster<false>;
         grids[nl++] = grid(L.plain ? 5 : 2);
     }
-    void *args[] = {&rp};
+    // (the first of several kernels ends the binning's use of the counters)
+    RasterParams rp2 = rp;
+    rp2.kept = rp2.meets = nullptr;
+    void *args1[] = {&rp}, *args2[] = {&rp2};
     if (ev0 && nl > 0) {
         // timed: the events are taken at the first kernel's start and the
         // last one's end, not around the launches' dispatch
         for (int i = 0; i < nl; i++)
-            HIPC(hipExtLaunchKernel(fns[i], grids[i], dim3(64), args, 0, x.stream, i == 0 ? ev0 : nullptr,
+            HIPC(hipExtLaunchKernel(fns[i], grids[i], dim3(64), i == 0 ? args1 : args2, 0, x.stream, i == 0 ? ev0 : nullptr,
                                     i == nl - 1 ? ev1 : nullptr, 0));
         x.pending_events.emplace_back(ev0, ev1);
     } else {
-        for (int i = 0; i < nl; i++) HIPC(hipLaunchKernel(fns[i], grids[i], dim3(64), args, 0, x.stream));
+        for (int i = 0; i < nl; i++) HIPC(hipLaunchKernel(fns[i], grids[i], dim3(64), i == 0 ? args1 : args2, 0, x.stream));
         if (ev0) {
             x.free_events.push_back(ev0);
             x.free_events.push_back(ev1);
         }
     }
+    x.last_work = L.work;
+    x.ctr_clean = true;   // (left so by k_expand, or by the raster stage's first kernel)
     return L.unsupported ? MTGL_ERR_UNSUPPORTED : MTGL_OK;
 }
 
@@ -5689,7 +6253,9 @@ int exec_take_poison(Exec &x, uint32_t &poison)
     HIPC(hipMemcpy(x.ctr_host, x.ctr, sizeof(Counters), hipMemcpyDeviceToHost));
     poison = x.ctr_host->poison;
     if (poison) {
-        HIPC(hipMemsetAsync((uint8_t *)x.ctr + offsetof(Counters, poison), 0, sizeof(uint32_t), x.stream));
+        // (poison, poison_pairs and poison_flags)
+        HIPC(hipMemsetAsync((uint8_t *)x.ctr + offsetof(Counters, poison), 0,
+                            offsetof(Counters, poison_flags) + sizeof(uint32_t) - offsetof(Counters, poison), x.stream));
         HIPC(hipStreamSynchronize(x.stream));
     }
     return MTGL_OK;
@@ -5921,13 +6487,10 @@ int batch_build_inner(mtgl_batch *b, int autotune)
     }
     // a later round may have grown a buffer that an earlier round's tables
     // point into: prepare every round's tables again, at the final sizes
-    size_t c = x.keys[0].cap;
-    for (int k = 0; k < 2; k++) c = std::min(c, std::min(x.keys[k].cap, x.vals[k].cap));
-    const uint64_t cap = std::min<uint64_t>(c / 4, 0x7FFFFFFFull);
     for (BatchRound &R : b->rounds) {
         if (R.scenes.empty()) continue;
         if ((rc = prepare_launch(x, R.launch, R.scenes.data(), (uint32_t)R.scenes.size()))) return rc;
-        R.launch.pairs_cap = cap;
+        R.launch.pairs_cap = pairs_room(x, R.launch.bins);
     }
     HIPC(hipStreamSynchronize(x.stream));
     ring_release(x);
@@ -6298,6 +6861,7 @@ static int read_window(mtgl_dev *d, int32_t x, int32_t y, int32_t flip, int32_t 
         }
         d->ops.clear();   // every queued op took effect
         ring_release(ex);
+        saw_meets(ex, ((volatile uint32_t *)ex.report)[1]);
         return MTGL_OK;
     }
     if ((rc = confirm(d))) return rc;
@@ -6793,6 +7357,7 @@ static int confirm(mtgl_dev *d)
     }
     d->ops.clear();
     ring_release(x);
+    saw_meets(x, x.ctr_host->meets);
     return MTGL_OK;
 }
 
