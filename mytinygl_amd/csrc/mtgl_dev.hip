@@ -4537,16 +4537,35 @@ struct GPx {
 };
 static_assert(sizeof(GPx) == sizeof(mtgl_gbuffer_px), "G-buffer pixel layout");
 
-// one captured view as the kernels see it
+// A covered pixel of a view as the shading kernels read it: its three
+// vertices are positions in the view's list of vertices that covered pixels
+// use (~0: an element outside the parameter array)
+struct __align__(16) DiffPx {
+    uint32_t pixel;
+    uint32_t v[3];
+    float b[3];
+    float fx;
+    uint32_t texel[4];
+    float fy;
+    uint32_t pad[3];
+};
+static_assert(sizeof(DiffPx) == 64, "covered pixel layout");
+
+// One captured view as the kernels see it.  The capture lists the covered
+// pixels and the vertices they use, so that the kernels run over those alone:
+// of the 64-view workload's pixels a tenth are covered, and they use a third
+// of its vertices.
 struct DiffView {
-    const GPx *gb;                 // w * h
-    const uint32_t *elems;         // 3 per triangle: element of each vertex
-    const float *pos;              // 3 per element, object space
-    const float *nrm;              // 3 per element
+    const uint2 *px;               // per pixel: index of its covered pixel, or ~0 and its packed colour
+    const DiffPx *cov;             // ncov covered pixels, in pixel order
+    const uint32_t *vlist;         // nvis elements, ascending
+    const uint32_t *vmap;          // per element: its position in vlist, or ~0
+    const float *pos;              // 3 per listed vertex, object space
+    const float *nrm;              // 3 per listed vertex
     const mtgl_vertex_state *vs;
-    uint32_t ntri;
+    unsigned long long off;        // first of the view's vertices in the arrays over every view's
+    uint32_t ncov, nvis;
     int32_t w, h;
-    uint32_t pad;
 };
 
 // Per pixel of a context's latest draw (a single-scene launch of a
@@ -4622,7 +4641,62 @@ __global__ void __launch_bounds__(256) k_diff_geom(const VertexParams *vp, uint3
     }
 }
 
-// eye-space position and normal of element e, and the material of its
+// Per pixel whether it is covered, and the elements covered pixels use
+// (vflag, zero before).
+__global__ void __launch_bounds__(256) k_diff_mark(const GPx *gb, uint32_t npx, const uint32_t *elems, uint32_t nvert,
+                                                   uint32_t *pflag, uint32_t *vflag)
+{
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= npx) return;
+    const int32_t tri = gb[p].tri;
+    pflag[p] = tri >= 0 ? 1u : 0u;
+    if (tri < 0) return;
+    for (int k = 0; k < 3; k++) {
+        const uint32_t e = elems[3u * (uint32_t)tri + (uint32_t)k];
+        if (e < nvert) vflag[e] = 1u;
+    }
+}
+
+// The view's lists, from the scans of those flags (pidx, vidx).
+__global__ void __launch_bounds__(256) k_diff_compact(const GPx *gb, uint32_t npx, const uint32_t *elems,
+                                                      uint32_t nvert, const uint32_t *pidx, const uint32_t *vflag,
+                                                      const uint32_t *vidx, const float *pos, const float *nrm,
+                                                      uint2 *px, DiffPx *cov, uint32_t *vlist, uint32_t *vmap,
+                                                      float *vpos, float *vnrm)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < npx) {
+        const GPx g = gb[i];
+        px[i] = g.tri >= 0 ? make_uint2(pidx[i], 0u) : make_uint2(0xFFFFFFFFu, g.texel[0]);
+        if (g.tri >= 0) {
+            DiffPx q = {};
+            q.pixel = i;
+            for (int k = 0; k < 3; k++) {
+                const uint32_t e = elems[3u * (uint32_t)g.tri + (uint32_t)k];
+                q.v[k] = e < nvert ? vidx[e] : 0xFFFFFFFFu;
+                q.b[k] = g.b[k];
+            }
+            for (int k = 0; k < 4; k++) q.texel[k] = g.texel[k];
+            q.fx = g.fx;
+            q.fy = g.fy;
+            cov[pidx[i]] = q;
+        }
+    }
+    if (i < nvert) {
+        const bool on = vflag[i] != 0u;
+        vmap[i] = on ? vidx[i] : 0xFFFFFFFFu;
+        if (on) {
+            const uint32_t k = vidx[i];
+            vlist[k] = i;
+            for (int c = 0; c < 3; c++) {
+                vpos[3u * k + c] = pos[3u * i + c];
+                vnrm[3u * k + c] = nrm[3u * i + c];
+            }
+        }
+    }
+}
+
+// eye-space position and normal of listed vertex k (element e), and the material of its
 // lighting with the vertex colour through GL_COLOR_MATERIAL, as k_vertex
 // computes them
 struct DiffVertex {
@@ -4631,10 +4705,11 @@ struct DiffVertex {
     Col amb, dif, spe, emi;
 };
 
-__device__ __forceinline__ void diff_vertex(const DiffView &D, uint32_t e, const float *vcol, DiffVertex &o)
+__device__ __forceinline__ void diff_vertex(const DiffView &D, uint32_t k0, const float *vcol, DiffVertex &o)
 {
     const mtgl_vertex_state *vs = D.vs;
-    const float *pp = D.pos + 3u * e, *nn = D.nrm + 3u * e;
+    const uint32_t e = D.vlist[k0];
+    const float *pp = D.pos + 3u * k0, *nn = D.nrm + 3u * k0;
     float eye[4];
     xform(vs->modelview, pp[0], pp[1], pp[2], 1.0f, eye);
     float en4[4];
@@ -4652,14 +4727,15 @@ __device__ __forceinline__ void diff_vertex(const DiffView &D, uint32_t e, const
     if (mode == GL_DIFFUSE || mode == GL_AMBIENT_AND_DIFFUSE) o.dif = k;
 }
 
-// lit colour of every (view, element): grid (elements, views).  With aux
-// (the backward's), also the unclamped sum and each light's att * N.L, in
-// three planes of views * nvert float4 each, for k_diff_lit_bwd.
-__global__ void __launch_bounds__(256) k_diff_lit(const DiffView *views, uint32_t nvert, const float *vcol,
+// lit colour of every listed vertex of every view: grid (vertices, views).
+// With aux (the backward's), also the unclamped sum and each light's att *
+// N.L, in three planes of nall float4 each, for k_diff_lit_bwd.
+__global__ void __launch_bounds__(256) k_diff_lit(const DiffView *views, unsigned long long nall, const float *vcol,
                                                   const float *light_rgb, float4 *lit, float4 *aux)
 {
     __shared__ float s_ld[3 * MTGL_MAX_LIGHTS];
     const DiffView &D = views[blockIdx.y];
+    if (blockIdx.x * blockDim.x >= D.nvis) return;   // (uniform)
     if (threadIdx.x < MTGL_MAX_LIGHTS) {
         const mtgl_light &lt = D.vs->lighting.lights[threadIdx.x];
         float Ld[3] = {lt.position[0], lt.position[1], lt.position[2]};
@@ -4667,34 +4743,33 @@ __global__ void __launch_bounds__(256) k_diff_lit(const DiffView *views, uint32_
         for (int k = 0; k < 3; k++) s_ld[3 * threadIdx.x + k] = Ld[k];
     }
     __syncthreads();
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nvert) return;
+    const uint32_t k0 = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k0 >= D.nvis) return;
     DiffVertex q;
-    diff_vertex(D, e, vcol, q);
+    diff_vertex(D, k0, vcol, q);
     float ndl[MTGL_MAX_LIGHTS];
     const Col u = lighting_sum<true>(&D.vs->lighting, D.vs->flags, q.ep, q.en, q.amb, q.dif, q.spe, q.emi,
                                      D.vs->lighting.front.shininess, light_rgb, ndl, s_ld);
     const Col r = col_clamp(u);
-    const size_t i = (size_t)blockIdx.y * nvert + e;
+    const size_t i = (size_t)D.off + k0;
     lit[i] = make_float4(r.r, r.g, r.b, r.a);
     if (aux) {
-        const size_t plane = (size_t)gridDim.y * nvert;
         aux[i] = make_float4(u.r, u.g, u.b, u.a);
-        aux[plane + i] = make_float4(ndl[0], ndl[1], ndl[2], ndl[3]);
-        aux[2 * plane + i] = make_float4(ndl[4], ndl[5], ndl[6], ndl[7]);
+        aux[nall + i] = make_float4(ndl[0], ndl[1], ndl[2], ndl[3]);
+        aux[2 * nall + i] = make_float4(ndl[4], ndl[5], ndl[6], ndl[7]);
     }
 }
 
 __device__ __forceinline__ Col col4(float4 v) { return {v.x, v.y, v.z, v.w}; }
 
-// colour and texture sample of a covered pixel (GL_MODULATE operands)
-__device__ __forceinline__ void diff_pixel(const GPx &g, const uint32_t *el, const float4 *litv, uint32_t nvert,
-                                           const float4 *tex, Col &c, Col &tc)
+// colour and texture sample of a covered pixel (GL_MODULATE operands); litv:
+// the view's listed vertices
+__device__ __forceinline__ void diff_pixel(const DiffPx &g, const float4 *litv, const float4 *tex, Col &c, Col &tc)
 {
     Col l[3];
     for (int k = 0; k < 3; k++) {
-        const uint32_t e = el[k];
-        l[k] = e < nvert ? col4(litv[e]) : Col{0.0f, 0.0f, 0.0f, 0.0f};
+        const uint32_t v = g.v[k];
+        l[k] = v != 0xFFFFFFFFu ? col4(litv[v]) : Col{0.0f, 0.0f, 0.0f, 0.0f};
     }
     const float b0 = g.b[0], b1 = g.b[1], b2 = g.b[2];
     c.r = l[0].r * b0 + l[1].r * b1 + l[2].r * b2;
@@ -4706,21 +4781,22 @@ __device__ __forceinline__ void diff_pixel(const GPx &g, const uint32_t *el, con
     tc = col_lerp(top, bot, g.fy);
 }
 
-// images: grid (pixels, views)
-__global__ void __launch_bounds__(256) k_diff_shade(const DiffView *views, uint32_t nvert, const float4 *lit,
-                                                    const float4 *tex, float4 *images)
+// images: grid (pixels, views); HBM-bound, 16 bytes written per pixel and 8
+// read (72 for a covered one)
+__global__ void __launch_bounds__(256) k_diff_shade(const DiffView *views, const float4 *lit, const float4 *tex,
+                                                    float4 *images)
 {
     const DiffView &D = views[blockIdx.y];
     const uint32_t npx = (uint32_t)D.w * (uint32_t)D.h;
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= npx) return;
-    const GPx g = D.gb[p];
+    const uint2 s = D.px[p];
     Col out;
-    if (g.tri < 0) {
-        out = col_unpack(g.texel[0]);
+    if (s.x == 0xFFFFFFFFu) {
+        out = col_unpack(s.y);
     } else {
         Col c, tc;
-        diff_pixel(g, D.elems + 3u * (uint32_t)g.tri, lit + (size_t)blockIdx.y * nvert, nvert, tex, c, tc);
+        diff_pixel(D.cov[s.x], lit + D.off, tex, c, tc);
         out = col_clamp(col_mul(c, tc));
     }
     images[(size_t)blockIdx.y * npx + p] = make_float4(out.r, out.g, out.b, out.a);
@@ -4728,54 +4804,65 @@ __global__ void __launch_bounds__(256) k_diff_shade(const DiffView *views, uint3
 
 __device__ __forceinline__ float clamp_grad(float v, float g) { return (v >= 0.0f && v <= 1.0f) ? g : 0.0f; }
 
-// adjoint of k_diff_shade: dL/dlit per (view, element) into dlit, dL/dtex.
+// adjoint of k_diff_shade: dL/dlit per listed vertex into dlit, dL/dtex.
 // Channels are independent through the shading, so a thread takes one
-// (pixel, channel): the four lanes of a pixel add to the four consecutive
-// floats of each target together, one L2 request per target and instruction.
-// Grid (4 x pixels, views).
-__global__ void __launch_bounds__(256) k_diff_shade_bwd(const DiffView *views, uint32_t nvert, const float *lit,
-                                                        const float *tex, const float *grad, float *dlit,
-                                                        float *g_tex)
+// (covered pixel, channel): the four lanes of a pixel add to the four
+// consecutive floats of each target together, one L2 request per target and
+// instruction.  Grid (4 x covered pixels, views).
+__global__ void __launch_bounds__(256) k_diff_shade_bwd(const DiffView *views, const float *lit, const float *tex,
+                                                        const float *grad, float *dlit, float *g_tex)
 {
     const DiffView &D = views[blockIdx.y];
-    const uint32_t npx = (uint32_t)D.w * (uint32_t)D.h;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t p = t >> 2, ch = t & 3u;
-    if (p >= npx) return;
-    const GPx g = D.gb[p];
-    if (g.tri < 0) return;
-    const uint32_t *el = D.elems + 3u * (uint32_t)g.tri;
-    const float *litv = lit + 4u * (size_t)blockIdx.y * nvert;
+    const uint32_t ch = t & 3u;
+    if ((t >> 2) >= D.ncov) return;
+    const DiffPx g = D.cov[t >> 2];
+    const size_t npx = (size_t)D.w * (size_t)D.h;
+    const float gr = grad[4u * ((size_t)blockIdx.y * npx + g.pixel) + ch];
     // the operations of diff_pixel, one channel
-    uint32_t e[3];
     float l[3];
-    for (int k = 0; k < 3; k++) {
-        e[k] = el[k];
-        l[k] = e[k] < nvert ? litv[4u * e[k] + ch] : 0.0f;
-    }
+    for (int k = 0; k < 3; k++) l[k] = g.v[k] != 0xFFFFFFFFu ? lit[4u * ((size_t)D.off + g.v[k]) + ch] : 0.0f;
     const float c = l[0] * g.b[0] + l[1] * g.b[1] + l[2] * g.b[2];
     const float fx = g.fx, fy = g.fy;
     const float t0 = tex[4u * (size_t)g.texel[0] + ch], t1 = tex[4u * (size_t)g.texel[1] + ch];
     const float t2 = tex[4u * (size_t)g.texel[2] + ch], t3 = tex[4u * (size_t)g.texel[3] + ch];
     const float top = t0 * (1.0f - fx) + t1 * fx, bot = t2 * (1.0f - fx) + t3 * fx;
     const float tc = top * (1.0f - fy) + bot * fy;
-    const float gm = clamp_grad(c * tc, grad[4u * ((size_t)blockIdx.y * npx + p) + ch]);
+    const float gm = clamp_grad(c * tc, gr);
     const float dc = gm * tc, dt = gm * c;
     for (int k = 0; k < 3; k++)
-        if (e[k] < nvert) unsafeAtomicAdd(dlit + 4u * ((size_t)blockIdx.y * nvert + e[k]) + ch, dc * g.b[k]);
+        if (g.v[k] != 0xFFFFFFFFu) unsafeAtomicAdd(dlit + 4u * ((size_t)D.off + g.v[k]) + ch, dc * g.b[k]);
     const float wt[4] = {(1.0f - fx) * (1.0f - fy), fx * (1.0f - fy), (1.0f - fx) * fy, fx * fy};
     for (int k = 0; k < 4; k++) unsafeAtomicAdd(g_tex + 4u * (size_t)g.texel[k] + ch, dt * wt[k]);
+}
+
+// sum over the 64 lanes, in lane 63 (the DPP pattern of dpp_incl_scan; lanes
+// without a source add zero)
+__device__ __forceinline__ float dpp_wave_sum_f(float v)
+{
+#define SUMF_STEP(ctrl, rm, bm) \
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rm, bm, false));
+    SUMF_STEP(0x111, 0xf, 0xf)   // row_shr:1
+    SUMF_STEP(0x112, 0xf, 0xf)   // row_shr:2
+    SUMF_STEP(0x114, 0xf, 0xe)   // row_shr:4, lanes 4..15
+    SUMF_STEP(0x118, 0xf, 0xc)   // row_shr:8, lanes 8..15
+    SUMF_STEP(0x142, 0xa, 0xf)   // row_bcast:15 into rows 1, 3
+    SUMF_STEP(0x143, 0xc, 0xf)   // row_bcast:31 into rows 2, 3
+#undef SUMF_STEP
+    return v;
 }
 
 // adjoint of k_diff_lit from the unclamped sums and N.L terms the
 // backward's k_diff_lit stored (aux): a block holds DIFF_BWD_E elements x
 // DIFF_BWD_G view groups (thread (x, y) takes element x over views y,
-// y + DIFF_BWD_G, ...); dL/dvcol is summed over the groups in LDS and
-// written, dL/dlight_rgb is reduced per block and added
+// y + DIFF_BWD_G, ... whose covered pixels use it: vmap); dL/dvcol is summed
+// over the groups in LDS and written, dL/dlight_rgb is summed over each wave
+// (a wave is one view group), then per block in LDS, and added
 constexpr int DIFF_BWD_E = 64, DIFF_BWD_G = 8;
 __global__ void __launch_bounds__(DIFF_BWD_E * DIFF_BWD_G) k_diff_lit_bwd(const DiffView *views, uint32_t nviews,
-                                                                          uint32_t nvert, const float *vcol,
-                                                                          const float *light_rgb, const float *dlit,
+                                                                          uint32_t nvert, unsigned long long nall,
+                                                                          const float *vcol, const float *light_rgb,
+                                                                          const float *dlit,
                                                                           const float4 *aux, float *g_vcol,
                                                                           float *g_light)
 {
@@ -4785,20 +4872,21 @@ __global__ void __launch_bounds__(DIFF_BWD_E * DIFF_BWD_G) k_diff_lit_bwd(const 
     if (tid < 3 * MTGL_MAX_LIGHTS) s_gl[tid] = 0.0f;
     __syncthreads();
     const uint32_t e = blockIdx.x * DIFF_BWD_E + threadIdx.x;
-    const size_t plane = (size_t)nviews * nvert;
     Col gv = {0.0f, 0.0f, 0.0f, 0.0f};
+    float gl[3 * MTGL_MAX_LIGHTS];
+    for (int i = 0; i < 3 * MTGL_MAX_LIGHTS; i++) gl[i] = 0.0f;
+    bool any_light = false;
     if (e < nvert) {
-        float gl[3 * MTGL_MAX_LIGHTS];
-        for (int i = 0; i < 3 * MTGL_MAX_LIGHTS; i++) gl[i] = 0.0f;
-        bool any_light = false;
         const float *c = vcol + 4u * e;
         const Col vc = {sanitize(c[0], 0.0f), sanitize(c[1], 0.0f), sanitize(c[2], 0.0f), sanitize(c[3], 1.0f)};
         const Col k = col_clamp(vc);
         for (uint32_t v = threadIdx.y; v < nviews; v += DIFF_BWD_G) {
-            const size_t i = (size_t)v * nvert + e;
+            const uint32_t at = views[v].vmap[e];
+            if (at == 0xFFFFFFFFu) continue;
+            const size_t i = (size_t)views[v].off + at;
             const float4 dl = reinterpret_cast<const float4 *>(dlit)[i];
             if (dl.x == 0.0f && dl.y == 0.0f && dl.z == 0.0f && dl.w == 0.0f) continue;
-            const float4 u = aux[i], n03 = aux[plane + i], n47 = aux[2 * plane + i];
+            const float4 u = aux[i], n03 = aux[nall + i], n47 = aux[2 * nall + i];
             const float ndl[MTGL_MAX_LIGHTS] = {n03.x, n03.y, n03.z, n03.w, n47.x, n47.y, n47.z, n47.w};
             const mtgl_vertex_state *vs = views[v].vs;
             const mtgl_lighting &L = vs->lighting;
@@ -4843,9 +4931,13 @@ __global__ void __launch_bounds__(DIFF_BWD_E * DIFF_BWD_G) k_diff_lit_bwd(const 
             gv.b += clamp_grad(vc.b, gk.b);
             gv.a += clamp_grad(vc.a, gk.a);
         }
-        if (any_light)
-            for (int i = 0; i < 3 * MTGL_MAX_LIGHTS; i++)
-                if (gl[i] != 0.0f) atomicAdd(&s_gl[i], gl[i]);
+    }
+    static_assert(DIFF_BWD_E == 64, "a wave is one view group");
+    if (__ballot(any_light)) {
+        for (int i = 0; i < 3 * MTGL_MAX_LIGHTS; i++) {
+            const float t = dpp_wave_sum_f(gl[i]);
+            if (threadIdx.x == 63 && t != 0.0f) atomicAdd(&s_gl[i], t);
+        }
     }
     s_gv[threadIdx.y][threadIdx.x] = make_float4(gv.r, gv.g, gv.b, gv.a);
     __syncthreads();
@@ -7530,8 +7622,8 @@ MTGL_API int mtgl_batch_stats_reset(mtgl_batch *b)
 namespace {
 
 struct DiffCapture {
-    Arena gb, elems, pos, nrm, vs;
-    uint32_t ntri = 0;
+    Arena gb, px, cov, vtx, vs;      // vtx: vlist, positions, normals, vmap
+    uint32_t ncov = 0, nvis = 0;
 };
 
 // the capture conditions of include/mtgl_diff.h
@@ -7563,6 +7655,9 @@ struct mtgl_diff {
     int32_t tex_w = 0, tex_h = 0, w = 0, h = 0;
     std::vector<DiffCapture> views;
     Arena table, lit, counter;
+    Arena scratch;                 // of a capture: dense geometry, flags and their scans
+    uint64_t nall = 0;             // listed vertices of every view
+    uint32_t max_cov = 0, max_vis = 0;
     bool table_ok = false;
 };
 
@@ -7572,17 +7667,25 @@ int diff_table(mtgl_diff *df, hipStream_t st)
 {
     if (df->table_ok) return MTGL_OK;
     std::vector<DiffView> t(df->views.size());
+    df->nall = 0;
+    df->max_cov = df->max_vis = 0;
     for (size_t i = 0; i < t.size(); i++) {
         DiffCapture &c = df->views[i];
-        t[i].gb = as<GPx>(c.gb);
-        t[i].elems = as<uint32_t>(c.elems);
-        t[i].pos = as<float>(c.pos);
-        t[i].nrm = as<float>(c.nrm);
+        t[i].px = as<uint2>(c.px);
+        t[i].cov = as<DiffPx>(c.cov);
+        t[i].vlist = as<uint32_t>(c.vtx);
+        t[i].pos = as<float>(c.vtx) + c.nvis;
+        t[i].nrm = as<float>(c.vtx) + 4 * (size_t)c.nvis;
+        t[i].vmap = as<uint32_t>(c.vtx) + 7 * (size_t)c.nvis;
         t[i].vs = as<mtgl_vertex_state>(c.vs);
-        t[i].ntri = c.ntri;
+        t[i].off = df->nall;
+        t[i].ncov = c.ncov;
+        t[i].nvis = c.nvis;
         t[i].w = df->w;
         t[i].h = df->h;
-        t[i].pad = 0;
+        df->nall += c.nvis;
+        df->max_cov = std::max(df->max_cov, c.ncov);
+        df->max_vis = std::max(df->max_vis, c.nvis);
     }
     if (df->table.cap < t.size() * sizeof(DiffView)) {
         if (df->table.ptr) HIPC(hipFree(df->table.ptr));
@@ -7591,7 +7694,7 @@ int diff_table(mtgl_diff *df, hipStream_t st)
         df->table.cap = std::max<size_t>(t.size() * sizeof(DiffView), 256);
     }
     HIPC(hipMemcpy(df->table.ptr, t.data(), t.size() * sizeof(DiffView), hipMemcpyHostToDevice));
-    const size_t lit_bytes = t.size() * (size_t)df->nvert * sizeof(float4);
+    const size_t lit_bytes = std::max<size_t>((size_t)df->nall, 1) * sizeof(float4);
     if (df->lit.cap < lit_bytes) {
         if (df->lit.ptr) HIPC(hipFree(df->lit.ptr));
         df->lit = Arena();
@@ -7642,11 +7745,12 @@ MTGL_API void mtgl_diff_destroy(mtgl_diff *df)
     (void)hipDeviceSynchronize();
     for (DiffCapture &c : df->views) {
         arena_free(c.gb);
-        arena_free(c.elems);
-        arena_free(c.pos);
-        arena_free(c.nrm);
+        arena_free(c.px);
+        arena_free(c.cov);
+        arena_free(c.vtx);
         arena_free(c.vs);
     }
+    arena_free(df->scratch);
     arena_free(df->table);
     arena_free(df->lit);
     arena_free(df->counter);
@@ -7671,36 +7775,55 @@ MTGL_API int mtgl_diff_add_view(mtgl_diff *df, mtgl_dev *d)
     Exec &x = d->ex;
     const LastDraw &l = d->last;
     DiffCapture c;
-    c.ntri = l.ntri;
-    const size_t npx = (size_t)d->w * d->h;
+    const size_t npx = (size_t)d->w * d->h, nvert = df->nvert, nel = std::max<size_t>(3u * (size_t)l.ntri, 1);
     do {
+        if ((rc = arena_reserve(x, df->scratch, (nel + 8 * nvert + 2 * npx) * 4))) break;
+        uint32_t *const elems = as<uint32_t>(df->scratch), *const vflag = elems + nel, *const vidx = vflag + nvert;
+        float *const pos = reinterpret_cast<float *>(vidx + nvert), *const nrm = pos + 3 * nvert;
+        uint32_t *const pflag = reinterpret_cast<uint32_t *>(nrm + 3 * nvert), *const pidx = pflag + npx;
+        uint32_t *const ctr = as<uint32_t>(df->counter);   // clipped pixels, covered pixels, listed vertices
         if ((rc = map_err(hipMalloc(&c.gb.ptr, npx * sizeof(GPx))))) break;
-        if ((rc = map_err(hipMalloc(&c.elems.ptr, std::max<size_t>(3u * (size_t)l.ntri, 1) * 4)))) break;
-        if ((rc = map_err(hipMalloc(&c.pos.ptr, 3u * (size_t)df->nvert * 4)))) break;
-        if ((rc = map_err(hipMalloc(&c.nrm.ptr, 3u * (size_t)df->nvert * 4)))) break;
+        if ((rc = map_err(hipMalloc(&c.px.ptr, npx * sizeof(uint2))))) break;
         if ((rc = map_err(hipMalloc(&c.vs.ptr, sizeof(mtgl_vertex_state))))) break;
         if ((rc = map_err(hipMemcpyAsync(c.vs.ptr, &l.vs, sizeof(mtgl_vertex_state), hipMemcpyHostToDevice,
                                          x.stream))))
             break;
-        if ((rc = map_err(hipMemsetAsync(df->counter.ptr, 0, 4, x.stream)))) break;
+        if ((rc = map_err(hipMemsetAsync(df->counter.ptr, 0, 12, x.stream)))) break;
+        if ((rc = map_err(hipMemsetAsync(vflag, 0, nvert * 4, x.stream)))) break;
         hipLaunchKernelGGL(k_gbuffer, dim3(blocks_for(npx, 256)), dim3(256), 0, x.stream, d->one.sr,
                            (const RTri *)as<RTri>(x.rt), (const uint32_t *)as<uint32_t>(d->writer),
-                           (const uint32_t *)as<uint32_t>(x.tile_gen), l.gen, l.over_base, as<GPx>(c.gb),
-                           as<uint32_t>(df->counter));
-        const uint64_t n = std::max<uint64_t>(3u * (uint64_t)l.ntri, df->nvert);
+                           (const uint32_t *)as<uint32_t>(x.tile_gen), l.gen, l.over_base, as<GPx>(c.gb), ctr);
+        const uint64_t n = std::max<uint64_t>(3u * (uint64_t)l.ntri, nvert);
         hipLaunchKernelGGL(k_diff_geom, dim3(blocks_for(n, 256)), dim3(256), 0, x.stream, d->one.vp, l.ntri,
-                           df->nvert, as<uint32_t>(c.elems), as<float>(c.pos), as<float>(c.nrm));
+                           df->nvert, elems, pos, nrm);
+        hipLaunchKernelGGL(k_diff_mark, dim3(blocks_for(npx, 256)), dim3(256), 0, x.stream,
+                           (const GPx *)as<GPx>(c.gb), (uint32_t)npx, (const uint32_t *)elems, df->nvert, pflag, vflag);
         if ((rc = map_err(hipGetLastError()))) break;
-        uint32_t clipped = 0;
-        if ((rc = map_err(hipMemcpyAsync(&clipped, df->counter.ptr, 4, hipMemcpyDeviceToHost, x.stream)))) break;
+        if ((rc = device_scan<uint32_t>(x, pflag, pidx, npx, false, ctr + 1))) break;
+        if ((rc = device_scan<uint32_t>(x, vflag, vidx, nvert, false, ctr + 2))) break;
+        uint32_t got[3] = {0, 0, 0};
+        if ((rc = map_err(hipMemcpyAsync(got, ctr, 12, hipMemcpyDeviceToHost, x.stream)))) break;
         if ((rc = map_err(hipStreamSynchronize(x.stream)))) break;
-        if (clipped) rc = MTGL_ERR_UNSUPPORTED;   // a triangle crossed a frustum plane
+        if (got[0]) { rc = MTGL_ERR_UNSUPPORTED; break; }   // a triangle crossed a frustum plane
+        c.ncov = got[1];
+        c.nvis = got[2];
+        if ((rc = map_err(hipMalloc(&c.cov.ptr, std::max<size_t>(c.ncov, 1) * sizeof(DiffPx))))) break;
+        if ((rc = map_err(hipMalloc(&c.vtx.ptr, (7 * (size_t)c.nvis + nvert) * 4)))) break;
+        float *const vpos = as<float>(c.vtx) + c.nvis;
+        hipLaunchKernelGGL(k_diff_compact, dim3(blocks_for(std::max(npx, nvert), 256)), dim3(256), 0, x.stream,
+                           (const GPx *)as<GPx>(c.gb), (uint32_t)npx, (const uint32_t *)elems, df->nvert,
+                           (const uint32_t *)pidx, (const uint32_t *)vflag, (const uint32_t *)vidx, (const float *)pos,
+                           (const float *)nrm, as<uint2>(c.px), as<DiffPx>(c.cov), as<uint32_t>(c.vtx),
+                           as<uint32_t>(c.vtx) + 7 * (size_t)c.nvis, vpos, vpos + 3 * (size_t)c.nvis);
+        if ((rc = map_err(hipGetLastError()))) break;
+        // (the shading kernels run on other streams)
+        if ((rc = map_err(hipStreamSynchronize(x.stream)))) break;
     } while (0);
     if (rc) {
         arena_free(c.gb);
-        arena_free(c.elems);
-        arena_free(c.pos);
-        arena_free(c.nrm);
+        arena_free(c.px);
+        arena_free(c.cov);
+        arena_free(c.vtx);
         arena_free(c.vs);
         return rc;
     }
@@ -7740,12 +7863,12 @@ MTGL_API int mtgl_diff_forward(mtgl_diff *df, const float *vcol, const float *li
     int rc = diff_table(df, st);
     if (rc) return rc;
     const uint32_t nv = (uint32_t)df->views.size(), npx = (uint32_t)df->w * (uint32_t)df->h;
-    hipLaunchKernelGGL(k_diff_lit, dim3(blocks_for(df->nvert, 256), nv), dim3(256), 0, st,
-                       (const DiffView *)df->table.ptr, df->nvert, vcol, light_rgb, as<float4>(df->lit),
-                       (float4 *)nullptr);
-    hipLaunchKernelGGL(k_diff_shade, dim3(blocks_for(npx, 256), nv), dim3(256), 0, st,
-                       (const DiffView *)df->table.ptr, df->nvert, (const float4 *)as<float4>(df->lit),
-                       (const float4 *)tex, (float4 *)images);
+    const DiffView *tab = (const DiffView *)df->table.ptr;
+    if (df->max_vis)
+        hipLaunchKernelGGL(k_diff_lit, dim3(blocks_for(df->max_vis, 256), nv), dim3(256), 0, st, tab,
+                           (unsigned long long)df->nall, vcol, light_rgb, as<float4>(df->lit), (float4 *)nullptr);
+    hipLaunchKernelGGL(k_diff_shade, dim3(blocks_for(npx, 256), nv), dim3(256), 0, st, tab,
+                       (const float4 *)as<float4>(df->lit), (const float4 *)tex, (float4 *)images);
     HIPC(hipGetLastError());
     return MTGL_OK;
 }
@@ -7760,23 +7883,25 @@ MTGL_API int mtgl_diff_backward(mtgl_diff *df, const float *vcol, const float *l
     hipStream_t st = (hipStream_t)stream;
     int rc = diff_table(df, st);
     if (rc) return rc;
-    const uint32_t nv = (uint32_t)df->views.size(), npx = (uint32_t)df->w * (uint32_t)df->h;
+    const uint32_t nv = (uint32_t)df->views.size();
     const DiffView *tab = (const DiffView *)df->table.ptr;
-    // work: dL/dlit (views * nvert float4), then the unclamped lit sums and
-    // the N.L terms of the current parameters (three planes of the same size)
-    const size_t plane = (size_t)nv * df->nvert;
-    float4 *aux = reinterpret_cast<float4 *>(work) + plane;
+    // work: dL/dlit (a float4 per listed vertex of every view), then the
+    // unclamped lit sums and the N.L terms of the current parameters (three
+    // planes of the same size)
+    const unsigned long long nall = df->nall;
+    float4 *aux = reinterpret_cast<float4 *>(work) + nall;
     // the lit colours of the current parameters (the forward's, recomputed)
-    hipLaunchKernelGGL(k_diff_lit, dim3(blocks_for(df->nvert, 256), nv), dim3(256), 0, st, tab, df->nvert, vcol,
-                       light_rgb, as<float4>(df->lit), aux);
-    if ((rc = fill_zero(work, plane * 4u, st))) return rc;
+    if (df->max_vis)
+        hipLaunchKernelGGL(k_diff_lit, dim3(blocks_for(df->max_vis, 256), nv), dim3(256), 0, st, tab, nall, vcol,
+                           light_rgb, as<float4>(df->lit), aux);
+    if ((rc = fill_zero(work, (size_t)nall * 4u, st))) return rc;
     if ((rc = fill_zero(g_tex, (size_t)df->tex_w * df->tex_h * 4u, st))) return rc;
     if ((rc = fill_zero(g_light_rgb, 3u * MTGL_MAX_LIGHTS, st))) return rc;
-    hipLaunchKernelGGL(k_diff_shade_bwd, dim3(blocks_for(4ull * npx, 256), nv), dim3(256), 0, st, tab, df->nvert,
-                       (const float *)as<float>(df->lit), tex, grad_images, work, g_tex);
+    if (df->max_cov)
+        hipLaunchKernelGGL(k_diff_shade_bwd, dim3(blocks_for(4ull * df->max_cov, 256), nv), dim3(256), 0, st, tab,
+                           (const float *)as<float>(df->lit), tex, grad_images, work, g_tex);
     hipLaunchKernelGGL(k_diff_lit_bwd, dim3(blocks_for(df->nvert, DIFF_BWD_E)), dim3(DIFF_BWD_E, DIFF_BWD_G), 0, st,
-                       tab, nv, df->nvert, vcol, light_rgb, (const float *)work, (const float4 *)aux, g_vcol,
-                       g_light_rgb);
+                       tab, nv, df->nvert, nall, vcol, light_rgb, (const float *)work, (const float4 *)aux, g_vcol, g_light_rgb);
     HIPC(hipGetLastError());
     return MTGL_OK;
 }
