@@ -296,36 +296,40 @@ __device__ __forceinline__ Col col_clamp(Col c) { return {clamp01(c.r), clamp01(
 __device__ __forceinline__ Col col_lerp(Col a, Col b, float t) { return col_add(col_scale(a, 1.0f - t), col_scale(b, t)); }
 __device__ __forceinline__ Col col_of(const mtgl_color &c) { return {c.r, c.g, c.b, c.a}; }
 
-// clamp then truncate x*255 (reference color_to_rgba32): fmaxf maps NaN to 0,
-// which is also the byte x86 produces for a NaN channel, and the converted
-// value always lies in [0, 255]
-__device__ __forceinline__ uint32_t pack8(float v)
-{
-    float x = fminf(fmaxf(v, 0.0f), 1.0f);
-    return (uint32_t)(x * 255.0f);
-}
-
-__device__ __forceinline__ uint32_t col_pack(Col c)
-{
-    return pack8(c.r) | (pack8(c.g) << 8) | (pack8(c.b) << 16) | (pack8(c.a) << 24);
-}
+// clamp then truncate x*255 (reference color_to_rgba32): NaN becomes 0 (med3
+// with a NaN operand is the least of the others), which is also the byte x86
+// produces for a NaN channel, and the value always lies in [0, 255].  The
+// reference's clamp of the colour before it changes no result.
+__device__ __forceinline__ float byte_of(float v) { return truncf(__builtin_amdgcn_fmed3f(v, 0.0f, 1.0f) * 255.0f); }
 
 // byte/255.0f, correctly rounded: one product by 1/255 and one FMA residual
 // correction reproduce the IEEE quotient for all 256 byte values (checked
 // exhaustively by the test suite)
-__device__ __forceinline__ float u8_to_unit(uint32_t b)
+__device__ __forceinline__ float unit_of(float fb)
 {
     const float r = 1.0f / 255.0f;
-    float fb = (float)b;
     float m = fb * r;
     float e = __builtin_fmaf(-m, 255.0f, fb);
     return __builtin_fmaf(e, r, m);
 }
 
-__device__ __forceinline__ Col col_unpack(uint32_t p)
+// An RGBA8 colour whose four bytes are held as floats: what a packed colour
+// becomes between two steps that would pack and unpack it.
+struct Bytes4 { float r, g, b, a; };
+
+__device__ __forceinline__ Bytes4 bytes_of(Col c) { return {byte_of(c.r), byte_of(c.g), byte_of(c.b), byte_of(c.a)}; }
+__device__ __forceinline__ Bytes4 bytes_load(uint32_t p)
 {
-    return {u8_to_unit(p & 0xFF), u8_to_unit((p >> 8) & 0xFF), u8_to_unit((p >> 16) & 0xFF), u8_to_unit(p >> 24)};
+    return {(float)(p & 0xFFu), (float)((p >> 8) & 0xFFu), (float)((p >> 16) & 0xFFu), (float)(p >> 24)};
 }
+__device__ __forceinline__ uint32_t bytes_pack(Bytes4 q)
+{
+    return (uint32_t)q.r | ((uint32_t)q.g << 8) | ((uint32_t)q.b << 16) | ((uint32_t)q.a << 24);
+}
+__device__ __forceinline__ Col units_of(Bytes4 q) { return {unit_of(q.r), unit_of(q.g), unit_of(q.b), unit_of(q.a)}; }
+
+__device__ __forceinline__ uint32_t col_pack(Col c) { return bytes_pack(bytes_of(c)); }
+__device__ __forceinline__ Col col_unpack(uint32_t p) { return units_of(bytes_load(p)); }
 
 __device__ __forceinline__ float dot3(const float *a, const float *b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
@@ -1661,7 +1665,8 @@ __device__ __forceinline__ bool exec_poisoned(const Counters *ctr)
 // stable LSD radix sort of (key, value) pairs by key
 // ---------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(SORT_THREADS) k_sort_hist(const uint32_t *keys, uint32_t n_max,
+// (a key every kstride words)
+__global__ void __launch_bounds__(SORT_THREADS) k_sort_hist(const uint32_t *keys, uint32_t kstride, uint32_t n_max,
                                                             const unsigned long long *n_dev, int shift,
                                                             uint32_t nblocks, uint32_t *counts)
 {
@@ -1675,7 +1680,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_hist(const uint32_t *keys
 #pragma unroll
     for (int r = 0; r < SORT_ITEMS; r++) {
         const uint32_t i = base + r * SORT_THREADS + threadIdx.x;
-        kk[r] = i < n ? keys[i] : 0u;
+        kk[r] = i < n ? keys[(size_t)i * kstride] : 0u;
     }
 #pragma unroll
     for (int r = 0; r < SORT_ITEMS; r++)
@@ -1684,6 +1689,12 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_hist(const uint32_t *keys
     counts[threadIdx.x * nblocks + blockIdx.x] = hist[threadIdx.x];
 }
 
+// One pass.  SORT_ARRAYS: keys and values in arrays of their own.
+// SORT_PAIRS: (key, value) pairs, so that a key's move is one 8-byte store.
+// SORT_FIRST: keys are the first words of pairs, values vals_in or, when
+// that is null, the key's index; pairs come out.
+enum : int { SORT_ARRAYS = 0, SORT_PAIRS = 1, SORT_FIRST = 2 };
+template <int FMT>
 __global__ void __launch_bounds__(SORT_THREADS) k_sort_scatter(const uint32_t *keys_in, const uint32_t *vals_in,
                                                                uint32_t n_max, const unsigned long long *n_dev,
                                                                int shift, uint32_t nblocks,
@@ -1706,8 +1717,14 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_scatter(const uint32_t *k
 #pragma unroll
     for (int r = 0; r < SORT_ITEMS; r++) {
         const uint32_t i = base + r * SORT_THREADS + threadIdx.x;
-        kk[r] = i < n ? keys_in[i] : 0u;
-        vv[r] = i < n ? vals_in[i] : 0u;
+        if (FMT == SORT_ARRAYS) {
+            kk[r] = i < n ? keys_in[i] : 0u;
+            vv[r] = i < n ? vals_in[i] : 0u;
+        } else {
+            const uint2 q = i < n ? reinterpret_cast<const uint2 *>(keys_in)[i] : make_uint2(0u, 0u);
+            kk[r] = q.x;
+            vv[r] = FMT == SORT_PAIRS ? q.y : vals_in && i < n ? vals_in[i] : i;
+        }
     }
 #pragma unroll
     for (int r = 0; r < SORT_ITEMS; r++) {
@@ -1730,8 +1747,12 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_scatter(const uint32_t *k
             uint32_t pos = running[d] + below;
             for (int w = 0; w < wave; w++) pos += wave_hist[w][d];
             if (pos < n) {
-                keys_out[pos] = key;
-                vals_out[pos] = val;
+                if (FMT == SORT_ARRAYS) {
+                    keys_out[pos] = key;
+                    vals_out[pos] = val;
+                } else {
+                    reinterpret_cast<uint2 *>(keys_out)[pos] = make_uint2(key, val);
+                }
             }
         }
         __syncthreads();
@@ -2648,7 +2669,7 @@ __device__ __forceinline__ void bilinear_taps(const TexLevel &L, bool rep_s, boo
     at[3] = (size_t)wy1 * L.w + wx1;
 }
 
-__device__ uint32_t sample_level(const TexLevel &L, bool rep_s, bool rep_t, float u, float v, bool linear, int &taps)
+__device__ Bytes4 sample_level(const TexLevel &L, bool rep_s, bool rep_t, float u, float v, bool linear, int &taps)
 {
     if (linear) {
         size_t at[4];
@@ -2661,7 +2682,7 @@ __device__ uint32_t sample_level(const TexLevel &L, bool rep_s, bool rep_t, floa
         taps += 4;
         Col top = col_lerp(col_unpack(c00), col_unpack(c10), fx);
         Col bot = col_lerp(col_unpack(c01), col_unpack(c11), fx);
-        return col_pack(col_lerp(top, bot, fy));
+        return bytes_of(col_lerp(top, bot, fy));
     }
     const float tx = u * (float)L.w - 0.5f;
     const float ty = v * (float)L.h - 0.5f;
@@ -2672,7 +2693,7 @@ __device__ uint32_t sample_level(const TexLevel &L, bool rep_s, bool rep_t, floa
     if (y < 0) y = 0;
     if (y >= L.h) y = L.h - 1;
     taps += 1;
-    return L.px[(size_t)y * L.w + x];
+    return bytes_load(L.px[(size_t)y * L.w + x]);
 }
 
 // reference texture_sample_lod (src/textures.c:457-557)
@@ -2685,15 +2706,15 @@ __device__ __forceinline__ void wrap_uv(bool rep_s, bool rep_t, float &u, float 
     else { if (v < 0.0f) v = 0.0f; if (v > 1.0f) v = 1.0f; }
 }
 
-__device__ uint32_t sample_texture(const RasterConsts &K, const TexLevel &L0, const TexLevel &L1, float u, float v,
-                                   float lod, int &taps)
+__device__ Bytes4 sample_texture(const RasterConsts &K, const TexLevel &L0, const TexLevel &L1, float u, float v,
+                                 float lod, int &taps)
 {
     const bool rep_s = K.rep_s, rep_t = K.rep_t;
     wrap_uv(rep_s, rep_t, u, v);
     uint32_t filter = lod > 0.0f ? K.min_filter : K.mag_filter;
     if (filter == GL_NEAREST_MIPMAP_NEAREST || filter == GL_LINEAR_MIPMAP_NEAREST) {
         if (lod >= 0.5f) {
-            if (!L1.px) return 0xFFFFFFFFu;
+            if (!L1.px) return {255.0f, 255.0f, 255.0f, 255.0f};
             return sample_level(L1, rep_s, rep_t, u, v, filter == GL_LINEAR_MIPMAP_NEAREST, taps);
         }
         filter = filter == GL_NEAREST_MIPMAP_NEAREST ? GL_NEAREST : GL_LINEAR;
@@ -2701,9 +2722,10 @@ __device__ uint32_t sample_texture(const RasterConsts &K, const TexLevel &L0, co
         if (lod > 0.0f) {
             float cl = lod > 1.0f ? 1.0f : lod;
             bool lin = filter == GL_LINEAR_MIPMAP_LINEAR;
-            uint32_t c0 = sample_level(L0, rep_s, rep_t, u, v, lin, taps);
-            uint32_t c1 = L1.px ? sample_level(L1, rep_s, rep_t, u, v, lin, taps) : 0xFFFFFFFFu;
-            return col_pack(col_lerp(col_unpack(c0), col_unpack(c1), cl));
+            const Bytes4 c0 = sample_level(L0, rep_s, rep_t, u, v, lin, taps);
+            const Bytes4 c1 = L1.px ? sample_level(L1, rep_s, rep_t, u, v, lin, taps)
+                                    : Bytes4{255.0f, 255.0f, 255.0f, 255.0f};
+            return bytes_of(col_lerp(units_of(c0), units_of(c1), cl));
         }
         filter = filter == GL_NEAREST_MIPMAP_LINEAR ? GL_NEAREST : GL_LINEAR;
     }
@@ -2713,7 +2735,7 @@ __device__ uint32_t sample_texture(const RasterConsts &K, const TexLevel &L0, co
 
 // per-pixel state a lane carries through its tile
 struct PixelState {
-    uint32_t c;          // packed colour
+    Bytes4 c;            // colour
     float d;             // depth
     uint32_t s;          // stencil
     bool dirty_c, dirty_d, dirty_s;
@@ -2805,7 +2827,7 @@ __device__ float pixel_lod(const RasterConsts &K, const RTri *r, float b0, float
 
 // GL 1.5 level selection over the chain; each level sampled and packed to
 // RGBA8, two levels blended like the reference's level 0 / level 1 blend
-__device__ uint32_t sample_chain(const RasterConsts &K, float u, float v, float lod, int &taps)
+__device__ Bytes4 sample_chain(const RasterConsts &K, float u, float v, float lod, int &taps)
 {
     const bool rep_s = K.rep_s, rep_t = K.rep_t;
     wrap_uv(rep_s, rep_t, u, v);
@@ -2821,9 +2843,9 @@ __device__ uint32_t sample_chain(const RasterConsts &K, float u, float v, float 
     if (lod >= (float)top) return sample_level(chain_level(K, top), rep_s, rep_t, u, v, lin, taps);
     const float fl = floorf(lod);
     const int d = (int)fl;
-    const uint32_t c0 = sample_level(chain_level(K, d), rep_s, rep_t, u, v, lin, taps);
-    const uint32_t c1 = sample_level(chain_level(K, d + 1), rep_s, rep_t, u, v, lin, taps);
-    return col_pack(col_lerp(col_unpack(c0), col_unpack(c1), lod - fl));
+    const Bytes4 c0 = sample_level(chain_level(K, d), rep_s, rep_t, u, v, lin, taps);
+    const Bytes4 c1 = sample_level(chain_level(K, d + 1), rep_s, rep_t, u, v, lin, taps);
+    return bytes_of(col_lerp(units_of(c0), units_of(c1), lod - fl));
 }
 
 // The part of one fragment's pipeline (src/raster.c:546-721) that does not
@@ -2872,8 +2894,8 @@ __device__ void fragment_source(const RasterConsts &K, const RTri *r, const RCol
         float u, v;
         texcoord_at(r, K.persp, b0, b1, b2, u, v);
         int taps = 0;
-        Col tc = col_unpack(K.chain_on ? sample_chain(K, u, v, pixel_lod(K, r, b0, b1, b2), taps)
-                                       : sample_texture(K, K.L0, K.L1, u, v, r->lod, taps));
+        Col tc = units_of(K.chain_on ? sample_chain(K, u, v, pixel_lod(K, r, b0, b1, b2), taps)
+                                     : sample_texture(K, K.L0, K.L1, u, v, r->lod, taps));
         if (K.alpha_on && !cmp_f(K.alpha_cmp, tc.a, K.alpha_ref)) {
             c_out = c;
             meta_out = (uint32_t)taps << 1;
@@ -2966,26 +2988,31 @@ __device__ __forceinline__ bool depth_stencil_step(const RasterConsts &K, float 
     return true;
 }
 
-// Second half: blend with the pixel's colour, clamp, colour mask, pack.
+// Second half: blend with the pixel's colour, clamp, colour mask, pack.  The
+// pixel's colour stays as four byte values between its fragments, and the
+// clamps fold into byte_of; GL_SRC_ALPHA over GL_ONE_MINUS_SRC_ALPHA, by far
+// the commonest, needs no choice of factors.
 __device__ __forceinline__ void color_step(const RasterConsts &K, Col c, PixelState &px)
 {
     if (K.blend_on) {
-        Col dst = col_unpack(px.c);
-        Col sf = blend_factor(K.blend_src, c, dst);
-        Col df = blend_factor(K.blend_dst, c, dst);
-        c = col_clamp(col_add(col_mul(c, sf), col_mul(dst, df)));
+        const Col dst = units_of(px.c);
+        if (K.blend_src == GL_SRC_ALPHA && K.blend_dst == GL_ONE_MINUS_SRC_ALPHA) {
+            const float ia = 1 - c.a;
+            c = {c.r * c.a + dst.r * ia, c.g * c.a + dst.g * ia, c.b * c.a + dst.b * ia, c.a * c.a + dst.a * ia};
+        } else {
+            Col sf = blend_factor(K.blend_src, c, dst);
+            Col df = blend_factor(K.blend_dst, c, dst);
+            c = col_add(col_mul(c, sf), col_mul(dst, df));
+        }
     }
-    c = col_clamp(c);
     if (K.cmask == 0xFu) {
-        px.c = col_pack(c);
+        px.c = bytes_of(c);
         px.dirty_c = true;
     } else if (K.cmask != 0u) {
-        Col d = col_unpack(px.c);
-        if (K.cmask & 1u) d.r = c.r;
-        if (K.cmask & 2u) d.g = c.g;
-        if (K.cmask & 4u) d.b = c.b;
-        if (K.cmask & 8u) d.a = c.a;
-        px.c = col_pack(d);
+        // (the channels kept are packed again too, as the reference does)
+        const Col d = units_of(px.c);
+        px.c = bytes_of({K.cmask & 1u ? c.r : d.r, K.cmask & 2u ? c.g : d.g, K.cmask & 4u ? c.b : d.b,
+                         K.cmask & 8u ? c.a : d.a});
         px.dirty_c = true;
     }
 }
@@ -3003,7 +3030,6 @@ __device__ __forceinline__ void edge_values(const RTri *r, int32_t x, int32_t y,
 }
 
 constexpr int CHUNK = 64;          // bin entries per coverage pass: one bit each in a pixel's mask
-constexpr int FCAP = 128;          // fragment colours held in LDS per batch (general kernel)
 
 // what the in-order depth pass reads per bin entry: the edge-function terms
 // in the reference's operation order, 1/area and the three window z
@@ -3053,38 +3079,31 @@ __device__ __forceinline__ void wave_sync()
 
 // The mask of the chunk's entries covering pixel (R, I): the AND of three
 // ballots (each compare writes its lane mask straight to scalar registers).
-// VIA_LDS: lane 0 stores it to the pixel's LDS slot and the pixel's lane
-// reads it back once every pixel is done (one wave: LDS operations complete
-// in order), 4 vector instructions per pixel; else the pixel's lane selects
-// it from the scalar result (no LDS traffic, about twice the instructions:
-// the general kernel, whose LDS is busier, keeps this form).
-template <int R, int I, bool VIA_LDS>
+// Lane 0 stores it to the pixel's LDS slot and the pixel's lane reads it back
+// once every pixel is done (one wave: LDS operations complete in order): 4
+// vector instructions per pixel, where selecting the scalar result into the
+// pixel's lane took about twice as many.
+template <int R, int I>
 __device__ __forceinline__ void cover_pixel(const float *a0, const float *a1, const float *a2, float b0, float b1,
-                                            float b2, uint64_t *s_mask, int32_t &mlo, int32_t &mhi)
+                                            float b2, uint64_t *s_mask)
 {
     const uint64_t bal = __builtin_amdgcn_ballot_w64(a0[I] >= b0) & __builtin_amdgcn_ballot_w64(a1[I] >= b1) &
                          __builtin_amdgcn_ballot_w64(a2[I] >= b2);
-    if (VIA_LDS) {
-        if (threadIdx.x == 0) s_mask[R * TILE + I] = bal;
-    } else if ((int)threadIdx.x == R * TILE + I) {
-        mlo = (int32_t)(uint32_t)bal;
-        mhi = (int32_t)(uint32_t)(bal >> 32);
-    }
+    if (threadIdx.x == 0) s_mask[R * TILE + I] = bal;
 }
 
-template <int R, bool VIA_LDS>
+template <int R>
 __device__ __forceinline__ void cover_row(const float *a0, const float *a1, const float *a2, const float *b0,
-                                          const float *b1, const float *b2, uint64_t *s_mask, int32_t &mlo,
-                                          int32_t &mhi)
+                                          const float *b1, const float *b2, uint64_t *s_mask)
 {
-    cover_pixel<R, 0, VIA_LDS>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask, mlo, mhi);
-    cover_pixel<R, 1, VIA_LDS>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask, mlo, mhi);
-    cover_pixel<R, 2, VIA_LDS>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask, mlo, mhi);
-    cover_pixel<R, 3, VIA_LDS>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask, mlo, mhi);
-    cover_pixel<R, 4, VIA_LDS>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask, mlo, mhi);
-    cover_pixel<R, 5, VIA_LDS>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask, mlo, mhi);
-    cover_pixel<R, 6, VIA_LDS>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask, mlo, mhi);
-    cover_pixel<R, 7, VIA_LDS>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask, mlo, mhi);
+    cover_pixel<R, 0>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask);
+    cover_pixel<R, 1>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask);
+    cover_pixel<R, 2>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask);
+    cover_pixel<R, 3>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask);
+    cover_pixel<R, 4>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask);
+    cover_pixel<R, 5>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask);
+    cover_pixel<R, 6>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask);
+    cover_pixel<R, 7>(a0, a1, a2, b0[R], b1[R], b2[R], s_mask);
 }
 
 
@@ -3111,7 +3130,6 @@ __device__ __forceinline__ RCov make_cov(const float4 *q)
 // covering it, kept by that pixel's lane.  Negative-area triangles are
 // tested with A and B negated; the bounding box and the framebuffer edge
 // fold in as -inf / +inf.
-template <bool VIA_LDS>
 __device__ __forceinline__ uint64_t cover_chunk(const RCov &cv, int32_t minX, int32_t minY, int32_t maxX, int32_t maxY,
                                                 float area, bool valid, int32_t X0, int32_t Y0, int32_t fb_w,
                                                 int32_t fb_h, int32_t r0, int32_t r1, uint64_t *s_mask)
@@ -3138,16 +3156,14 @@ __device__ __forceinline__ uint64_t cover_chunk(const RCov &cv, int32_t minX, in
         if (!(yi >= minY && yi <= maxY && yi < fb_h)) b0[i] = __builtin_inff();
     }
     // only the rows [r0, r1) of the item (a part of a heavy tile, or all)
-    int32_t mlo = 0, mhi = 0;
-    if (r0 <= 0 && 0 < r1) cover_row<0, VIA_LDS>(a0, a1, a2, b0, b1, b2, s_mask, mlo, mhi);
-    if (r0 <= 1 && 1 < r1) cover_row<1, VIA_LDS>(a0, a1, a2, b0, b1, b2, s_mask, mlo, mhi);
-    if (r0 <= 2 && 2 < r1) cover_row<2, VIA_LDS>(a0, a1, a2, b0, b1, b2, s_mask, mlo, mhi);
-    if (r0 <= 3 && 3 < r1) cover_row<3, VIA_LDS>(a0, a1, a2, b0, b1, b2, s_mask, mlo, mhi);
-    if (r0 <= 4 && 4 < r1) cover_row<4, VIA_LDS>(a0, a1, a2, b0, b1, b2, s_mask, mlo, mhi);
-    if (r0 <= 5 && 5 < r1) cover_row<5, VIA_LDS>(a0, a1, a2, b0, b1, b2, s_mask, mlo, mhi);
-    if (r0 <= 6 && 6 < r1) cover_row<6, VIA_LDS>(a0, a1, a2, b0, b1, b2, s_mask, mlo, mhi);
-    if (r0 <= 7 && 7 < r1) cover_row<7, VIA_LDS>(a0, a1, a2, b0, b1, b2, s_mask, mlo, mhi);
-    if (!VIA_LDS) return ((uint64_t)(uint32_t)mhi << 32) | (uint32_t)mlo;
+    if (r0 <= 0 && 0 < r1) cover_row<0>(a0, a1, a2, b0, b1, b2, s_mask);
+    if (r0 <= 1 && 1 < r1) cover_row<1>(a0, a1, a2, b0, b1, b2, s_mask);
+    if (r0 <= 2 && 2 < r1) cover_row<2>(a0, a1, a2, b0, b1, b2, s_mask);
+    if (r0 <= 3 && 3 < r1) cover_row<3>(a0, a1, a2, b0, b1, b2, s_mask);
+    if (r0 <= 4 && 4 < r1) cover_row<4>(a0, a1, a2, b0, b1, b2, s_mask);
+    if (r0 <= 5 && 5 < r1) cover_row<5>(a0, a1, a2, b0, b1, b2, s_mask);
+    if (r0 <= 6 && 6 < r1) cover_row<6>(a0, a1, a2, b0, b1, b2, s_mask);
+    if (r0 <= 7 && 7 < r1) cover_row<7>(a0, a1, a2, b0, b1, b2, s_mask);
     wave_sync();
     const int32_t row = (int32_t)(threadIdx.x >> 3);
     const uint64_t m = row >= r0 && row < r1 ? s_mask[threadIdx.x] : 0ull;
@@ -3159,8 +3175,7 @@ __device__ __forceinline__ uint64_t cover_chunk(const RCov &cv, int32_t minX, in
 // submission order; returns the entries that passed (the ones whose colour
 // step runs).  Valid when no alpha test reads the texture.
 __device__ __forceinline__ uint64_t depth_pass(const RasterConsts &K, const RCov *s_cov, const uint32_t *s_tap,
-                                               uint64_t m, float xf, float yf, PixelState &px,
-                                               unsigned long long &bytes)
+                                               uint64_t m, float xf, float yf, PixelState &px, uint32_t &bytes)
 {
     uint64_t pass = 0;
     while (m) {
@@ -3437,7 +3452,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
     const int32_t fb_w = S.fb_w, fb_h = S.fb_h;
     const bool in_fb = (lane >> 3) >= r0 && (lane >> 3) < r1 && x < fb_w && y < fb_h;   // this item's pixel
     const size_t pix = in_fb ? (size_t)y * fb_w + x : 0;
-    PixelState px = {0u, 1.0f, 0u, false, false, false};
+    PixelState px = {{0.0f, 0.0f, 0.0f, 0.0f}, 1.0f, 0u, false, false, false};
     if (in_fb) {
         if (K.depth_on) px.d = S.depth[pix];
         if (K.stencil_on) px.s = S.stencil[pix];
@@ -3560,7 +3575,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
             s_rid[lane] = rid;
             s_tap[lane] = texel_taps(K, REC_F(q, lod));
         }
-        const uint64_t m = cover_chunk<true>(cv, REC_I(q, minX), REC_I(q, minY), REC_I(q, maxX), REC_I(q, maxY),
+        const uint64_t m = cover_chunk(cv, REC_I(q, minX), REC_I(q, minY), REC_I(q, maxX), REC_I(q, maxY),
                                        REC_F(q, area), valid, X0, Y0, fb_w, fb_h, r0, r1, s_mask);
         const uint32_t cnt = (uint32_t)__popcll(m);
         frag_count += cnt;
@@ -3671,7 +3686,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
             uint32_t meta;
             fragment_source(K, r, P.rcold ? P.rcold + (writer - 1u) : nullptr, w0e * inv, w1e * inv, w2e * inv, c, dep,
                             meta);
-            packed = col_pack(col_clamp(c));
+            packed = col_pack(c);
         }
         if (in_fb) {
             if (px.dirty_d) S.depth[pix] = px.d;
@@ -3684,6 +3699,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
     add_stats(P, frag_count, frag_bytes);
 }
 
+// What the scenes of a launch that the general kernel draws need of it:
+// everything; no per-fragment lighting and no full-chain sampling; no texture
+// either.
+enum : int { GEN_ALL = 0, GEN_SIMPLE = 1, GEN_PLAIN = 2 };
+
 // K4, general: blending, a partial colour mask, or an alpha test on a
 // texture.  One 8x8 tile per one-wave block.  Per chunk of 64 bin entries:
 // coverage (cover_chunk); unless the alpha test decides depth writes, the
@@ -3692,19 +3712,24 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
 // fragment per lane in batches of at most FCAP, applied per pixel in
 // submission order.  The colour step reads each fragment's record from
 // global memory (L1/L2: a chunk's fragments share few records) rather than
-// staging the chunk's 176-byte records in LDS: with 7.5 KB of LDS and at
-// most 168 VGPRs (a few spill) three waves share a SIMD instead of two (the
-// 4K overdraw stage took 1.41 ms so, 1.57 with the records in LDS).  PLAIN:
-// every scene of the launch that this kernel draws has no texture and no
-// per-fragment lighting (Phong or two-sided), so those paths compile away:
-// 124 VGPRs, no spills and four waves per SIMD (that stage: 0.94 ms).
-template <bool PLAIN>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PLAIN ? 4 : 3))) k_raster(RasterParams P)
+// staging the chunk's 176-byte records in LDS, which would leave fewer waves.
+// NEED (the GEN_* above) compiles away what no scene of the launch has: with
+// everything 168 VGPRs and a few spills at three waves per SIMD; without
+// per-fragment lighting and the full chain four waves (128 VGPRs, a few
+// spills): 6,000 textured quads blended over 720p, 24 million fragments,
+// take 473 us, 582 with everything compiled in; without textures 124 VGPRs
+// and no spills: 4K overdraw, 109 million fragments, 822 us.  It is bound by
+// the vector ALU, so the pixel's colour stays unpacked between its fragments
+// (color_step): that took the two from 528 and 919 us.  Batches of 256
+// colours: 822 against 840 us untextured, 534 against 473 textured.
+template <int NEED>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NEED == GEN_ALL ? 3 : 4))) k_raster(RasterParams P)
 {
     __shared__ RCov s_cov[CHUNK];
     __shared__ uint64_t s_mask[TILE * TILE];   // coverage masks of a chunk, per pixel
     __shared__ uint32_t s_rid[CHUNK];
     __shared__ uint32_t s_tap[CHUNK];
+    constexpr int FCAP = NEED == GEN_PLAIN ? 256 : 128;   // fragment colours held in LDS per batch
     __shared__ float4 s_col[FCAP];
     __shared__ float s_dep[FCAP];
     __shared__ uint16_t s_slot[FCAP];
@@ -3731,10 +3756,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PLAIN ?
     // items they spill scalar registers on every pass
     RasterConsts K;
     raster_consts(S, K);
-    if (PLAIN) {
-        // what these scenes hold already (the launch checked them), as
-        // constants; phong and two_side only matter with lighting on
-        K.textured = false;
+    // what these scenes hold already (the launch checked them), as constants;
+    // phong and two_side only matter with lighting on
+    if (NEED == GEN_PLAIN) K.textured = false;
+    if (NEED != GEN_ALL) {
         K.chain_on = false;
         K.phong = false;
         K.two_side = false;
@@ -3748,9 +3773,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PLAIN ?
     const int32_t fb_w = S.fb_w, fb_h = S.fb_h;
     const bool in_fb = (lane >> 3) >= r0 && (lane >> 3) < r1 && x < fb_w && y < fb_h;   // this item's pixel
     const size_t pix = in_fb ? (size_t)y * fb_w + x : 0;
-    PixelState px = {0u, 1.0f, 0u, false, false, false};
+    PixelState px = {{0.0f, 0.0f, 0.0f, 0.0f}, 1.0f, 0u, false, false, false};
     if (in_fb) {
-        if (need_color) px.c = S.color[pix];
+        if (need_color) px.c = bytes_load(S.color[pix]);
         if (K.depth_on) px.d = S.depth[pix];
         if (K.stencil_on) px.s = S.stencil[pix];
     }
@@ -3781,12 +3806,13 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PLAIN ?
             s_rid[lane] = rid;
             s_tap[lane] = texel_taps(K, REC_F(q, lod));
         }
-        const uint64_t m = cover_chunk<false>(cv, REC_I(q, minX), REC_I(q, minY), REC_I(q, maxX), REC_I(q, maxY),
+        const uint64_t m = cover_chunk(cv, REC_I(q, minX), REC_I(q, minY), REC_I(q, maxX), REC_I(q, maxY),
                                        REC_F(q, area), valid, X0, Y0, fb_w, fb_h, r0, r1, s_mask);
         frag_count += (unsigned long long)__popcll(m);
         wave_sync();   // staged entries visible to every lane
 
-        const uint64_t todo = alpha_dep ? m : depth_pass(K, s_cov, s_tap, m, xf, yf, px, frag_bytes);
+        uint32_t bytes32 = 0;   // (a chunk gives a pixel at most 64 fragments of at most 50 bytes)
+        const uint64_t todo = alpha_dep ? m : depth_pass(K, s_cov, s_tap, m, xf, yf, px, bytes32);
         // batches: each pixel takes its next L fragments, L the largest quota
         // that keeps the batch within FCAP (L >= 1 fits since 64 <= FCAP)
         uint64_t rem = todo;
@@ -3834,14 +3860,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PLAIN ?
                 const uint32_t f = off + qn;
                 const float4 cc = s_col[f];
                 const uint32_t meta = s_meta[f];
-                if (!alpha_dep || depth_stencil_step(K, s_dep[f], meta >> 1, (meta & 1u) != 0u, px, frag_bytes))
+                if (!alpha_dep || depth_stencil_step(K, s_dep[f], meta >> 1, (meta & 1u) != 0u, px, bytes32))
                     color_step(K, Col{cc.x, cc.y, cc.z, cc.w}, px);
             }
             wave_sync();   // slots and colours are reused by the next batch
         }
+        frag_bytes += bytes32;
     }
     if (in_fb) {
-        if (px.dirty_c) S.color[pix] = px.c;
+        if (px.dirty_c) S.color[pix] = bytes_pack(px.c);
         if (px.dirty_d) S.depth[pix] = px.d;
         if (px.dirty_s) S.stencil[pix] = (uint8_t)px.s;
     }
@@ -3869,13 +3896,15 @@ constexpr uint64_t PRIM_MAX_FRAGS = 1ull << 30;   // fragments one primitive may
 struct PrimParams {
     SceneRaster S;                     // state, texture, framebuffer size
     uint32_t mode, count, units;
-    uint32_t tri;                      // 1: units are assembled triangles (glPolygonMode LINE / POINT)
     const VHot *vhot;
     const VCold *vcold;                // null when no per-vertex lighting reads it
     unsigned long long *counts;        // count pass: fragments per unit
     const unsigned long long *base;    // emit pass: first fragment of each unit
-    uint32_t *keys, *vals;
-    float *dep;
+    // per fragment: pixel and depth, colour (one line of memory each: the
+    // stores of neighbouring threads lie apart); vals: null, or the values of
+    // a draw with filled faces
+    uint2 *kd;
+    uint32_t *vals;
     float4 *col;
     Counters *ctr;
 };
@@ -3932,9 +3961,8 @@ __device__ __forceinline__ uint32_t prim_key(const PrimParams &P, const RasterCo
 
 __device__ __forceinline__ void prim_put(const PrimParams &P, uint64_t j, uint32_t key, float depth, Col c)
 {
-    P.keys[j] = key;
-    P.vals[j] = (uint32_t)j;
-    P.dep[j] = depth;
+    P.kd[j] = make_uint2(key, __float_as_uint(depth));
+    if (P.vals) P.vals[j] = (uint32_t)j;
     P.col[j] = make_float4(c.r, c.g, c.b, c.a);
 }
 
@@ -3977,7 +4005,7 @@ __device__ uint64_t prim_line(const PrimParams &P, const RasterConsts &K, int32_
         if (K.textured) {
             const float u = u0 + t * (u1 - u0), v = v0 + t * (v1 - v0);
             int taps = 0;
-            const Col tc = col_unpack(sample_texture(K, K.L0, K.L1, u, v, 0.0f, taps));
+            const Col tc = units_of(sample_texture(K, K.L0, K.L1, u, v, 0.0f, taps));
             if (K.alpha_on && !cmp_f(K.alpha_cmp, tc.a, K.alpha_ref)) keep = false;
             else c = col_mul(c, tc);
         } else if (K.alpha_on && !cmp_f(K.alpha_cmp, c.a, K.alpha_ref)) {
@@ -4073,7 +4101,7 @@ __device__ uint64_t prim_point(const PrimParams &P, const RasterConsts &K, uint3
     bool keep = true;
     if (K.textured) {
         int taps = 0;
-        const Col tc = col_unpack(sample_texture(K, K.L0, K.L1, q.s, q.t, 0.0f, taps));
+        const Col tc = units_of(sample_texture(K, K.L0, K.L1, q.s, q.t, 0.0f, taps));
         if (K.alpha_on && !cmp_f(K.alpha_cmp, tc.a, K.alpha_ref)) keep = false;
         else c = col_mul(c, tc);
     } else if (K.alpha_on && !cmp_f(K.alpha_cmp, c.a, K.alpha_ref)) {
@@ -4127,9 +4155,8 @@ __device__ uint64_t prim_fill(const PrimParams &P, const RasterConsts &K, const 
                 fragment_source(K, &r, cold ? &q : nullptr, e0 * r.inv_area, e1 * r.inv_area, e2 * r.inv_area, c,
                                 dep, meta);
                 const uint64_t j = base + n;
-                P.keys[j] = (uint32_t)y * (uint32_t)P.S.fb_w + (uint32_t)x;
+                P.kd[j] = make_uint2((uint32_t)y * (uint32_t)P.S.fb_w + (uint32_t)x, __float_as_uint(dep));
                 P.vals[j] = (uint32_t)j | PRIM_TRI_BIT | ((meta & 1u) ? 0u : PRIM_KILL_BIT);
-                P.dep[j] = dep;
                 P.col[j] = make_float4(c.r, c.g, c.b, c.a);
             }
             n++;
@@ -4213,7 +4240,11 @@ __device__ uint64_t prim_triangle(const PrimParams &P, const RasterConsts &K, ui
     return total;
 }
 
-template <bool EMIT>
+// KIND: what the draw's units are.  A kernel for each, since the triangles'
+// clipping and filling would leave the others two waves per SIMD: points and
+// lines wait for their scattered fragment stores, which more waves overlap.
+enum : int { PRIM_POINTS = 0, PRIM_LINES = 1, PRIM_TRIS = 2 };
+template <bool EMIT, int KIND>
 __global__ void __launch_bounds__(64) k_prim(PrimParams P)
 {
     const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
@@ -4222,9 +4253,9 @@ __global__ void __launch_bounds__(64) k_prim(PrimParams P)
     raster_consts(P.S, K);
     const uint64_t base = EMIT ? P.base[u] : 0;
     uint64_t n;
-    if (P.tri) {
+    if (KIND == PRIM_TRIS) {
         n = prim_triangle<EMIT>(P, K, u, base);
-    } else if (P.mode == GL_POINTS) {
+    } else if (KIND == PRIM_POINTS) {
         n = prim_point<EMIT>(P, K, u, base);
     } else {
         uint32_t ia, ib;
@@ -4237,19 +4268,21 @@ __global__ void __launch_bounds__(64) k_prim(PrimParams P)
 
 // One thread per pixel of the sorted fragments (the first of its run): the
 // reference's per-pixel steps over the pixel's fragments in order.
-__global__ void __launch_bounds__(256) k_prim_resolve(SceneRaster S, const uint32_t *keys, const uint32_t *vals,
-                                                      uint32_t n, const float *dep, const float4 *col, uint32_t npix)
+__global__ void __launch_bounds__(256) k_prim_resolve(SceneRaster S, const uint2 *sorted, uint32_t n,
+                                                      const uint2 *kd, const float4 *col, uint32_t npix)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const uint32_t k = keys[i];
-    if (k >= npix || (i > 0 && keys[i - 1] == k)) return;
+    const uint32_t k = sorted[i].x;
+    if (k >= npix || (i > 0 && sorted[i - 1].x == k)) return;
     RasterConsts K;
     raster_consts(S, K);
-    PixelState px = {S.color[k], S.depth[k], K.stencil_on ? (uint32_t)S.stencil[k] : 0u, false, false, false};
-    for (uint32_t j = i; j < n && keys[j] == k; j++) {
-        const uint32_t v = vals[j], f = v & PRIM_INDEX_MASK;
-        const float d = dep[f];
+    PixelState px = {bytes_load(S.color[k]), S.depth[k], K.stencil_on ? (uint32_t)S.stencil[k] : 0u, false, false, false};
+    for (uint32_t j = i; j < n; j++) {
+        const uint2 q = sorted[j];
+        if (q.x != k) break;
+        const uint32_t v = q.y, f = v & PRIM_INDEX_MASK;
+        const float d = __uint_as_float(kd[f].y);
         if (v & PRIM_TRI_BIT) {
             // a filled face's fragment: stencil and depth tests, stencil
             // update, alpha-test discard, depth write, colour
@@ -4268,7 +4301,7 @@ __global__ void __launch_bounds__(256) k_prim_resolve(SceneRaster S, const uint3
         color_step(K, Col{c.x, c.y, c.z, c.w}, px);
     }
     if (px.dirty_d) S.depth[k] = px.d;
-    if (px.dirty_c) S.color[k] = px.c;
+    if (px.dirty_c) S.color[k] = bytes_pack(px.c);
     if (px.dirty_s) S.stencil[k] = (uint8_t)px.s;
 }
 
@@ -4994,7 +5027,7 @@ struct Exec {
     int cu_count = 256;
     // blocks at once: depth<stencil>, depth<no stencil>, general, then the
     // depth kernels at four waves per SIMD (launches of several scenes)
-    uint32_t resident[8] = {256, 256, 256, 256, 256, 256, 256, 256};
+    uint32_t resident[9] = {256, 256, 256, 256, 256, 256, 256, 256, 256};
     Counters *ctr = nullptr;                       // device
     Counters *ctr_host = nullptr;                  // pinned mirror for readback
     uint32_t *report = nullptr;                    // pinned: the poison the latest read reported
@@ -5052,7 +5085,7 @@ struct Launch {
     bool multi_vs = false;         // some scene switches vertex states per vertex
     bool unsupported = false;
     uint32_t kinds = 0;            // bit (1 << kind) for each raster kind present
-    bool plain = true;             // no scene for the general kernel has a texture or per-fragment lighting
+    int gen_need = GEN_PLAIN;      // what the general kernel's scenes need of it (the least GEN_* that serves all)
     bool simple = true;            // no scene for the depth kernel lights per fragment or samples the full chain
     uint64_t pairs_cap = 0;        // pairs of the sizing run (frozen replays use it)
     const VertexParams *vp = nullptr;
@@ -5118,7 +5151,7 @@ struct mtgl_dev {
     Arena pixels;                  // glDrawPixels source bytes
     Arena readback;                // glReadPixels: packed rows of one band
     Arena prim_params;             // states, staged bytes and vertex parameters of a point / line draw
-    Arena prim_dep, prim_col;      // fragments of a point / line draw: depth, colour
+    Arena prim_col;                // fragments of a point / line draw: colour
     std::unordered_map<uint32_t, DevBuf> segs;   // display-list segments by id
     DevTex tex[MTGL_MAX_OBJECTS + 1];
     DevBuf buf[MTGL_MAX_OBJECTS + 1];
@@ -5340,11 +5373,12 @@ int exec_init(Exec &x, int device)
         x.cu_count <= 0)
         x.cu_count = 256;
     // resident one-wave blocks of each raster kernel (registers and LDS bound)
-    const void *kern[8] = {(const void *)k_raster_depth<true, 3, false>, (const void *)k_raster_depth<false, 3, false>,
-                           (const void *)k_raster<false>, (const void *)k_raster_depth<true, 4, false>,
-                           (const void *)k_raster_depth<false, 4, false>, (const void *)k_raster<true>,
-                           (const void *)k_raster_depth<true, 3, true>, (const void *)k_raster_depth<false, 3, true>};
-    for (int k = 0; k < 8; k++) {
+    const void *kern[9] = {(const void *)k_raster_depth<true, 3, false>, (const void *)k_raster_depth<false, 3, false>,
+                           (const void *)k_raster<GEN_ALL>, (const void *)k_raster_depth<true, 4, false>,
+                           (const void *)k_raster_depth<false, 4, false>, (const void *)k_raster<GEN_PLAIN>,
+                           (const void *)k_raster_depth<true, 3, true>, (const void *)k_raster_depth<false, 3, true>,
+                           (const void *)k_raster<GEN_SIMPLE>};
+    for (int k = 0; k < 9; k++) {
         int nb = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern[k], 64, 0) != hipSuccess || nb <= 0) nb = 2;
         x.resident[k] = std::min<uint32_t>((uint32_t)nb * (uint32_t)x.cu_count, STAT_SLOTS);
@@ -5693,7 +5727,7 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
     L.region_items = L.bins ? (uint32_t)z.items : 0u;
     L.work = z.work_sum;
     L.any_cold = z.cold;
-    L.plain = true;
+    L.gen_need = GEN_PLAIN;
     L.simple = true;
 
     int rc;
@@ -5820,7 +5854,12 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
         r.tile_off = tileoff;
         sr[s] = r;
         L.kinds |= 1u << r.kind;
-        if (!(r.kind & KIND_LAST_WRITER) && (r.tex != nullptr || needs_cold(dr->raster))) L.plain = false;
+        if (!(r.kind & KIND_LAST_WRITER)) {
+            const bool chain = r.tex != nullptr && r.lod_mode == MTGL_LOD_FULL_CHAIN;
+            L.gen_need = std::min<int>(L.gen_need, needs_cold(dr->raster) || chain ? GEN_ALL
+                                                   : r.tex != nullptr             ? GEN_SIMPLE
+                                                                                  : GEN_PLAIN);
+        }
         if ((r.kind & KIND_LAST_WRITER) && (needs_cold(dr->raster) || r.lod_mode == MTGL_LOD_FULL_CHAIN)) L.simple = false;
 
         bnp[s] = bno;
@@ -5921,10 +5960,10 @@ int tile_sort(Exec &x, Launch &L, bool frozen, uint32_t seq, uint32_t cap, uint3
                            (const uint32_t *)counts, (const uint32_t *)loc, ntiles, vals, as<uint32_t>(x.tile_gen),
                            x.gen, x.heavy_bin, L.tmap, L.tile_pre, L.ns, as<uint4>(x.tile_list), list_cap, x.ctr, x.regions);
     } else if (ntiles > 0u && shift <= BINS_MAX_SHIFT) {
-        hipLaunchKernelGGL(k_sort_hist, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys, cap, np,
+        hipLaunchKernelGGL(k_sort_hist, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys, 1u, cap, np,
                            shift, nblocks, counts);
         if ((rc = device_scan<uint32_t>(x, counts, counts, (uint64_t)RADIX * nblocks, frozen))) return rc;
-        hipLaunchKernelGGL(k_sort_scatter, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys,
+        hipLaunchKernelGGL(k_sort_scatter<SORT_ARRAYS>, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys,
                            (const uint32_t *)vals, cap, np, shift, nblocks, (const uint32_t *)counts, keys2, vals2);
         hipLaunchKernelGGL(k_tile_bins, dim3(((ntiles - 1u) >> shift) + 1u), dim3(BINS_THREADS), 0, x.stream,
                            (const uint32_t *)keys2, (const uint32_t *)vals2, cap, np, shift, nblocks,
@@ -5935,11 +5974,11 @@ int tile_sort(Exec &x, Launch &L, bool frozen, uint32_t seq, uint32_t cap, uint3
         int key_bits = 1;
         while ((1u << key_bits) <= ntiles) key_bits++;
         for (int sh = 0; sh < key_bits; sh += RADIX_BITS) {
-            hipLaunchKernelGGL(k_sort_hist, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys, cap,
+            hipLaunchKernelGGL(k_sort_hist, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys, 1u, cap,
                                np, sh, nblocks, counts);
             if ((rc = device_scan<uint32_t>(x, counts, counts, (uint64_t)RADIX * nblocks, frozen))) return rc;
-            hipLaunchKernelGGL(k_sort_scatter, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys,
-                               (const uint32_t *)vals, cap, np, sh, nblocks, (const uint32_t *)counts, keys2, vals2);
+            hipLaunchKernelGGL(k_sort_scatter<SORT_ARRAYS>, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream,
+                               (const uint32_t *)keys, (const uint32_t *)vals, cap, np, sh, nblocks, (const uint32_t *)counts, keys2, vals2);
             std::swap(keys, keys2);
             std::swap(vals, vals2);
         }
@@ -6100,7 +6139,7 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
         // twice is 20% slower on the 1080p depth stage, four and six times
         // equal to three there; on the 4K overdraw stage six times is 1.5%
         // faster than three)
-        const uint32_t over = k == 2 || k == 5 ? 6u : 3u;
+        const uint32_t over = k == 2 || k == 5 || k == 8 ? 6u : 3u;
         const uint32_t g = std::min<uint32_t>(over * x.resident[k] / x.grid_div, STAT_SLOTS);
         uint32_t n = std::max<uint32_t>(1u, std::min<uint32_t>(nlist, g));
         if (n >= 64u) n &= ~63u;
@@ -6126,8 +6165,10 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
         grids[nl++] = grid(many ? 4 : L.simple ? 7 : 1);
     }
     if (L.kinds & general) {
-        fns[nl] = L.plain ? (const void *)k_raster<true> : (const void *)k_raster<false>;
-        grids[nl++] = grid(L.plain ? 5 : 2);
+        fns[nl] = L.gen_need == GEN_PLAIN    ? (const void *)k_raster<GEN_PLAIN>
+                  : L.gen_need == GEN_SIMPLE ? (const void *)k_raster<GEN_SIMPLE>
+                                             : (const void *)k_raster<GEN_ALL>;
+        grids[nl++] = grid(L.gen_need == GEN_PLAIN ? 5 : L.gen_need == GEN_SIMPLE ? 8 : 2);
     }
     // (the first of several kernels ends the binning's use of the counters)
     RasterParams rp2 = rp;
@@ -6264,13 +6305,21 @@ int run_prims(mtgl_dev *d, const mtgl_draw *dr, int cls)
     P.mode = dr->mode;
     P.count = dr->count;
     P.units = units;
-    P.tri = cls >= 2 ? 1u : 0u;
     P.vhot = as<VHot>(x.vhot);
     P.vcold = cold ? as<VCold>(x.vcold) : nullptr;
     P.counts = counts;
     P.base = base;
     P.ctr = x.ctr;
-    hipLaunchKernelGGL(k_prim<false>, dim3(blocks_for(units, 64)), dim3(64), 0, x.stream, P);
+    const bool pts = dr->mode == GL_POINTS;
+    auto count = k_prim<false, PRIM_LINES>, emit = k_prim<true, PRIM_LINES>;
+    if (pts) {
+        count = k_prim<false, PRIM_POINTS>;
+        emit = k_prim<true, PRIM_POINTS>;
+    } else if (cls >= 2) {
+        count = k_prim<false, PRIM_TRIS>;
+        emit = k_prim<true, PRIM_TRIS>;
+    }
+    hipLaunchKernelGGL(count, dim3(blocks_for(units, 64)), dim3(64), 0, x.stream, P);
     HIPC(hipGetLastError());
     if ((rc = device_scan<unsigned long long>(x, counts, base, (uint64_t)units, false, &x.ctr->npairs))) return rc;
     HIPC(hipMemcpyAsync(x.ctr_host, x.ctr, sizeof(Counters), hipMemcpyDeviceToHost, x.stream));
@@ -6282,19 +6331,16 @@ int run_prims(mtgl_dev *d, const mtgl_draw *dr, int cls)
     // fragment indices travel through the sort in the value's low bits
     if (total > (cls == 3 ? (uint64_t)PRIM_INDEX_MASK + 1u : 0x7FFFFFFFull)) return MTGL_ERR_OUT_OF_MEMORY;
     const uint32_t n = (uint32_t)total;
-    for (int k = 0; k < 2; k++) {
-        if ((rc = arena_reserve(x, x.keys[k], (size_t)n * 4))) return rc;
-        if ((rc = arena_reserve(x, x.vals[k], (size_t)n * 4))) return rc;
-    }
-    if ((rc = arena_reserve(x, d->prim_dep, (size_t)n * 4))) return rc;
+    // fragments' (pixel, depth), two buffers of (pixel, value) pairs for the
+    // sort, and the values of a draw with filled faces
+    for (Arena *a : {&x.keys[0], &x.keys[1], &x.vals[1]})
+        if ((rc = arena_reserve(x, *a, (size_t)n * 8))) return rc;
+    if (cls == 3 && (rc = arena_reserve(x, x.vals[0], (size_t)n * 4))) return rc;
     if ((rc = arena_reserve(x, d->prim_col, (size_t)n * 16))) return rc;
-    uint32_t *keys = as<uint32_t>(x.keys[0]), *vals = as<uint32_t>(x.vals[0]);
-    uint32_t *keys2 = as<uint32_t>(x.keys[1]), *vals2 = as<uint32_t>(x.vals[1]);
-    P.keys = keys;
-    P.vals = vals;
-    P.dep = as<float>(d->prim_dep);
+    P.kd = as<uint2>(x.keys[0]);
+    P.vals = cls == 3 ? as<uint32_t>(x.vals[0]) : nullptr;
     P.col = as<float4>(d->prim_col);
-    hipLaunchKernelGGL(k_prim<true>, dim3(blocks_for(units, 64)), dim3(64), 0, x.stream, P);
+    hipLaunchKernelGGL(emit, dim3(blocks_for(units, 64)), dim3(64), 0, x.stream, P);
     // stable LSD radix sort by pixel; the all-ones key of discarded fragments stays last
     const uint32_t npix = (uint32_t)d->w * (uint32_t)d->h;
     int key_bits = 1;
@@ -6302,19 +6348,21 @@ int run_prims(mtgl_dev *d, const mtgl_draw *dr, int cls)
     const uint32_t nblocks = (n + SORT_TILE - 1) / SORT_TILE;
     if ((rc = arena_reserve(x, x.sort_tmp, (size_t)RADIX * nblocks * 4))) return rc;
     uint32_t *sc = as<uint32_t>(x.sort_tmp);
+    const uint32_t *from = as<uint32_t>(x.keys[0]);
+    uint32_t *to = as<uint32_t>(x.keys[1]), *other = as<uint32_t>(x.vals[1]);
     for (int shift = 0; shift < key_bits; shift += RADIX_BITS) {
-        hipLaunchKernelGGL(k_sort_hist, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys, n,
+        hipLaunchKernelGGL(k_sort_hist, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, from, 2u, n,
                            (const unsigned long long *)nullptr, shift, nblocks, sc);
         if ((rc = device_scan<uint32_t>(x, sc, sc, (uint64_t)RADIX * nblocks, false))) return rc;
-        hipLaunchKernelGGL(k_sort_scatter, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, (const uint32_t *)keys,
-                           (const uint32_t *)vals, n, (const unsigned long long *)nullptr, shift, nblocks,
-                           (const uint32_t *)sc, keys2, vals2);
-        std::swap(keys, keys2);
-        std::swap(vals, vals2);
+        auto scatter = shift == 0 ? k_sort_scatter<SORT_FIRST> : k_sort_scatter<SORT_PAIRS>;
+        hipLaunchKernelGGL(scatter, dim3(nblocks), dim3(SORT_THREADS), 0, x.stream, from, (const uint32_t *)P.vals, n,
+                           (const unsigned long long *)nullptr, shift, nblocks, (const uint32_t *)sc, to,
+                           (uint32_t *)nullptr);
+        from = to;
+        std::swap(to, other);
     }
-    hipLaunchKernelGGL(k_prim_resolve, dim3(blocks_for(n, 256)), dim3(256), 0, x.stream, S, (const uint32_t *)keys,
-                       (const uint32_t *)vals, n, (const float *)as<float>(d->prim_dep),
-                       (const float4 *)as<float4>(d->prim_col), npix);
+    hipLaunchKernelGGL(k_prim_resolve, dim3(blocks_for(n, 256)), dim3(256), 0, x.stream, S, (const uint2 *)from, n,
+                       (const uint2 *)P.kd, (const float4 *)as<float4>(d->prim_col), npix);
     HIPC(hipGetLastError());
     return MTGL_OK;
 }
@@ -6802,7 +6850,6 @@ MTGL_API void mtgl_dev_destroy(mtgl_dev *d)
     arena_free(d->pixels);
     arena_free(d->readback);
     arena_free(d->prim_params);
-    arena_free(d->prim_dep);
     arena_free(d->prim_col);
     for (auto &kv : d->segs)
         if (kv.second.data) (void)hipFree(kv.second.data);
