@@ -4857,19 +4857,43 @@ __global__ void __launch_bounds__(256) k_diff_shade(const DiffView *views, const
 
 __device__ __forceinline__ float clamp_grad(float v, float g) { return (v >= 0.0f && v <= 1.0f) ? g : 0.0f; }
 
+// x0 to component t & 3 of element i0 of p and x1 to that of i1 (0xFFFFFFFF:
+// none), for the pixel of lanes t & ~3: lanes t and t ^ 4 swap one of theirs,
+// so that an instruction adds both elements of the pair's first pixel, the
+// next one both of the second's.
+__device__ __forceinline__ void add_pair(float *p, uint32_t t, uint32_t i0, uint32_t i1, float x0, float x1)
+{
+    const uint32_t h = (t >> 2) & 1u;
+    const uint32_t mi = h ? i1 : i0, oi = (uint32_t)__shfl_xor((int)(h ? i0 : i1), 4, 64);
+    const float mx = h ? x1 : x0, ox = __shfl_xor(h ? x0 : x1, 4, 64);
+    for (uint32_t s = 0; s < 2u; s++) {
+        const uint32_t i = h == s ? mi : oi;
+        if (i != 0xFFFFFFFFu) unsafeAtomicAdd(p + 4u * (size_t)i + (t & 3u), h == s ? mx : ox);
+    }
+}
+
 // adjoint of k_diff_shade: dL/dlit per listed vertex into dlit, dL/dtex.
 // Channels are independent through the shading, so a thread takes one
 // (covered pixel, channel): the four lanes of a pixel add to the four
-// consecutive floats of each target together, one L2 request per target and
-// instruction.  Grid (4 x covered pixels, views).
+// consecutive floats of a target together.  Bound by the requests of these
+// atomics, so two neighbouring pixels' lanes work on one pixel's targets at a
+// time where these are neighbours in memory: the two taps of a texture row,
+// and the two corners that follow each other in the view's vertex list (in a
+// mesh most triangles have such a pair), 32 bytes in one request.  64 views
+// of 256x256 took 159 us with a request per target, 122 with the taps in
+// pairs, 114 with corners 1 and 2 in pairs too, and take 110.  Gathering over
+// lists of each texel's and vertex's uses instead took about the same for 64
+// views, but a long run of uses is a serial chain: 16 small views 197 us a
+// step, against 125.  Grid (4 x covered pixels, views).
 __global__ void __launch_bounds__(256) k_diff_shade_bwd(const DiffView *views, const float *lit, const float *tex,
                                                         const float *grad, float *dlit, float *g_tex)
 {
     const DiffView &D = views[blockIdx.y];
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t ch = t & 3u;
-    if ((t >> 2) >= D.ncov) return;
-    const DiffPx g = D.cov[t >> 2];
+    if (((t >> 2) & ~1u) >= D.ncov) return;
+    const bool on = (t >> 2) < D.ncov;   // (an odd last pixel's neighbour only adds for it)
+    const DiffPx g = D.cov[on ? t >> 2 : D.ncov - 1u];
     const size_t npx = (size_t)D.w * (size_t)D.h;
     const float gr = grad[4u * ((size_t)blockIdx.y * npx + g.pixel) + ch];
     // the operations of diff_pixel, one channel
@@ -4883,10 +4907,17 @@ __global__ void __launch_bounds__(256) k_diff_shade_bwd(const DiffView *views, c
     const float tc = top * (1.0f - fy) + bot * fy;
     const float gm = clamp_grad(c * tc, gr);
     const float dc = gm * tc, dt = gm * c;
-    for (int k = 0; k < 3; k++)
-        if (g.v[k] != 0xFFFFFFFFu) unsafeAtomicAdd(dlit + 4u * ((size_t)D.off + g.v[k]) + ch, dc * g.b[k]);
+    // r: the corner left over; p and q: the two that are neighbours in the list, if two are
+    const bool n12 = g.v[1] - g.v[2] + 1u <= 2u, n02 = g.v[0] - g.v[2] + 1u <= 2u;
+    const uint32_t vp = n12 ? g.v[1] : g.v[0], vq = n12 || n02 ? g.v[2] : g.v[1];
+    const uint32_t vr = n12 ? g.v[0] : n02 ? g.v[1] : g.v[2];
+    const float bp = n12 ? g.b[1] : g.b[0], bq = n12 || n02 ? g.b[2] : g.b[1];
+    const float br = n12 ? g.b[0] : n02 ? g.b[1] : g.b[2];
+    add_pair(dlit + 4u * (size_t)D.off, t, on ? vp : 0xFFFFFFFFu, on ? vq : 0xFFFFFFFFu, dc * bp, dc * bq);
+    if (on && vr != 0xFFFFFFFFu) unsafeAtomicAdd(dlit + 4u * ((size_t)D.off + vr) + ch, dc * br);
     const float wt[4] = {(1.0f - fx) * (1.0f - fy), fx * (1.0f - fy), (1.0f - fx) * fy, fx * fy};
-    for (int k = 0; k < 4; k++) unsafeAtomicAdd(g_tex + 4u * (size_t)g.texel[k] + ch, dt * wt[k]);
+    for (int k = 0; k < 4; k += 2)
+        add_pair(g_tex, t, on ? g.texel[k] : 0xFFFFFFFFu, on ? g.texel[k + 1] : 0xFFFFFFFFu, dt * wt[k], dt * wt[k + 1]);
 }
 
 // sum over the 64 lanes, in lane 63 (the DPP pattern of dpp_incl_scan; lanes
