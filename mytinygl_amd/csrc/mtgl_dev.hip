@@ -2169,9 +2169,9 @@ __global__ void __launch_bounds__(BINS_THREADS) k_tile_bins(const uint32_t *keys
 // ---------------------------------------------------------------------------
 
 // One workgroup per square of a scene, BIN_T tiles a side (32 pixels) or, in
-// scenes with many triangles per tile, fewer (bin_side).  It walks the scene's set-up blocks in order, then
-// the triangles of those whose tile bounds meet the square, and lists the
-// records that do (s_list, in submission order).  Per 64 listed records a
+// scenes with many triangles per tile, fewer (bin_side).  It walks the scene's
+// set-up blocks in order, then the triangles of those whose tile bounds meet
+// the square, and lists the records that do (s_list, in submission order).  Per 64 listed records a
 // wave, one record per lane, tests the 64 tiles exactly (box_tile_mask's
 // argument: a tile whose best corner fails an edge holds no covered pixel)
 // and leaves, per tile, the mask of the records it can hold; the masks'
@@ -4445,8 +4445,9 @@ __global__ void __launch_bounds__(256) k_clear_span(uint32_t *color, float *dept
 // cache lines (out is 16-byte aligned for BPP 4, 4-byte for BPP 3): out is
 // device memory, or the caller's own pinned memory over PCIe, which bounds
 // the kernel then.  poison (null: not wanted) receives the Exec's poison, and
-// the latest launch's count of met squares after it, in pinned host memory, so that the wait for the pixels also tells the host
-// whether the queued work took effect; no pixel is stored when it did not.
+// the latest launch's count of met squares after it, in pinned host memory, so
+// that the wait for the pixels also tells the host whether the queued work
+// took effect; no pixel is stored when it did not.
 template <int BPP>
 __global__ void __launch_bounds__(256) k_read_pixels(const uint32_t *color, int32_t fb_w, int32_t fb_h, int32_t x,
                                                      int32_t y, int32_t flip, uint32_t w, int32_t r0, uint64_t n,
