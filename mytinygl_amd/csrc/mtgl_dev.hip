@@ -4946,7 +4946,8 @@ __device__ __forceinline__ float dpp_wave_sum_f(float v)
 // chain of loads per view (map, gradient, stored terms, the view's lights);
 // the view's number is made a scalar, so that its lights come by scalar loads
 // once per wave: 64 views of 50,625 vertices took 104 us with vector loads of
-// them and take 71.  16 groups a block took 92, 4 took 99.
+// them and 71 so (16 groups a block 92, 4 groups 99); with the next view's map
+// entry loaded ahead they take 65 (its gradient ahead too: 64).
 constexpr int DIFF_BWD_E = 64, DIFF_BWD_G = 8;
 __global__ void __launch_bounds__(DIFF_BWD_E * DIFF_BWD_G) k_diff_lit_bwd(const DiffView *views, uint32_t nviews,
                                                                           uint32_t nvert, unsigned long long nall,
@@ -4969,8 +4970,11 @@ __global__ void __launch_bounds__(DIFF_BWD_E * DIFF_BWD_G) k_diff_lit_bwd(const 
         const float *c = vcol + 4u * e;
         const Col vc = {sanitize(c[0], 0.0f), sanitize(c[1], 0.0f), sanitize(c[2], 0.0f), sanitize(c[3], 1.0f)};
         const Col k = col_clamp(vc);
-        for (uint32_t v = __builtin_amdgcn_readfirstlane(threadIdx.y); v < nviews; v += DIFF_BWD_G) {
-            const uint32_t at = views[v].vmap[e];
+        const uint32_t v0 = __builtin_amdgcn_readfirstlane(threadIdx.y);
+        uint32_t at_next = v0 < nviews ? views[v0].vmap[e] : 0xFFFFFFFFu;
+        for (uint32_t v = v0; v < nviews; v += DIFF_BWD_G) {
+            const uint32_t at = at_next;
+            if (v + DIFF_BWD_G < nviews) at_next = views[v + DIFF_BWD_G].vmap[e];
             if (at == 0xFFFFFFFFu) continue;
             const size_t i = (size_t)views[v].off + at;
             const float4 dl = reinterpret_cast<const float4 *>(dlit)[i];
