@@ -7022,20 +7022,30 @@ MTGL_API int mtgl_dev_read(mtgl_dev *d, uint32_t which, int32_t x, int32_t y, in
     return MTGL_OK;
 }
 
-// The device's address of host memory [p, p + bytes) when all of it is
-// pinned and mapped for the current device (hipHostMalloc or registered by
-// the caller), else null: a kernel can then write it.
-static uint8_t *mapped_host(void *p, size_t bytes)
+// The device's address of host memory [p, p + bytes) when all of it lies in
+// one pinned allocation mapped for the current device (hipHostMalloc or
+// registered by the caller), else null: a kernel can then write it.  Both
+// ends being pinned is not enough: host and device addresses agree here, so
+// two allocations with ordinary memory between them would look like one.
+static uint8_t *mapped_host(const void *p, size_t bytes)
 {
-    hipPointerAttribute_t a, b;
-    uint8_t *const last = (uint8_t *)p + bytes - 1;
-    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipPointerGetAttributes(&b, last) != hipSuccess) {
+    hipPointerAttribute_t a;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeHost || !a.devicePointer ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)a.devicePointer) != hipSuccess) {
         (void)hipGetLastError();   // (memory the runtime does not know)
         return nullptr;
     }
-    if (a.type != hipMemoryTypeHost || b.type != hipMemoryTypeHost || !a.devicePointer || !b.devicePointer) return nullptr;
-    if ((uint8_t *)b.devicePointer - (uint8_t *)a.devicePointer != (ptrdiff_t)(bytes - 1)) return nullptr;
+    const uintptr_t at = (uintptr_t)a.devicePointer, lo = (uintptr_t)base;
+    if (at < lo || bytes > size || at - lo > size - bytes) return nullptr;
     return (uint8_t *)a.devicePointer;
+}
+
+// Whether reads into [p, p + bytes) take that path (no header declares it: for tests).
+MTGL_API int mtgl_dev_host_direct(const void *p, uint64_t bytes)
+{
+    return p && bytes && mapped_host(p, (size_t)bytes) ? 1 : 0;
 }
 
 // A tightly packed window of the colour plane to host memory (k_read_pixels'

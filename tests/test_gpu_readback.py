@@ -73,3 +73,21 @@ def test_present(mtgl, oracle, pinned, fb, extra, shift):
     rows = m[GUARD + shift:GUARD + shift + H * pitch].reshape(H, pitch)
     assert (rows[:, :4 * W] == want.view(np.uint8).reshape(H, 4 * W)).all()
     assert (rows[:, 4 * W:] == 0xA5).all() and (m[:GUARD + shift] == 0xA5).all()
+
+
+def test_direct_only_within_one_allocation(mtgl):
+    """Reads the device may write itself: the whole range must be one pinned
+    allocation's.  A range from one into the next, with other memory between
+    them, is not (the check alone: nothing is read into it)."""
+    direct = mtgl.lib.mtgl_dev_host_direct
+    direct.argtypes = [ctypes.c_void_p, ctypes.c_uint64]
+    n = 1 << 20
+    a, b = sorted((torch.empty(n, dtype=torch.uint8, pin_memory=True) for _ in range(2)), key=lambda t: t.data_ptr())
+    assert b.data_ptr() - a.data_ptr() >= n
+    for t in (a, b):
+        assert direct(t.data_ptr(), n) == 1 and direct(t.data_ptr() + 4096, n - 4096) == 1
+        assert direct(t.data_ptr() + n - 1, 1) == 1
+        assert direct(t.data_ptr() + 1, n) == 0   # one byte past the allocation
+    assert direct(a.data_ptr(), b.data_ptr() - a.data_ptr() + n) == 0
+    assert direct(a.data_ptr() + n - 16, b.data_ptr() - a.data_ptr() - n + 32) == 0
+    assert direct(torch.empty(n, dtype=torch.uint8).data_ptr(), n) == 0
