@@ -5080,6 +5080,11 @@ struct Arena {
     size_t cap = 0;
 };
 
+// How an owner's launches ran, for tests (mtgl_dev_launch_trace).
+struct LaunchTrace {
+    uint64_t raster_blocks = 0;    // grid of the latest raster kernel
+};
+
 // Stream, pipeline buffers and counters shared by the launches of one owner
 // (a context for its own draws, a batch for its rounds).
 struct Exec {
@@ -5123,6 +5128,7 @@ struct Exec {
     uint32_t timing_count = 0;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pending_events;
     std::vector<hipEvent_t> free_events;
+    LaunchTrace trace;
 };
 
 // Device tables of one launch and what its kernels are launched with.  A
@@ -6183,8 +6189,6 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
         return rc;
     }
     HIPC(hipGetLastError());
-    // raster grids: no more blocks than items, which the estimated pairs bound
-    const uint64_t est_items = std::min<uint64_t>(cap, (uint64_t)est_pairs + 64u);
 
     // ---- K4
     RasterParams rp = {};
@@ -6205,9 +6209,14 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
     rp.stats = x.stat_slots;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     if (x.timing && !frozen && x.timing_count++ % x.timing_every == 0u) (void)take_event_pair(x, ev0, ev1);
-    // persistent grids over the work list (longest items first): at most one
-    // block per item, at most as many as are resident at once
-    const uint32_t nlist = (uint32_t)std::min<uint64_t>(est_items, (uint64_t)HEAVY_SPLIT * ntiles);
+    // persistent grids over the work list (longest items first), bounded by
+    // the items the launch's framebuffers can give, not by its triangles: two
+    // triangles may fill the screen.  Blocks past the list's end leave after
+    // one load, which 64 draws of a 12-triangle box at 1080p do not show (2.46
+    // ms; 2.50 with a grid bounded by 4 items per triangle, with which a
+    // full-screen quad ran on 64 waves: 3,690 us a frame, 300 now; at 4K
+    // 14,700 and 1,077)
+    const uint64_t nlist = (uint64_t)HEAVY_SPLIT * ntiles;
     auto grid = [&](int k) {
         // statistics take one slot per block: grids stay within STAT_SLOTS;
         // larger grids are whole runs of the XCD interleave (xcd_block)
@@ -6217,8 +6226,9 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
         // faster than three)
         const uint32_t over = k == 2 || k == 5 || k == 8 ? 6u : 3u;
         const uint32_t g = std::min<uint32_t>(over * x.resident[k] / x.grid_div, STAT_SLOTS);
-        uint32_t n = std::max<uint32_t>(1u, std::min<uint32_t>(nlist, g));
+        uint32_t n = std::max<uint32_t>(1u, (uint32_t)std::min<uint64_t>(nlist, g));
         if (n >= 64u) n &= ~63u;
+        x.trace.raster_blocks = n;
         return dim3(n);
     };
     const uint32_t LW = KIND_LAST_WRITER, ST = KIND_STENCIL, CO = KIND_COLOR;
@@ -7594,6 +7604,14 @@ static int confirm(mtgl_dev *d)
     d->ops.clear();
     ring_release(x);
     saw_meets(x, x.ctr_host->meets);
+    return MTGL_OK;
+}
+
+// (no header declares it: for tests)
+MTGL_API int mtgl_dev_launch_trace(const mtgl_dev *d, uint64_t *raster_blocks)
+{
+    if (!d || !raster_blocks) return MTGL_ERR_INVALID;
+    *raster_blocks = d->ex.trace.raster_blocks;
     return MTGL_OK;
 }
 
