@@ -139,6 +139,9 @@ struct __align__(16) RCold {
     float pad[2];
 };
 
+// launches between two waits whose met squares the host learns (use_bins)
+constexpr uint32_t MEETS_SLOTS = 16, MEETS_NONE = 0xFFFFFFFFu;
+
 // Counters of an Exec.  The first group belongs to one launch and is reset
 // by the launch's first kernel; the second persists across launches.
 struct Counters {
@@ -154,9 +157,11 @@ struct Counters {
                                   // later framebuffer write of this Exec is skipped until the host clears it
     unsigned long long poison_pairs;   // pairs that launch needed
     unsigned int poison_flags;    // its overflow_full
-    unsigned int meets;           // the latest launch's (set-up block, square it meets) pairs, capped at 2^32 - 1
+    unsigned int pad1;
     unsigned long long acc_tri_raster; // fan triangles and pairs of every launch that did not overflow
     unsigned long long acc_bin_pairs;
+    unsigned int meets[MEETS_SLOTS];   // of the launches the host keeps count of: (set-up block, square it meets)
+                                       // pairs, capped at 2^32 - 1
 };
 
 // A launch's work list lies in BIN_REGIONS regions of the list's memory, each
@@ -270,6 +275,7 @@ struct RasterParams {
     const RegionCounters *regions;
     uint32_t *kept, *meets;        // k_setup's 64 partial counts, for the first kernel of the stage (kept: only after
                                    // k_bin), else null
+    uint32_t meets_slot;           // of Counters::meets, or MEETS_NONE
     unsigned long long *stats;     // per block: fragments, algorithmic bytes (summed when read)
     Counters *ctr;
 };
@@ -3357,7 +3363,7 @@ __device__ __forceinline__ void end_binning(const RasterParams &P)
     Counters *c = P.ctr;
     const unsigned long long met = wave_inclusive_scan((unsigned long long)P.meets[threadIdx.x]);
     P.meets[threadIdx.x] = 0u;
-    if (threadIdx.x == 63) c->meets = (uint32_t)min(met, 0xFFFFFFFFull);
+    if (threadIdx.x == 63 && P.meets_slot < MEETS_SLOTS) c->meets[P.meets_slot] = (uint32_t)min(met, 0xFFFFFFFFull);
     if (!P.kept) return;
     const uint32_t k = P.kept[threadIdx.x];
     P.kept[threadIdx.x] = 0u;
@@ -4445,20 +4451,19 @@ __global__ void __launch_bounds__(256) k_clear_span(uint32_t *color, float *dept
 // cache lines (out is 16-byte aligned for BPP 4, 4-byte for BPP 3): out is
 // device memory, or the caller's own pinned memory over PCIe, which bounds
 // the kernel then.  poison (null: not wanted) receives the Exec's poison, and
-// the latest launch's count of met squares after it, in pinned host memory, so
-// that the wait for the pixels also tells the host whether the queued work
-// took effect; no pixel is stored when it did not.
+// the first nmeets of its launches' counts of met squares after it, in pinned
+// host memory, so that the wait for the pixels also tells the host whether the
+// queued work took effect; no pixel is stored when it did not.
 template <int BPP>
 __global__ void __launch_bounds__(256) k_read_pixels(const uint32_t *color, int32_t fb_w, int32_t fb_h, int32_t x,
                                                      int32_t y, int32_t flip, uint32_t w, int32_t r0, uint64_t n,
-                                                     uint8_t *out, const Counters *ctr, uint32_t *poison)
+                                                     uint8_t *out, const Counters *ctr, uint32_t *poison,
+                                                     uint32_t nmeets)
 {
     static_assert(BPP == 3 || BPP == 4, "GL_RGB or GL_RGBA");
     if (poison) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            poison[0] = ctr->poison;
-            poison[1] = ctr->meets;
-        }
+        if (blockIdx.x == 0 && threadIdx.x <= nmeets)
+            poison[threadIdx.x] = threadIdx.x == 0 ? ctr->poison : ctr->meets[threadIdx.x - 1u];
         if (exec_poisoned(ctr)) return;
     }
     const uint64_t i = 4ull * ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x);
@@ -5083,6 +5088,15 @@ struct Arena {
 // How an owner's launches ran, for tests (mtgl_dev_launch_trace).
 struct LaunchTrace {
     uint64_t raster_blocks = 0;    // grid of the latest raster kernel
+    uint64_t binned = 0, sorted = 0;   // launches k_bin and the tile sort took
+};
+
+// What tells a launch apart when the next frame has it again, and the part of
+// its (set-up block, square) pairs that meet.
+struct Spread {
+    uint64_t tri = 0, bins = 0, work = 0;
+    uint32_t nth = 0;              // among the launches of this many triangles and squares since the last wait
+    double part = 1.0;
 };
 
 // Stream, pipeline buffers and counters shared by the launches of one owner
@@ -5110,8 +5124,12 @@ struct Exec {
     Arena tbox, blk_box;                  // tile bounds per triangle and per set-up block (k_bin)
     RegionCounters *regions = nullptr;    // BIN_REGIONS: the work list's and vals' regions
     uint32_t *sums = nullptr;             // k_setup's partial counts: 64 of kept fan triangles, 64 of met squares
-    double spread = -1.0;                 // of the latest launch seen to end: the part of the (set-up block, square)
-    uint64_t last_work = 0;               // pairs that meet, of last_work in all (-1: none seen yet)
+    // how far apart the triangles of earlier launches lay (use_bins): launches
+    // seen to end, and those of the queue that the host will learn of
+    std::vector<Spread> seen;
+    uint32_t seen_next = 0;               // replaced next once the table is full
+    Spread queued[MEETS_SLOTS];           // by slot of Counters::meets
+    uint32_t nqueued = 0;                 // since the last wait; the latest MEETS_SLOTS of them are known
     uint32_t overflow_cap = 0;
     Arena keys[2], vals[2], sort_tmp, tile_list;   // (tile, record) pairs and their sort
     Arena tile_start, tile_end, tile_gen;          // per launch-wide tile: bin range, generation of the range
@@ -5142,8 +5160,8 @@ struct Launch {
     uint32_t sblocks = 0;
     uint32_t nbins = 0;            // k_bin's squares
     uint32_t region_items = 0;     // items a region of the work list may hold then
-    uint64_t work = 0;             // (set-up block, square) pairs
     bool bins = false;             // binned by k_bin (else by the tile sort)
+    uint32_t meets_slot = MEETS_NONE;
     uint32_t ntri1 = 0;            // one scene: its triangles and framebuffer
     int32_t fb_w1 = 0, fb_h1 = 0, tiles_x1 = 0, side1 = 0;
     uint32_t cols1 = 0;
@@ -5635,7 +5653,7 @@ struct Sizes {
     uint64_t tri = 0, tiles = 0;
     uint64_t sblocks = 0;          // set-up blocks (each scene starts a block of its own)
     uint64_t bins = 0;             // k_bin's squares
-    uint64_t work = 0, work_sum = 0;   // (set-up block, square) pairs of the largest scene and of all
+    uint64_t work = 0;             // (set-up block, square) pairs
     uint64_t items = 0;            // work list items of one region after k_bin
     bool crowded = false;          // a scene of over BIN_LARGE triangles, over BIN_LARGE_DENSE per tile
     bool cold = false;
@@ -5646,33 +5664,80 @@ struct Sizes {
 // of those that meet it: little where a block's triangles lie together, as a
 // mesh's do (a 1080p frame's 32,768-triangle sphere, of whose 1.04M (block,
 // square) pairs 1% meet, takes 88 us so and 104 sorted), all of them where
-// they lie anywhere (10,000 triangles scattered over 1080p, 0.32M pairs
-// nearly all of which meet: 117 and 105; 40,000: 247 and 163; 2,000, 0.06M
-// pairs: 72 and 71).  The set-up counts the pairs that meet, and the host
-// takes the part of them in the latest launch it has seen end for the next
-// one's; before it has seen any, launches of at most BIN_UNSEEN pairs.  Two
-// more go through the sort: meshes so large and dense that many squares list
-// more than a window holds (204,800 triangles of a sphere take 459 us at
-// 1080p and 353 sorted, 100,352 181 and 187; at 4K, 439 and 818), and
-// launches of so many squares that they wait for the chip in turn (the 512
-// scenes of the batched workload 2.37 ms and 2.22).  The choice changes no
-// pixel.
-constexpr double BIN_MEETS = 200e3;
+// they lie anywhere.  Of frames of triangles scattered over the screen, those
+// with fewer pairs are faster with k_bin and those with more sorted: at 1080p
+// 128,000 pairs 265 us and 271, 192,000 281 and 283, 255,000 296 and 295,
+// 320,000 305 and 299, 1.28M 423 and 339; at 4K 261,000 743 and 727, at 720p
+// 144,000 183 and 195, at 640x480 187,000 163 and 156.  The set-up counts the
+// pairs that meet.  Launches of few pairs need no count; for the others the
+// host expects the part that met in the same launch of an earlier frame: one
+// of as many squares and (nearly) as many triangles, by its place among those
+// when there are several.  Before it has seen one, launches of at most
+// BIN_UNSEEN pairs go to k_bin.  Two more kinds are sorted: meshes so large
+// and dense that many squares list more than a window holds (204,800
+// triangles of a sphere take 459 us at 1080p and 353 sorted, 100,352 181 and
+// 187; at 4K, 439 and 818), and launches of so many squares that they wait for
+// the chip in turn (the 512 scenes of the batched workload 2.37 ms and 2.22).
+// The choice changes no pixel.
+constexpr uint64_t BIN_MEETS = 200'000;
 constexpr uint64_t BIN_UNSEEN = 1'500'000;
 constexpr uint64_t BIN_MAX = 16384;      // squares of a launch
 constexpr uint64_t BIN_LARGE = 128u << 10, BIN_LARGE_DENSE = 4;   // triangles of a scene, and per tile of it
 constexpr uint32_t BIN_DENSE = 24;       // triangles per tile above which squares shrink
+constexpr size_t SPREADS = 64;           // launches of earlier frames a table holds
 
-bool use_bins(const Exec &x, const Sizes &z)
+// The part of a launch's pairs expected to meet: that of the seen launch with
+// as many squares and the nearest number of triangles, at most a quarter away
+// (of equal ones the one of the same place); -1 when there is none.
+double expected_part(const Exec &x, const Spread &q)
 {
-    if (z.bins > BIN_MAX || z.crowded) return false;
-    return x.spread < 0.0 ? z.work <= BIN_UNSEEN : x.spread * (double)z.work <= BIN_MEETS;
+    uint64_t best = UINT64_MAX;
+    double part = -1.0;
+    for (const Spread &e : x.seen) {
+        if (e.bins != q.bins) continue;
+        const uint64_t diff = e.tri > q.tri ? e.tri - q.tri : q.tri - e.tri;
+        if (4u * diff > q.tri) continue;
+        const uint64_t rank = 2u * diff + (e.nth != q.nth ? 1u : 0u);
+        if (rank >= best) continue;
+        best = rank;
+        part = e.part;
+    }
+    return part;
 }
 
-// the met squares of the launch the host has just seen end
-void saw_meets(Exec &x, uint32_t meets)
+// Whether k_bin takes a launch about to be queued; slot: where its count of
+// met squares goes when the host wants it.
+bool use_bins(Exec &x, const Sizes &z, uint32_t &slot)
 {
-    if (x.last_work) x.spread = (double)meets / (double)x.last_work;
+    slot = MEETS_NONE;
+    if (z.bins > BIN_MAX || z.crowded) return false;
+    if (z.work <= BIN_MEETS) return true;
+    Spread q;
+    q.tri = z.tri;
+    q.bins = z.bins;
+    q.work = z.work;
+    for (uint32_t k = 0; k < std::min(x.nqueued, MEETS_SLOTS); k++)
+        if (x.queued[k].tri == q.tri && x.queued[k].bins == q.bins) q.nth++;
+    slot = x.nqueued++ % MEETS_SLOTS;
+    x.queued[slot] = q;
+    const double part = expected_part(x, q);
+    return part < 0.0 ? z.work <= BIN_UNSEEN : part * (double)z.work <= (double)BIN_MEETS;
+}
+
+// The host has seen the queued launches end, with these counts of met squares.
+void saw_meets(Exec &x, const volatile uint32_t *meets)
+{
+    for (uint32_t k = 0; k < std::min(x.nqueued, MEETS_SLOTS); k++) {
+        Spread e = x.queued[k];
+        e.part = (double)meets[k] / (double)e.work;
+        auto same = std::find_if(x.seen.begin(), x.seen.end(), [&](const Spread &o) {
+            return o.tri == e.tri && o.bins == e.bins && o.nth == e.nth;
+        });
+        if (same != x.seen.end()) *same = e;
+        else if (x.seen.size() < SPREADS) x.seen.push_back(e);
+        else x.seen[x.seen_next++ % SPREADS] = e;
+    }
+    x.nqueued = 0;
 }
 
 // Tiles per side of k_bin's squares: BIN_T while the scene has few triangles
@@ -5703,8 +5768,7 @@ Sizes scene_sizes(const SceneIn *in, uint32_t n)
         const uint64_t bins = scene_bins(in[i].dev, ntri), side = bin_side(in[i].dev, ntri);
         z.bins += bins;
         z.crowded |= ntri > BIN_LARGE && ntri > BIN_LARGE_DENSE * (uint64_t)in[i].dev->tiles_x * (uint64_t)in[i].dev->tiles_y;
-        z.work = std::max<uint64_t>(z.work, bins * blocks_for(ntri, SETUP_BLOCK));
-        z.work_sum += bins * blocks_for(ntri, SETUP_BLOCK);
+        z.work += bins * blocks_for(ntri, SETUP_BLOCK);
         z.items += HEAVY_SPLIT * side * side * ((bins + BIN_REGIONS - 1) / BIN_REGIONS);
         z.tiles += (uint64_t)in[i].dev->tiles_x * (uint64_t)in[i].dev->tiles_y;
         z.cold |= needs_cold(dr->raster);
@@ -5712,7 +5776,8 @@ Sizes scene_sizes(const SceneIn *in, uint32_t n)
     return z;
 }
 
-int reserve_scene_buffers(Exec &x, const Sizes &z)
+// (bins: for k_bin, else for the tile sort)
+int reserve_scene_buffers(Exec &x, const Sizes &z, bool bins)
 {
     int rc;
     const size_t t = (size_t)z.tri;
@@ -5724,7 +5789,7 @@ int reserve_scene_buffers(Exec &x, const Sizes &z)
     if ((rc = arena_reserve(x, x.n_rt, t * sizeof(uint32_t)))) return rc;
     if ((rc = arena_reserve(x, x.rec_base, t * sizeof(uint32_t)))) return rc;
     const size_t sb = (size_t)std::max<uint64_t>(z.sblocks, 1u);
-    if (use_bins(x, z)) {
+    if (bins) {
         if ((rc = arena_reserve(x, x.tbox, t * sizeof(uint2)))) return rc;
         return arena_reserve(x, x.blk_box, sb * sizeof(uint2));
     }
@@ -5804,16 +5869,15 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
     L.tri_total = (uint32_t)z.tri;
     L.tiles_total = (uint32_t)z.tiles;
     L.sblocks = (uint32_t)sb;
-    L.bins = use_bins(x, z);
+    L.bins = use_bins(x, z, L.meets_slot);
     L.nbins = L.bins ? (uint32_t)z.bins : 0u;
     L.region_items = L.bins ? (uint32_t)z.items : 0u;
-    L.work = z.work_sum;
     L.any_cold = z.cold;
     L.gen_need = GEN_PLAIN;
     L.simple = true;
 
     int rc;
-    if ((rc = reserve_scene_buffers(x, z))) return rc;
+    if ((rc = reserve_scene_buffers(x, z, L.bins))) return rc;
     for (const Plan &p : plan) {
         if ((raster_kind(p.s->dr->raster, p.tx) & KIND_LAST_WRITER) && p.s->dev->capture) {
             mtgl_dev *d = p.s->dev;
@@ -6156,6 +6220,7 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
 
     // ---- K3: every tile's records in submission order and the work list
     uint32_t *vals = as<uint32_t>(x.vals[0]);
+    (L.bins ? x.trace.binned : x.trace.sorted)++;
     if (L.bins) {
         BinParams bp = {};
         bp.scenes = L.sp;
@@ -6206,6 +6271,7 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
     rp.ctr = x.ctr;
     rp.kept = L.bins ? x.sums : nullptr;
     rp.meets = x.sums + 64;
+    rp.meets_slot = frozen ? MEETS_NONE : L.meets_slot;
     rp.stats = x.stat_slots;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     if (x.timing && !frozen && x.timing_count++ % x.timing_every == 0u) (void)take_event_pair(x, ev0, ev1);
@@ -6274,7 +6340,6 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
             x.free_events.push_back(ev1);
         }
     }
-    x.last_work = L.work;
     x.ctr_clean = true;   // (left so by k_expand, or by the raster stage's first kernel)
     return L.unsupported ? MTGL_ERR_UNSUPPORTED : MTGL_OK;
 }
@@ -6691,7 +6756,7 @@ int batch_reserve(mtgl_batch *b)
         m.cold |= z.cold;
     }
     if (m.tri > 0x0FFFFFFFull) return MTGL_ERR_OUT_OF_MEMORY;
-    return m.tri ? reserve_scene_buffers(b->ex, m) : MTGL_OK;
+    return m.tri ? reserve_scene_buffers(b->ex, m, true) : MTGL_OK;
 }
 
 int batch_build_inner(mtgl_batch *b, int autotune)
@@ -7078,10 +7143,11 @@ static int read_window(mtgl_dev *d, int32_t x, int32_t y, int32_t flip, int32_t 
     int rc = dev_join(d);
     if (rc) return rc;
     const size_t row_bytes = (size_t)width * (size_t)bpp;
+    const uint32_t nmeets = std::min(ex.nqueued, MEETS_SLOTS);
     auto launch = [&](int32_t r0, uint64_t n, uint8_t *out, uint32_t *poison) {
         hipLaunchKernelGGL(bpp == 4 ? k_read_pixels<4> : k_read_pixels<3>, dim3((uint32_t)blocks_for((n + 3) / 4, 256)),
                            dim3(256), 0, ex.stream, d->color, d->w, d->h, x, y, flip, (uint32_t)width, r0, n, out,
-                           (const Counters *)ex.ctr, poison);
+                           (const Counters *)ex.ctr, poison, nmeets);
         return hipGetLastError();
     };
     uint8_t *const host = row_bytes <= SIZE_MAX / (size_t)height ? mapped_host(dst, row_bytes * (size_t)height) : nullptr;
@@ -7096,7 +7162,7 @@ static int read_window(mtgl_dev *d, int32_t x, int32_t y, int32_t flip, int32_t 
         }
         d->ops.clear();   // every queued op took effect
         ring_release(ex);
-        saw_meets(ex, ((volatile uint32_t *)ex.report)[1]);
+        saw_meets(ex, (const volatile uint32_t *)ex.report + 1);
         return MTGL_OK;
     }
     if ((rc = confirm(d))) return rc;
@@ -7493,6 +7559,7 @@ MTGL_API int mtgl_dev_draw_pixels_static(mtgl_dev *d, const mtgl_pixels *p)
         }
         d->ops.clear();
         ring_release(d->ex);
+        saw_meets(d->ex, d->ex.ctr_host->meets);
     }
     uint8_t *buf = (uint8_t *)g_scratch[d->device];
     std::lock_guard<std::mutex> lock(g_scratch_mu[d->device]);
@@ -7576,6 +7643,7 @@ static int confirm(mtgl_dev *d)
         uint32_t poison = 0;
         int rc = exec_take_poison(x, poison);
         if (rc) return rc;
+        saw_meets(x, x.ctr_host->meets);
         if (!poison) break;
         size_t first = d->ops.size();
         for (size_t i = 0; i < d->ops.size(); i++)
@@ -7603,15 +7671,17 @@ static int confirm(mtgl_dev *d)
     }
     d->ops.clear();
     ring_release(x);
-    saw_meets(x, x.ctr_host->meets);
     return MTGL_OK;
 }
 
 // (no header declares it: for tests)
-MTGL_API int mtgl_dev_launch_trace(const mtgl_dev *d, uint64_t *raster_blocks)
+MTGL_API int mtgl_dev_launch_trace(const mtgl_dev *d, uint64_t *out)
 {
-    if (!d || !raster_blocks) return MTGL_ERR_INVALID;
-    *raster_blocks = d->ex.trace.raster_blocks;
+    if (!d || !out) return MTGL_ERR_INVALID;
+    const LaunchTrace &t = d->ex.trace;
+    out[0] = t.raster_blocks;
+    out[1] = t.binned;
+    out[2] = t.sorted;
     return MTGL_OK;
 }
 

@@ -1,10 +1,12 @@
-"""How launches are sized: grids by what a draw can cover, whatever its number
-of triangles."""
+"""How launches are sized and binned: grids by what a draw can cover, whatever
+its number of triangles; k_bin or the tile sort by what each draw of a frame
+was in an earlier one."""
 import ctypes
 
 import pytest
 
 from mytinygl_amd.gl import ENUMS as E
+from test_gpu_bins import _ortho, _triangles
 
 pytestmark = pytest.mark.gpu
 
@@ -14,9 +16,9 @@ ALL = E["GL_COLOR_BUFFER_BIT"] | E["GL_DEPTH_BUFFER_BIT"] | E["GL_STENCIL_BUFFER
 def trace(g, ctx):
     fn = g.lib.mtgl_dev_launch_trace
     fn.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint64)]
-    out = ctypes.c_uint64()
-    assert fn(g.device(ctx), ctypes.byref(out)) == 0
-    return out.value
+    out = (ctypes.c_uint64 * 3)()
+    assert fn(g.device(ctx), out) == 0
+    return dict(zip(("raster_blocks", "binned", "sorted"), out))
 
 
 @pytest.mark.parametrize("blend", [False, True])
@@ -40,7 +42,63 @@ def test_few_triangles_get_a_whole_grid(mtgl, fb, blend):
         mtgl.finish(ctx)
         tiles = ((W + 7) // 8) * ((H + 7) // 8)
         # four waves on each of 256 CUs, or a wave per tile where there are fewer
-        assert trace(mtgl, ctx) >= min(1024, max(1, tiles if tiles < 64 else tiles & ~63))
+        assert trace(mtgl, ctx)["raster_blocks"] >= min(1024, max(1, tiles if tiles < 64 else tiles & ~63))
     finally:
         mtgl.destroy_context(ctx)
         mtgl.release()
+
+
+def _frames(g, W, H, frames):
+    """Draws frames of (triangles, together) draws with a wait after each;
+    returns the launches of each frame by binner."""
+    import numpy as np
+    ctx = g.create_context(W, H)
+    out = []
+    try:
+        _ortho(g, W, H)
+        g.glEnableClientState(E["GL_VERTEX_ARRAY"])
+        g.glEnableClientState(E["GL_COLOR_ARRAY"])
+        for draws in frames:
+            before = trace(g, ctx)
+            g.glClear(ALL)
+            for n, together in draws:
+                pos, col = _triangles(np.random.default_rng(n), W, H, n, 9, together)
+                g.glVertexPointer(3, E["GL_FLOAT"], 0, g.keep(pos))
+                g.glColorPointer(4, E["GL_FLOAT"], 0, g.keep(col))
+                g.glDrawArrays(E["GL_TRIANGLES"], 0, 3 * n)
+            g.finish(ctx)
+            after = trace(g, ctx)
+            out.append((after["binned"] - before["binned"], after["sorted"] - before["sorted"]))
+    finally:
+        g.destroy_context(ctx)
+        g.release()
+    return out
+
+
+MESH, SCATTERED, OVERLAY = (32_768, True), (40_000, False), (2, False)
+
+
+@pytest.mark.parametrize("frame,binned,sort", [
+    ([MESH], 1, 0), ([SCATTERED], 0, 1),
+    ([MESH, OVERLAY], 2, 0),                # a small draw at the end says nothing of the mesh
+    ([SCATTERED, OVERLAY], 1, 1),
+    ([MESH, SCATTERED], 1, 1), ([SCATTERED, MESH], 1, 1),
+    ([SCATTERED, MESH, OVERLAY, SCATTERED, MESH], 3, 2),
+    ([(32_768, False), MESH], 1, 1),        # as many triangles: told apart by their places
+], ids=lambda v: "".join("MSO"[min(d[0] == 40_000, 1) + 2 * (d[0] == 2)] for d in v) if isinstance(v, list) else None)
+def test_each_draw_is_binned_by_its_own_spread(mtgl, frame, binned, sort):
+    got = _frames(mtgl, 1920, 1080, [frame] * 4)
+    assert got[1:] == [(binned, sort)] * 3
+
+
+def test_draws_of_changing_sizes(mtgl):
+    """A cloud of points that grows and shrinks from frame to frame stays sorted."""
+    got = _frames(mtgl, 1920, 1080, [[(n, False)] for n in (40_000, 41_000, 38_500, 44_000, 36_000)])
+    assert got[1:] == [(0, 1)] * 4
+
+
+def test_more_large_draws_than_counts_are_kept_for(mtgl):
+    """The counts of the latest 16 large draws of a frame reach the host."""
+    n = 20
+    got = _frames(mtgl, 640, 480, [[(48_000 + 64 * k, False) for k in range(n)]] * 3)
+    assert got[0] == (n, 0) and got[2] == (0, n)
