@@ -6759,21 +6759,37 @@ int batch_reserve(mtgl_batch *b)
     return m.tri ? reserve_scene_buffers(b->ex, m, true) : MTGL_OK;
 }
 
+// Whether some round would now be binned the other way than it was.
+bool batch_rebins(mtgl_batch *b)
+{
+    Exec &x = b->ex;
+    bool other = false;
+    for (BatchRound &R : b->rounds) {
+        if (R.launch.ns == 0) continue;
+        uint32_t slot;
+        other |= use_bins(x, scene_sizes(R.scenes.data(), (uint32_t)R.scenes.size()), slot) != R.launch.bins;
+    }
+    x.nqueued = 0;   // (asked, not queued)
+    return other;
+}
+
 int batch_build_inner(mtgl_batch *b, int autotune)
 {
     Exec &x = b->ex;
     int rc;
     if ((rc = batch_reserve(b))) return rc;
     // sizing runs: every round in order, until none needs larger arrays than
-    // the earlier rounds grew them to
+    // the earlier rounds grew them to, and each is binned as its own count of
+    // met squares asks for (the replays' rounds stay as this leaves them)
     for (int attempt = 0;; attempt++) {
         if ((rc = batch_run(b, false))) return rc;
         HIPC(hipStreamSynchronize(x.stream));
         uint32_t poison = 0;
         if ((rc = exec_take_poison(x, poison))) return rc;
-        if (!poison) break;
+        saw_meets(x, x.ctr_host->meets);
+        if (!poison && !batch_rebins(b)) break;
         if (attempt >= 16) return MTGL_ERR_OUT_OF_MEMORY;
-        exec_grow(x, *x.ctr_host, b->rounds[poison - 1].launch.tri_total);
+        if (poison) exec_grow(x, *x.ctr_host, b->rounds[poison - 1].launch.tri_total);
         ring_release(x);
     }
     // a later round may have grown a buffer that an earlier round's tables
@@ -6783,6 +6799,7 @@ int batch_build_inner(mtgl_batch *b, int autotune)
         if ((rc = prepare_launch(x, R.launch, R.scenes.data(), (uint32_t)R.scenes.size()))) return rc;
         R.launch.pairs_cap = pairs_room(x, R.launch.bins);
     }
+    x.nqueued = 0;   // (prepared, not run)
     HIPC(hipStreamSynchronize(x.stream));
     ring_release(x);
     b->info.heavy_bin = x.heavy_bin;
@@ -7847,6 +7864,17 @@ MTGL_API int mtgl_batch_stats_reset(mtgl_batch *b)
 {
     if (!b) return MTGL_ERR_INVALID;
     return exec_stats_reset(b->ex);
+}
+
+// The rounds of the captured replay that k_bin and the tile sort take (no
+// header declares it: for tests).
+MTGL_API int mtgl_batch_launch_trace(const mtgl_batch *b, uint64_t *out)
+{
+    if (!b || !out) return MTGL_ERR_INVALID;
+    out[0] = out[1] = 0;
+    for (const BatchRound &R : b->rounds)
+        if (R.launch.ns) out[R.launch.bins ? 0 : 1]++;
+    return MTGL_OK;
 }
 
 // ---- differentiable shading

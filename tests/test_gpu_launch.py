@@ -3,8 +3,10 @@ its number of triangles; k_bin or the tile sort by what each draw of a frame
 was in an earlier one."""
 import ctypes
 
+import numpy as np
 import pytest
 
+from conftest import plane_diffs
 from mytinygl_amd.gl import ENUMS as E
 from test_gpu_bins import _ortho, _triangles
 
@@ -51,7 +53,6 @@ def test_few_triangles_get_a_whole_grid(mtgl, fb, blend):
 def _frames(g, W, H, frames):
     """Draws frames of (triangles, together) draws with a wait after each;
     returns the launches of each frame by binner."""
-    import numpy as np
     ctx = g.create_context(W, H)
     out = []
     try:
@@ -102,3 +103,54 @@ def test_more_large_draws_than_counts_are_kept_for(mtgl):
     n = 20
     got = _frames(mtgl, 640, 480, [[(48_000 + 64 * k, False) for k in range(n)]] * 3)
     assert got[0] == (n, 0) and got[2] == (0, n)
+
+
+def _batch(g, W, H, n, rounds):
+    """n contexts' (triangles, together) draws, a round each, recorded and
+    launched once; the planes of each context and the rounds by binner."""
+    ctxs = [g.create_context(W, H) for _ in range(n)]
+    b = g.batch()
+    try:
+        b.begin()
+        for k, c in enumerate(ctxs):
+            g.gl_make_current(c)
+            _ortho(g, W, H)
+            g.glEnableClientState(E["GL_VERTEX_ARRAY"])
+            g.glEnableClientState(E["GL_COLOR_ARRAY"])
+            g.glClear(ALL)
+            for m, together in rounds:
+                pos, col = _triangles(np.random.default_rng(m + k), W, H, m, 9, together)
+                g.glVertexPointer(3, E["GL_FLOAT"], 0, g.keep(pos))
+                g.glColorPointer(4, E["GL_FLOAT"], 0, g.keep(col))
+                g.glDrawArrays(E["GL_TRIANGLES"], 0, 3 * m)
+        b.end(False)
+        by = None
+        if g.kind == "mtgl":
+            fn = g.lib.mtgl_batch_launch_trace
+            fn.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint64)]
+            out = (ctypes.c_uint64 * 2)()
+            assert fn(b.h, out) == 0
+            by = tuple(out)
+        b.launch()
+        assert b.sync() == 0
+        return [g.read_framebuffer(c, W, H) for c in ctxs], by
+    finally:
+        b.destroy()
+        for c in ctxs:
+            g.destroy_context(c)
+        g.release()
+
+
+@pytest.mark.parametrize("rounds,by", [
+    ([(40_000, False)], (0, 1)), ([(32_768, True)], (1, 0)), ([(40_000, False), (32_768, True)], (1, 1)),
+    ([(32_768, True), (40_000, False), (500, False)], (2, 1)),
+    ([(32_768, True), (32_768, False)], (1, 1)),
+], ids=["s", "m", "sm", "mso", "same"])
+def test_batch_rounds_are_binned_by_their_own_spread(mtgl, oracle, rounds, by):
+    """A batch learns how far its rounds' triangles lie apart while it is built."""
+    W, H, n = 1024, 600, 2
+    want, _ = _batch(oracle, W, H, n, rounds)
+    got, took = _batch(mtgl, W, H, n, rounds)
+    assert took == by
+    for a, b in zip(want, got):
+        assert plane_diffs(a, b) == {"color": 0, "depth": 0, "stencil": 0}
