@@ -266,6 +266,7 @@ struct RasterParams {
     const uint32_t *tile_pre;      // nscenes + 1 first global tiles
     const uint32_t *tile_scene;    // global tile -> scene (nscenes > 1)
     uint32_t nscenes;
+    uint32_t meets_slot;           // of Counters::meets, or MEETS_NONE
     const RTri *rt;
     const RCold *rcold;
     const uint32_t *vals;          // per bin, in submission order: record slot
@@ -275,7 +276,6 @@ struct RasterParams {
     const RegionCounters *regions;
     uint32_t *kept, *meets;        // k_setup's 64 partial counts, for the first kernel of the stage (kept: only after
                                    // k_bin), else null
-    uint32_t meets_slot;           // of Counters::meets, or MEETS_NONE
     unsigned long long *stats;     // per block: fragments, algorithmic bytes (summed when read)
     Counters *ctr;
 };
@@ -5650,10 +5650,10 @@ VSlots vertex_slots(const mtgl_dev *d, const mtgl_draw *dr)
 
 // Triangle and tile totals of a set of scenes and the buffers they need.
 struct Sizes {
-    uint64_t tri = 0, tiles = 0;
+    uint64_t scenes = 0, tri = 0, tiles = 0;
     uint64_t sblocks = 0;          // set-up blocks (each scene starts a block of its own)
     uint64_t bins = 0;             // k_bin's squares
-    uint64_t work = 0;             // (set-up block, square) pairs
+    uint64_t work = 0, work_max = 0;   // (set-up block, square) pairs, of all scenes and of the largest
     uint64_t items = 0;            // work list items of one region after k_bin
     bool crowded = false;          // a scene of over BIN_LARGE triangles, over BIN_LARGE_DENSE per tile
     bool cold = false;
@@ -5672,16 +5672,21 @@ struct Sizes {
 // pairs that meet.  Launches of few pairs need no count; for the others the
 // host expects the part that met in the same launch of an earlier frame: one
 // of as many squares and (nearly) as many triangles, by its place among those
-// when there are several.  Before it has seen one, launches of at most
-// BIN_UNSEEN pairs go to k_bin.  Two more kinds are sorted: meshes so large
-// and dense that many squares list more than a window holds (204,800
+// when there are several.  Before it has seen one, launches with at most
+// BIN_UNSEEN pairs in any scene go to k_bin.  Two more kinds are sorted: meshes
+// so large and dense that many squares list more than a window holds (204,800
 // triangles of a sphere take 459 us at 1080p and 353 sorted, 100,352 181 and
 // 187; at 4K, 439 and 818), and launches of so many squares that they wait for
-// the chip in turn (the 512 scenes of the batched workload 2.37 ms and 2.22).
-// The choice changes no pixel.
+// the chip in turn: any of more than BIN_MAX (the 512 scenes of the batched
+// workload 2.37 ms and 2.22), and those of several scenes of more than
+// BIN_MANY with few triangles for them (500 triangles a scene: 32 scenes of
+// 256 squares 160 us and 138, 96 of 64 202 and 169, 64 of 64 159 and 145, 12
+// of 256 103 and 107; 20,000 in 32 scenes of 256 squares 517 and 555).  The
+// choice changes no pixel.
 constexpr uint64_t BIN_MEETS = 200'000;
 constexpr uint64_t BIN_UNSEEN = 1'500'000;
 constexpr uint64_t BIN_MAX = 16384;      // squares of a launch
+constexpr uint64_t BIN_MANY = 4096, BIN_SPARSE = 32;   // ... of several scenes with fewer triangles per square
 constexpr uint64_t BIN_LARGE = 128u << 10, BIN_LARGE_DENSE = 4;   // triangles of a scene, and per tile of it
 constexpr uint32_t BIN_DENSE = 24;       // triangles per tile above which squares shrink
 constexpr size_t SPREADS = 64;           // launches of earlier frames a table holds
@@ -5711,6 +5716,7 @@ bool use_bins(Exec &x, const Sizes &z, uint32_t &slot)
 {
     slot = MEETS_NONE;
     if (z.bins > BIN_MAX || z.crowded) return false;
+    if (z.scenes > 1u && z.bins > BIN_MANY && z.tri < BIN_SPARSE * z.bins) return false;
     if (z.work <= BIN_MEETS) return true;
     Spread q;
     q.tri = z.tri;
@@ -5721,7 +5727,7 @@ bool use_bins(Exec &x, const Sizes &z, uint32_t &slot)
     slot = x.nqueued++ % MEETS_SLOTS;
     x.queued[slot] = q;
     const double part = expected_part(x, q);
-    return part < 0.0 ? z.work <= BIN_UNSEEN : part * (double)z.work <= (double)BIN_MEETS;
+    return part < 0.0 ? z.work_max <= BIN_UNSEEN : part * (double)z.work <= (double)BIN_MEETS;
 }
 
 // The host has seen the queued launches end, with these counts of met squares.
@@ -5763,12 +5769,14 @@ Sizes scene_sizes(const SceneIn *in, uint32_t n)
         if (!draw_mode_ok(dr->mode)) continue;
         const uint32_t ntri = tri_count(dr->mode, dr->count);
         if (ntri == 0) continue;
+        z.scenes++;
         z.tri += ntri;
         z.sblocks += blocks_for(ntri, SETUP_BLOCK);
         const uint64_t bins = scene_bins(in[i].dev, ntri), side = bin_side(in[i].dev, ntri);
         z.bins += bins;
         z.crowded |= ntri > BIN_LARGE && ntri > BIN_LARGE_DENSE * (uint64_t)in[i].dev->tiles_x * (uint64_t)in[i].dev->tiles_y;
         z.work += bins * blocks_for(ntri, SETUP_BLOCK);
+        z.work_max = std::max<uint64_t>(z.work_max, bins * blocks_for(ntri, SETUP_BLOCK));
         z.items += HEAVY_SPLIT * side * side * ((bins + BIN_REGIONS - 1) / BIN_REGIONS);
         z.tiles += (uint64_t)in[i].dev->tiles_x * (uint64_t)in[i].dev->tiles_y;
         z.cold |= needs_cold(dr->raster);
