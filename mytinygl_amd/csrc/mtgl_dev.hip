@@ -139,6 +139,8 @@ struct __align__(16) RCold {
     float pad[2];
 };
 
+// what a launch may need more of: clip slots, pairs for the tile sort, records in a region of k_bin
+constexpr uint32_t OVERFLOW_CLIP = 1u, OVERFLOW_PAIRS = 2u, OVERFLOW_BINS = 4u;
 // launches between two waits whose met squares the host learns (use_bins)
 constexpr uint32_t MEETS_SLOTS = 16, MEETS_NONE = 0xFFFFFFFFu;
 
@@ -148,7 +150,7 @@ struct Counters {
     unsigned long long npairs;    // (tile, record) pairs of the launch (the pair-count scan or k_expand)
     unsigned int unsupported;
     unsigned int noverflow;       // overflow slots requested by clipped triangles
-    unsigned int overflow_full;   // bit 0: the clip pool was too small; bit 1: the pair arrays were
+    unsigned int overflow_full;   // OVERFLOW_*: what was too small
     unsigned int nbig;            // triangles queued for the one-wave pair expansion
     unsigned int pad0;
     // persistent
@@ -1086,7 +1088,7 @@ __device__ __noinline__ uint32_t setup_clipped(const SetupParams &P, const mtgl_
     if (n < 3) return 0;
     base = atomicAdd(&P.ctr->noverflow, (uint32_t)(n - 2));
     if (base + (uint32_t)(n - 2) > P.overflow_cap) {
-        atomicOr(&P.ctr->overflow_full, 1u);
+        atomicOr(&P.ctr->overflow_full, OVERFLOW_CLIP);
         return 0;
     }
     uint32_t nout = 0;
@@ -1584,7 +1586,7 @@ __global__ void __launch_bounds__(SETUP_BLOCK) k_expand(const SetupParams *Ss, c
             const unsigned long long total = blk_off ? ctr->npairs : sum_all;
             const uint32_t ovf = ctr->overflow_full, poison = ctr->poison, sticky = ctr->sticky;
             const unsigned long long acc_tri = ctr->acc_tri_raster, acc_pairs = ctr->acc_bin_pairs;
-            const uint32_t over = ovf | (total > cap ? 2u : 0u);
+            const uint32_t over = ovf | (total > cap ? OVERFLOW_PAIRS : 0u);
             if (over) {
                 if (atomicCAS(&ctr->poison, 0u, seq) == 0u) {
                     ctr->poison_pairs = total;
@@ -2221,6 +2223,14 @@ struct BinParams {
     Counters *ctr;
 };
 
+// The region of a square, by its column and row: a row's squares and a
+// column's both go round all regions, so that a narrow or a flat object fills
+// them alike.
+__device__ __forceinline__ uint32_t bin_region(uint32_t col, uint32_t row, uint32_t scene)
+{
+    return (col + 5u * row + scene) % BIN_REGIONS;
+}
+
 struct BinArea {
     uint32_t lo, hi;                   // first and last tile column | row << 16 (TBox layout)
 };
@@ -2417,7 +2427,7 @@ __global__ void __launch_bounds__(BIN_THREADS) k_bin(BinParams P)
     if (w == 0u) {
         // the square's range of vals and its items' places in the work list,
         // in its region of both
-        const uint32_t region = blockIdx.x % BIN_REGIONS;
+        const uint32_t region = bin_region(bin % cols, bin / cols, sc);
         const uint32_t inc = dpp_incl_scan(run);
         const uint32_t sum = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
         const bool hv = run > P.heavy_bin, md = !hv && run > MED_BIN, ltl = !hv && !md && run != 0u;
@@ -2431,15 +2441,15 @@ __global__ void __launch_bounds__(BIN_THREADS) k_bin(BinParams P)
             const bool over = at + sum > P.cap;
             if (over) {
                 // more records than the region of vals holds: the launch
-                // poisons the Exec, with the pairs that BIN_REGIONS regions of
-                // this one's need would hold (the last square of the fullest
-                // region to reserve its range has the largest)
+                // poisons the Exec, with the records that regions of this
+                // one's need would hold (the last square of the fullest region
+                // to reserve its range has the largest)
                 const uint32_t was = atomicCAS(&P.ctr->poison, 0u, P.seq);
                 if (was == 0u || was == P.seq) {
-                    atomicOr(&P.ctr->poison_flags, 2u);
+                    atomicOr(&P.ctr->poison_flags, OVERFLOW_BINS);
                     atomicMax(&P.ctr->poison_pairs, (at + sum) * BIN_REGIONS);
                 }
-                atomicOr(&P.ctr->sticky, 2u);
+                atomicOr(&P.ctr->sticky, OVERFLOW_BINS);
             }
             s_over = over ? 1u : 0u;
         }
@@ -5089,6 +5099,8 @@ struct Arena {
 struct LaunchTrace {
     uint64_t raster_blocks = 0;    // grid of the latest raster kernel
     uint64_t binned = 0, sorted = 0;   // launches k_bin and the tile sort took
+    uint64_t room = 0;             // records or pairs the latest launch had room for
+    uint64_t reruns = 0;           // times the queue ran again after an overflow
 };
 
 // What tells a launch apart when the next frame has it again, and the part of
@@ -5134,7 +5146,9 @@ struct Exec {
     Arena keys[2], vals[2], sort_tmp, tile_list;   // (tile, record) pairs and their sort
     Arena tile_start, tile_end, tile_gen;          // per launch-wide tile: bin range, generation of the range
     uint32_t gen = 0;                              // launch generation stamped into tile_gen
-    float pair_ratio = 4.0f;                       // pairs per triangle a launch is sized for (grows)
+    float pair_ratio = 4.0f;                       // pairs per triangle the tile sort is sized for (grows)
+    uint64_t bin_room = 0;                         // records k_bin's regions are sized for at least (grows)
+    bool bins_off = false;                         // a launch needed more of them than can be addressed
     uint32_t heavy_bin = HEAVY_BIN;                // bins longer than this go to the front of the tile list
     uint32_t grid_div = 1;                         // raster grids: resident blocks / grid_div
     unsigned long long *stat_slots = nullptr;      // 2 x STAT_SLOTS
@@ -5715,7 +5729,7 @@ double expected_part(const Exec &x, const Spread &q)
 bool use_bins(Exec &x, const Sizes &z, uint32_t &slot)
 {
     slot = MEETS_NONE;
-    if (z.bins > BIN_MAX || z.crowded) return false;
+    if (z.bins > BIN_MAX || z.crowded || x.bins_off) return false;
     if (z.scenes > 1u && z.bins > BIN_MANY && z.tri < BIN_SPARSE * z.bins) return false;
     if (z.work <= BIN_MEETS) return true;
     Spread q;
@@ -5761,6 +5775,14 @@ uint32_t scene_bins(const mtgl_dev *d, uint32_t ntri)
     return (uint32_t)((d->tiles_x + t - 1) / t) * (uint32_t)((d->tiles_y + t - 1) / t);
 }
 
+// Squares of a scene in one region at most (bin_region): sixteen rows give each
+// region as many as a row has, the rows left over a sixteenth of each, rounded up.
+uint32_t region_squares(uint32_t cols, uint32_t rows)
+{
+    const uint32_t left = rows % BIN_REGIONS;
+    return rows / BIN_REGIONS * cols + std::min(cols, left * ((cols + BIN_REGIONS - 1u) / BIN_REGIONS));
+}
+
 Sizes scene_sizes(const SceneIn *in, uint32_t n)
 {
     Sizes z;
@@ -5777,7 +5799,8 @@ Sizes scene_sizes(const SceneIn *in, uint32_t n)
         z.crowded |= ntri > BIN_LARGE && ntri > BIN_LARGE_DENSE * (uint64_t)in[i].dev->tiles_x * (uint64_t)in[i].dev->tiles_y;
         z.work += bins * blocks_for(ntri, SETUP_BLOCK);
         z.work_max = std::max<uint64_t>(z.work_max, bins * blocks_for(ntri, SETUP_BLOCK));
-        z.items += HEAVY_SPLIT * side * side * ((bins + BIN_REGIONS - 1) / BIN_REGIONS);
+        const uint32_t cols = (uint32_t)((in[i].dev->tiles_x + side - 1) / side);
+        z.items += HEAVY_SPLIT * side * side * region_squares(cols, (uint32_t)(bins / cols));
         z.tiles += (uint64_t)in[i].dev->tiles_x * (uint64_t)in[i].dev->tiles_y;
         z.cold |= needs_cold(dr->raster);
     }
@@ -6059,12 +6082,14 @@ int prepare_launch(Exec &x, Launch &L, const SceneIn *in, uint32_t n)
     return MTGL_OK;
 }
 
+constexpr uint64_t MAX_PAIRS = 0x7FFFFFFF;   // of a launch
+
 // pairs the arrays of x hold for a launch binned by k_bin or by the tile sort
 uint64_t pairs_room(const Exec &x, bool bins)
 {
     size_t c = x.vals[0].cap;
     if (!bins) c = std::min(std::min(c, x.vals[1].cap), std::min(x.keys[0].cap, x.keys[1].cap));
-    return std::min<uint64_t>(c / 4, 0x7FFFFFFFull);
+    return std::min<uint64_t>(c / 4, MAX_PAIRS);
 }
 
 // K3 of launches k_bin does not take: pair offsets and total (read on the
@@ -6149,32 +6174,33 @@ int tile_sort(Exec &x, Launch &L, bool frozen, uint32_t seq, uint32_t cap, uint3
 }
 
 // The pipeline over the scenes of L, queued on x.stream without waiting for
-// the GPU.  The pair arrays are sized from x.pair_ratio (a frozen run, a
-// replay or one being captured into a graph, allocates nothing and uses the
-// capacity of its sizing run); a launch that needs more pairs, or more clip
-// slots than the pool holds, poisons the Exec with seq (k_bin_scatter) and
-// writes nothing: the host learns of it when it next waits for the stream and
+// the GPU.  The arrays are sized by the launch's triangles and tiles and by
+// what earlier launches needed (exec_grow); a frozen run, a replay or one being
+// captured into a graph, allocates nothing and uses the capacity of its sizing
+// run.  A launch that needs more, or more clip slots than the pool holds,
+// poisons the Exec with seq (k_bin, or k_expand) and writes nothing: the host learns of it when it next waits for the stream and
 // runs the launch again with larger arrays.
 int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
 {
     if (L.ns == 0) return L.unsupported ? MTGL_ERR_UNSUPPORTED : MTGL_OK;
     int rc;
     const uint32_t ttot = L.tri_total, ntiles = L.tiles_total;
-    const double est_pairs = (double)x.pair_ratio * (double)ttot;
     if (!frozen) {
         // k_bin keeps 4 bytes per pair: room for many more pairs than most
         // draws have, so that a context's first draws seldom run twice
-        const double want = L.bins ? std::min(2147483647.0, std::max(est_pairs, 32.0 * ttot) + 4.0 * ntiles + 65536.0)
-                                   : std::min(2147483647.0, est_pairs + 4096.0);
+        const uint64_t room = std::max<uint64_t>(32ull * ttot + 4ull * ntiles + 65536u, x.bin_room);
+        const uint64_t want = L.bins ? std::min<uint64_t>(MAX_PAIRS, room)
+                                     : (uint64_t)std::min((double)MAX_PAIRS, (double)x.pair_ratio * ttot + 4096.0);
         for (int k = 0; k < (L.bins ? 1 : 2); k++) {
             if (!L.bins && (rc = arena_reserve(x, x.keys[k], (size_t)want * 4))) return rc;
             if ((rc = arena_reserve(x, x.vals[k], (size_t)want * 4))) return rc;
         }
         // the estimate, not the arenas' power-of-two size, bounds the tile
         // sort (its grid and histograms scale with it)
-        L.pairs_cap = std::min<uint64_t>(pairs_room(x, L.bins), (uint64_t)want);
+        L.pairs_cap = std::min<uint64_t>(pairs_room(x, L.bins), want);
     }
     const uint32_t cap = (uint32_t)L.pairs_cap;
+    x.trace.room = cap;
     // up to HEAVY_SPLIT items per tile, in one region or in each one's squares
     const uint32_t list_cap = L.bins ? L.region_items : HEAVY_SPLIT * ntiles;
     if ((rc = arena_reserve(x, x.tile_list, (size_t)list_cap * (L.bins ? BIN_REGIONS : 1u) * sizeof(uint4), frozen)))
@@ -6534,16 +6560,29 @@ int execute_scenes(Exec &x, Launch &L, const SceneIn *in, uint32_t n, uint32_t s
     return run_launch(x, L, false, seq);
 }
 
-// After a launch poisoned x (it needed more pairs or clip slots than x
-// held): larger arrays for its next run.  ntri: the launch's triangles.
+// After a launch poisoned x (it needed more pairs, records in a region or clip
+// slots than x held): larger arrays for its next run.  ntri: the launch's
+// triangles.  The tile sort is sized by pairs per triangle, which also bounds
+// its grids, k_bin by the room its fullest region needed sixteen times over:
+// neither sizes the other.
 void exec_grow(Exec &x, const Counters &c, uint32_t ntri)
 {
-    if (c.poison_flags & 1u) x.overflow_cap = std::min<uint32_t>(std::max<uint32_t>(x.overflow_cap * 2u, 4096u), 1u << 26);
-    if (c.poison_flags & 2u) {
+    if (c.poison_flags & OVERFLOW_CLIP) x.overflow_cap = std::min<uint32_t>(std::max<uint32_t>(x.overflow_cap * 2u, 4096u), 1u << 26);
+    if (c.poison_flags & OVERFLOW_BINS) {
+        // (at least doubled, so that a queue of ever larger launches is through
+        // after a few of them)
+        x.bin_room = std::min<uint64_t>(std::max<uint64_t>(2u * x.bin_room, c.poison_pairs + c.poison_pairs / 4u),
+                                        MAX_PAIRS);
+        x.bins_off |= c.poison_pairs > MAX_PAIRS;
+    }
+    if (c.poison_flags & OVERFLOW_PAIRS) {
         const double r = 1.25 * (double)c.poison_pairs / (double)std::max<uint32_t>(ntri, 1u) + 1.0;
         x.pair_ratio = (float)std::max<double>(x.pair_ratio, std::min(r, 2.0e9));
     }
 }
+
+// (the clip pool and the room of k_bin's regions double each time, 14 and 15 times in all)
+constexpr int MAX_RERUNS = 48;
 
 // Reads x's counters back (the stream must have drained) and clears the
 // poison it carries, returning it (0: none).
@@ -6796,7 +6835,7 @@ int batch_build_inner(mtgl_batch *b, int autotune)
         if ((rc = exec_take_poison(x, poison))) return rc;
         saw_meets(x, x.ctr_host->meets);
         if (!poison && !batch_rebins(b)) break;
-        if (attempt >= 16) return MTGL_ERR_OUT_OF_MEMORY;
+        if (attempt >= MAX_RERUNS) return MTGL_ERR_OUT_OF_MEMORY;
         if (poison) exec_grow(x, *x.ctr_host, b->rounds[poison - 1].launch.tri_total);
         ring_release(x);
     }
@@ -7673,7 +7712,8 @@ static int confirm(mtgl_dev *d)
         size_t first = d->ops.size();
         for (size_t i = 0; i < d->ops.size(); i++)
             if (d->ops[i].seq == poison) first = i;
-        if (first == d->ops.size() || attempt >= 16) return MTGL_ERR_OUT_OF_MEMORY;
+        if (first == d->ops.size() || attempt >= MAX_RERUNS) return MTGL_ERR_OUT_OF_MEMORY;
+        x.trace.reruns++;
         exec_grow(x, *x.ctr_host, d->ops[first].ntri);
         d->replaying = true;
         const bool timing = x.timing;
@@ -7707,6 +7747,8 @@ MTGL_API int mtgl_dev_launch_trace(const mtgl_dev *d, uint64_t *out)
     out[0] = t.raster_blocks;
     out[1] = t.binned;
     out[2] = t.sorted;
+    out[3] = t.room;
+    out[4] = t.reruns;
     return MTGL_OK;
 }
 

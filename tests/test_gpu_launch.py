@@ -18,9 +18,9 @@ ALL = E["GL_COLOR_BUFFER_BIT"] | E["GL_DEPTH_BUFFER_BIT"] | E["GL_STENCIL_BUFFER
 def trace(g, ctx):
     fn = g.lib.mtgl_dev_launch_trace
     fn.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint64)]
-    out = (ctypes.c_uint64 * 3)()
+    out = (ctypes.c_uint64 * 5)()
     assert fn(g.device(ctx), out) == 0
-    return dict(zip(("raster_blocks", "binned", "sorted"), out))
+    return dict(zip(("raster_blocks", "binned", "sorted", "room", "reruns"), out))
 
 
 @pytest.mark.parametrize("blend", [False, True])
@@ -154,3 +154,87 @@ def test_batch_rounds_are_binned_by_their_own_spread(mtgl, oracle, rounds, by):
     assert took == by
     for a, b in zip(want, got):
         assert plane_diffs(a, b) == {"color": 0, "depth": 0, "stencil": 0}
+
+
+def _array(g, pos, col):
+    g.glEnableClientState(E["GL_VERTEX_ARRAY"])
+    g.glEnableClientState(E["GL_COLOR_ARRAY"])
+    g.glVertexPointer(3, E["GL_FLOAT"], 0, g.keep(np.ascontiguousarray(pos.reshape(-1, 3), dtype=np.float32)))
+    g.glColorPointer(4, E["GL_FLOAT"], 0, g.keep(np.ascontiguousarray(col, dtype=np.float32)))
+    g.glDrawArrays(E["GL_TRIANGLES"], 0, pos.size // 3)
+
+
+def _bars(W, H, n, upright):
+    """n triangles along one edge of the screen, 16 pixels thick: one column or
+    row of squares holds all their records."""
+    rng = np.random.default_rng(n)
+    p = np.empty((n, 3, 3))
+    long_, thick = (H, 16.0) if upright else (W, 16.0)
+    a = rng.uniform(0, thick, (n, 3))
+    b = np.stack([np.zeros(n), np.full(n, float(long_)), rng.uniform(0, long_, n)], 1)
+    p[..., 0], p[..., 1] = (a, b) if upright else (b, a)
+    p[..., 2] = -rng.uniform(1.0, 90.0, (n, 1))
+    return p, rng.random((3 * n, 4))
+
+
+@pytest.mark.parametrize("fb,upright", [((512, 1024), True), ((480, 1024), True), ((1024, 512), False)])
+def test_regions_fill_alike_and_size_only_k_bin(mtgl, oracle, fb, upright):
+    """A draw whose records all lie in one column or row of squares overflows
+    k_bin's room once; the room it then gets is in proportion to its records,
+    and the next draw that is sorted has room for four pairs a triangle."""
+    W, H = fb
+    n, scattered = 3000, 80_000
+    planes = []
+    for g in (oracle, mtgl):
+        ctx = g.create_context(W, H)
+        try:
+            _ortho(g, W, H)
+            g.glClear(ALL)
+            if g is mtgl:
+                g.stats_reset(ctx)
+            _array(g, *_bars(W, H, n, upright))
+            planes.append(g.read_framebuffer(ctx, W, H))
+            if g is mtgl:
+                t = trace(g, ctx)
+                pairs = g.stats(ctx).bin_pairs
+                first = 32 * n + 4 * ((W + 7) // 8) * ((H + 7) // 8) + 65536
+                assert pairs > first and t["reruns"] == 1 and t["sorted"] == 0
+                assert pairs <= t["room"] <= 1.7 * pairs
+                for _ in range(2):
+                    _array(g, *_triangles(np.random.default_rng(1), W, H, scattered, 2, False))
+                    g.finish(ctx)
+                t = trace(g, ctx)
+                assert t["sorted"] == 1 and t["room"] == 4 * scattered + 4096
+        finally:
+            g.destroy_context(ctx)
+            g.release()
+    assert plane_diffs(*planes) == {"color": 0, "depth": 0, "stencil": 0}
+
+
+@pytest.mark.parametrize("fb", [(136, 72), (40, 600), (600, 40), (544, 32), (32, 544), (545, 33), (8, 8)])
+def test_every_tile_heavy(mtgl, oracle, fb):
+    """Eight work items for every tile: the fullest a region of the list gets,
+    for rows and columns of squares around sixteen."""
+    W, H = fb
+    rng = np.random.default_rng(7)
+    n = 260
+    p = np.empty((n, 3, 3))
+    p[:, 0, :2], p[:, 1, :2], p[:, 2, :2] = (-2 * W, -2 * H), (5 * W, -2 * H), (-2 * W, 5 * H)
+    p[..., 2] = -rng.uniform(1.0, 90.0, (n, 3))
+    col = rng.random((3 * n, 4))
+    planes = []
+    for g in (oracle, mtgl):
+        ctx = g.create_context(W, H)
+        try:
+            _ortho(g, W, H)
+            g.glEnable(E["GL_BLEND"])
+            g.glBlendFunc(E["GL_SRC_ALPHA"], E["GL_ONE_MINUS_SRC_ALPHA"])
+            g.glClear(ALL)
+            _array(g, p, col)
+            planes.append(g.read_framebuffer(ctx, W, H))
+            if g is mtgl:
+                assert trace(g, ctx)["binned"] >= 1
+        finally:
+            g.destroy_context(ctx)
+            g.release()
+    assert plane_diffs(*planes) == {"color": 0, "depth": 0, "stencil": 0}
