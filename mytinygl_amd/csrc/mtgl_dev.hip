@@ -5101,6 +5101,7 @@ struct LaunchTrace {
     uint64_t binned = 0, sorted = 0;   // launches k_bin and the tile sort took
     uint64_t room = 0;             // records or pairs the latest launch had room for
     uint64_t reruns = 0;           // times the queue ran again after an overflow
+    uint64_t regrown = 0;          // times a buffer of triangles or set-up blocks had to grow
 };
 
 // What tells a launch apart when the next frame has it again, and the part of
@@ -5815,22 +5816,26 @@ int reserve_scene_buffers(Exec &x, const Sizes &z, bool bins)
     // record pool: one slot per triangle plus an overflow pool for clipped ones
     if (x.overflow_cap < 4096u) x.overflow_cap = 4096u;
     x.overflow_cap = std::max<uint32_t>(x.overflow_cap, std::min<uint32_t>((uint32_t)(z.tri / 8u), 1u << 24));
-    if ((rc = arena_reserve(x, x.rt, (t + x.overflow_cap) * sizeof(RTri)))) return rc;
-    if (z.cold && (rc = arena_reserve(x, x.rcold, (t + x.overflow_cap) * sizeof(RCold)))) return rc;
-    if ((rc = arena_reserve(x, x.n_rt, t * sizeof(uint32_t)))) return rc;
-    if ((rc = arena_reserve(x, x.rec_base, t * sizeof(uint32_t)))) return rc;
+    auto need = [&](Arena &a, size_t n) {
+        x.trace.regrown += a.ptr && n > a.cap;
+        return arena_reserve(x, a, n);
+    };
+    if ((rc = need(x.rt, (t + x.overflow_cap) * sizeof(RTri)))) return rc;
+    if (z.cold && (rc = need(x.rcold, (t + x.overflow_cap) * sizeof(RCold)))) return rc;
+    if ((rc = need(x.n_rt, t * sizeof(uint32_t)))) return rc;
+    if ((rc = need(x.rec_base, t * sizeof(uint32_t)))) return rc;
     const size_t sb = (size_t)std::max<uint64_t>(z.sblocks, 1u);
     if (bins) {
-        if ((rc = arena_reserve(x, x.tbox, t * sizeof(uint2)))) return rc;
-        return arena_reserve(x, x.blk_box, sb * sizeof(uint2));
+        if ((rc = need(x.tbox, t * sizeof(uint2)))) return rc;
+        return need(x.blk_box, sb * sizeof(uint2));
     }
-    if ((rc = arena_reserve(x, x.box, (t + x.overflow_cap) * sizeof(RBox)))) return rc;
-    if ((rc = arena_reserve(x, x.big_list, t * sizeof(uint32_t)))) return rc;
-    if ((rc = arena_reserve(x, x.blk_kept, sb * sizeof(uint32_t)))) return rc;
-    if ((rc = arena_reserve(x, x.blk_pairs, sb * sizeof(unsigned long long)))) return rc;
-    if ((rc = arena_reserve(x, x.blk_off, sb * sizeof(unsigned long long)))) return rc;
-    if ((rc = arena_reserve(x, x.tri_tiles, (t + 1) * sizeof(unsigned long long)))) return rc;
-    if ((rc = arena_reserve(x, x.pair_base, (t + 1) * sizeof(unsigned long long)))) return rc;
+    if ((rc = need(x.box, (t + x.overflow_cap) * sizeof(RBox)))) return rc;
+    if ((rc = need(x.big_list, t * sizeof(uint32_t)))) return rc;
+    if ((rc = need(x.blk_kept, sb * sizeof(uint32_t)))) return rc;
+    if ((rc = need(x.blk_pairs, sb * sizeof(unsigned long long)))) return rc;
+    if ((rc = need(x.blk_off, sb * sizeof(unsigned long long)))) return rc;
+    if ((rc = need(x.tri_tiles, (t + 1) * sizeof(unsigned long long)))) return rc;
+    if ((rc = need(x.pair_base, (t + 1) * sizeof(unsigned long long)))) return rc;
     return MTGL_OK;
 }
 
@@ -6791,19 +6796,30 @@ void planes_copy(mtgl_batch *b, uint8_t *mem, bool restore)
     }
 }
 
-// The largest round fixes the sizes of the shared buffers up front, so that
-// the sizing run seldom has to grow them between rounds.
+// The largest rounds that k_bin and the tile sort are about to take fix the
+// sizes of the buffers that rounds share, so that the sizing run seldom has to
+// grow them between rounds.
 int batch_reserve(mtgl_batch *b)
 {
-    Sizes m;
+    Exec &x = b->ex;
+    Sizes most[2];
     for (BatchRound &R : b->rounds) {
         const Sizes z = scene_sizes(R.scenes.data(), (uint32_t)R.scenes.size());
+        if (z.tri > 0x0FFFFFFFull) return MTGL_ERR_OUT_OF_MEMORY;
+        if (z.tri == 0) continue;
+        uint32_t slot;
+        Sizes &m = most[use_bins(x, z, slot) ? 1 : 0];
         m.tri = std::max(m.tri, z.tri);
-        m.tiles = std::max(m.tiles, z.tiles);
+        m.sblocks = std::max(m.sblocks, z.sblocks);
         m.cold |= z.cold;
     }
-    if (m.tri > 0x0FFFFFFFull) return MTGL_ERR_OUT_OF_MEMORY;
-    return m.tri ? reserve_scene_buffers(b->ex, m, true) : MTGL_OK;
+    x.nqueued = 0;   // (asked, not queued)
+    // (the larger first: its triangles size the clip pool that both hold)
+    const int first = most[1].tri > most[0].tri ? 1 : 0;
+    int rc;
+    for (int bins : {first, 1 - first})
+        if (most[bins].tri && (rc = reserve_scene_buffers(x, most[bins], bins != 0))) return rc;
+    return MTGL_OK;
 }
 
 // Whether some round would now be binned the other way than it was.
@@ -6824,11 +6840,11 @@ int batch_build_inner(mtgl_batch *b, int autotune)
 {
     Exec &x = b->ex;
     int rc;
-    if ((rc = batch_reserve(b))) return rc;
     // sizing runs: every round in order, until none needs larger arrays than
     // the earlier rounds grew them to, and each is binned as its own count of
     // met squares asks for (the replays' rounds stay as this leaves them)
     for (int attempt = 0;; attempt++) {
+        if ((rc = batch_reserve(b))) return rc;
         if ((rc = batch_run(b, false))) return rc;
         HIPC(hipStreamSynchronize(x.stream));
         uint32_t poison = 0;
@@ -7916,14 +7932,15 @@ MTGL_API int mtgl_batch_stats_reset(mtgl_batch *b)
     return exec_stats_reset(b->ex);
 }
 
-// The rounds of the captured replay that k_bin and the tile sort take (no
-// header declares it: for tests).
+// The rounds of the captured replay that k_bin and the tile sort take, and how
+// often the build had to grow a buffer of theirs (no header declares it: for tests).
 MTGL_API int mtgl_batch_launch_trace(const mtgl_batch *b, uint64_t *out)
 {
     if (!b || !out) return MTGL_ERR_INVALID;
     out[0] = out[1] = 0;
     for (const BatchRound &R : b->rounds)
         if (R.launch.ns) out[R.launch.bins ? 0 : 1]++;
+    out[2] = b->ex.trace.regrown;
     return MTGL_OK;
 }
 

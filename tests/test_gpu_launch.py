@@ -128,7 +128,7 @@ def _batch(g, W, H, n, rounds):
         if g.kind == "mtgl":
             fn = g.lib.mtgl_batch_launch_trace
             fn.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint64)]
-            out = (ctypes.c_uint64 * 2)()
+            out = (ctypes.c_uint64 * 3)()
             assert fn(b.h, out) == 0
             by = tuple(out)
         b.launch()
@@ -151,7 +151,7 @@ def test_batch_rounds_are_binned_by_their_own_spread(mtgl, oracle, rounds, by):
     W, H, n = 1024, 600, 2
     want, _ = _batch(oracle, W, H, n, rounds)
     got, took = _batch(mtgl, W, H, n, rounds)
-    assert took == by
+    assert took[:2] == by
     for a, b in zip(want, got):
         assert plane_diffs(a, b) == {"color": 0, "depth": 0, "stencil": 0}
 
