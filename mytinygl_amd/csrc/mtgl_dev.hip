@@ -5120,8 +5120,8 @@ struct Exec {
     // blocks at once: depth<stencil>, depth<no stencil>, general, then the
     // depth kernels at four waves per SIMD (launches of several scenes)
     uint32_t resident[9] = {256, 256, 256, 256, 256, 256, 256, 256, 256};
-    Counters *ctr = nullptr;                       // device
-    Counters *ctr_host = nullptr;                  // pinned mirror for readback
+    Counters *ctr = nullptr;                       // device (regions, sums and stat_slots are of its block)
+    Counters *ctr_host = nullptr;                  // pinned mirror for readback (report is of its block)
     uint32_t *report = nullptr;                    // pinned: the poison the latest read reported
     uint8_t *pinned = nullptr;                     // staging for uploads that wait for their copy
     size_t pinned_cap = 0;
@@ -5499,18 +5499,21 @@ int exec_init(Exec &x, int device)
         x.resident[k] = std::min<uint32_t>((uint32_t)nb * (uint32_t)x.cu_count, STAT_SLOTS);
     }
     HIPC(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
-    HIPC(hipMalloc((void **)&x.ctr, sizeof(Counters)));
-    HIPC(hipMalloc((void **)&x.stat_slots, 2 * STAT_SLOTS * sizeof(unsigned long long)));
-    HIPC(hipMalloc((void **)&x.regions, BIN_REGIONS * sizeof(RegionCounters)));
-    HIPC(hipMemsetAsync(x.regions, 0, BIN_REGIONS * sizeof(RegionCounters), x.stream));
-    HIPC(hipMalloc((void **)&x.sums, 128 * sizeof(uint32_t)));
-    HIPC(hipMemsetAsync(x.sums, 0, 128 * sizeof(uint32_t), x.stream));
-    HIPC(hipHostMalloc((void **)&x.ctr_host, sizeof(Counters), hipHostMallocDefault));
-    HIPC(hipHostMalloc((void **)&x.report, 256, hipHostMallocDefault));
+    // the counters in one block of device memory, cleared at once, and the
+    // host's copy and report in one of pinned memory (each allocation of which
+    // takes about 35 us)
+    const size_t at_regions = up256(sizeof(Counters)), at_sums = at_regions + BIN_REGIONS * sizeof(RegionCounters);
+    const size_t at_stats = up256(at_sums + 128 * sizeof(uint32_t));
+    const size_t all = at_stats + 2 * STAT_SLOTS * sizeof(unsigned long long);
+    HIPC(hipMalloc((void **)&x.ctr, all));
+    x.regions = reinterpret_cast<RegionCounters *>((uint8_t *)x.ctr + at_regions);
+    x.sums = reinterpret_cast<uint32_t *>((uint8_t *)x.ctr + at_sums);
+    x.stat_slots = reinterpret_cast<unsigned long long *>((uint8_t *)x.ctr + at_stats);
+    HIPC(hipHostMalloc((void **)&x.ctr_host, up256(sizeof(Counters)) + 256, hipHostMallocDefault));
+    x.report = reinterpret_cast<uint32_t *>((uint8_t *)x.ctr_host + up256(sizeof(Counters)));
     *x.report = 0u;
     HIPC(hipEventCreateWithFlags(&x.upload_done, hipEventDisableTiming));
-    HIPC(hipMemsetAsync(x.stat_slots, 0, 2 * STAT_SLOTS * sizeof(unsigned long long), x.stream));
-    HIPC(hipMemsetAsync(x.ctr, 0, sizeof(Counters), x.stream));
+    HIPC(hipMemsetAsync(x.ctr, 0, all, x.stream));
     HIPC(hipStreamSynchronize(x.stream));
     return MTGL_OK;
 }
@@ -5529,12 +5532,8 @@ void exec_free(Exec &x)
     for (hipEvent_t e : x.free_events) (void)hipEventDestroy(e);
     x.pending_events.clear();
     x.free_events.clear();
-    if (x.ctr) (void)hipFree(x.ctr);
-    if (x.stat_slots) (void)hipFree(x.stat_slots);
-    if (x.sums) (void)hipFree(x.sums);
-    if (x.regions) (void)hipFree(x.regions);
-    if (x.ctr_host) (void)hipHostFree(x.ctr_host);
-    if (x.report) (void)hipHostFree(x.report);
+    if (x.ctr) (void)hipFree(x.ctr);             // (with regions, sums and stat_slots)
+    if (x.ctr_host) (void)hipHostFree(x.ctr_host);   // (with report)
     if (x.pinned) (void)hipHostFree(x.pinned);
     for (auto &b : x.ring) (void)hipHostFree(b.first);
     x.ring.clear();
