@@ -6,6 +6,7 @@ the CPU restatement of the pipeline) and oracle/_ref/libmtgl_ref.so (the
 reference renderer compiled strict from its own sources, present where it was
 built).
 """
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -67,3 +68,12 @@ def color_histogram(a, b):
     cb = b.view(np.uint8).reshape(b.shape + (4,)).astype(np.int16)
     mx = np.abs(ca - cb).max(-1)
     return np.bincount(mx.reshape(-1), minlength=256)
+
+
+def trace(g, ctx):
+    """How the launches of a context of libmtgl.so ran."""
+    fn = g.lib.mtgl_dev_launch_trace
+    fn.argtypes = [C.c_void_p, C.POINTER(C.c_uint64)]
+    out = (C.c_uint64 * 5)()
+    assert fn(g.device(ctx), out) == 0
+    return dict(zip(("raster_blocks", "binned", "sorted", "room", "reruns"), out))

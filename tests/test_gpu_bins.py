@@ -1,7 +1,7 @@
 """The two ways a launch's triangles reach its tiles: k_bin, or the sort by
 tile.  Which one a launch takes depends on its sizes and on how far the
-triangles of a set-up block lay apart in the launch before, so both must leave
-the same pixels.  The scenes sit at the edges: one triangle and one tile,
+triangles of a set-up block lay apart in the same draw of the frame before, so
+both must leave the same pixels.  The scenes sit at the edges: one triangle and one tile,
 partial squares of tiles, squares whose list is longer than a window, a
 framebuffer dense enough for each square size, triangles clipped into several
 records, and draws whose triangles lie together and anywhere in turn, with a
@@ -9,7 +9,7 @@ read between them (which is when the choice moves)."""
 import numpy as np
 import pytest
 
-from conftest import plane_diffs
+from conftest import plane_diffs, trace
 from mytinygl_amd.gl import ENUMS as E
 from mytinygl_amd import scenes as S
 
@@ -73,6 +73,12 @@ def test_scattered_and_together_in_turn(mtgl, oracle, fb, n, size, blend):
                     g.glClear(ALL)
             st = g.stats(ctx)
             out.append((st.fragments, st.triangles_raster))
+            if g is mtgl:
+                # large draws go as the last count asks: the second (after
+                # scattered triangles) and the fifth are sorted
+                t = trace(g, ctx)
+                assert t["binned"] + t["sorted"] == 5 + t["reruns"]
+                assert t["sorted"] >= 2 and t["binned"] >= 3 if n >= 20_000 else t["sorted"] == 0
         finally:
             g.destroy_context(ctx)
             g.release()
@@ -88,5 +94,8 @@ def test_dense_sphere(mtgl, oracle, grid, side):
     tiles, squares of one tile; 290: 168,200 over 1,024, past the limit)."""
     def scene(g, W, H, seed):
         S.draw_textured_sphere(g, S.setup_textured_sphere(g, W, H, seed, grid, 64))
+        if g is mtgl:
+            t = trace(g, g.gl_get_current_context())
+            assert (t["binned"], t["sorted"]) == ((0, 1) if grid == 290 else (1, 0))
     (a, ea), (b, eb) = S.render(oracle, scene, side, side, 3), S.render(mtgl, scene, side, side, 3)
     assert ea == eb and plane_diffs(a, b) == {"color": 0, "depth": 0, "stencil": 0}

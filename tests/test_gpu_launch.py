@@ -6,21 +6,13 @@ import ctypes
 import numpy as np
 import pytest
 
-from conftest import plane_diffs
+from conftest import plane_diffs, trace
 from mytinygl_amd.gl import ENUMS as E
 from test_gpu_bins import _ortho, _triangles
 
 pytestmark = pytest.mark.gpu
 
 ALL = E["GL_COLOR_BUFFER_BIT"] | E["GL_DEPTH_BUFFER_BIT"] | E["GL_STENCIL_BUFFER_BIT"]
-
-
-def trace(g, ctx):
-    fn = g.lib.mtgl_dev_launch_trace
-    fn.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint64)]
-    out = (ctypes.c_uint64 * 5)()
-    assert fn(g.device(ctx), out) == 0
-    return dict(zip(("raster_blocks", "binned", "sorted", "room", "reruns"), out))
 
 
 @pytest.mark.parametrize("blend", [False, True])
