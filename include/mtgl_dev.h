@@ -207,7 +207,8 @@ typedef struct {
     uint64_t frag_bytes;
     uint64_t triangles_in;      /* triangles assembled */
     uint64_t triangles_raster;  /* fan triangles reaching setup */
-    uint64_t bin_pairs;         /* (tile, triangle) pairs binned */
+    uint64_t bin_pairs;         /* (tile, triangle) pairs binned: tiles a triangle can cover, or, in draws
+                                   that are sorted by tile, all tiles of a box of more than 64 */
     uint64_t draws;
     double   raster_ms;         /* summed duration of the fragment kernel launches
                                    (the draws' fragment stages and glDrawPixels),

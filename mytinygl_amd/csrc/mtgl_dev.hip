@@ -2180,7 +2180,7 @@ __global__ void __launch_bounds__(BINS_THREADS) k_tile_bins(const uint32_t *keys
 // scenes with many triangles per tile, fewer (bin_side).  It walks the scene's
 // set-up blocks in order, then the triangles of those whose tile bounds meet
 // the square, and lists the records that do (s_list, in submission order).  Per 64 listed records a
-// wave, one record per lane, tests the 64 tiles exactly (box_tile_mask's
+// wave, one record per lane, tests the square's tiles exactly (box_tile_mask's
 // argument: a tile whose best corner fails an edge holds no covered pixel)
 // and leaves, per tile, the mask of the records it can hold; the masks'
 // running counts place each tile's records, in order, in one range of vals
@@ -2508,8 +2508,8 @@ __global__ void __launch_bounds__(BIN_THREADS) k_bin(BinParams P)
 
 
 // per-launch counters at zero: k_launch_begin before the point / line path,
-// and before a tile launch when the previous one stopped before k_expand
-// (which, with k_setup, otherwise leaves them at zero)
+// and before a tile launch when the previous one stopped on the way (k_expand,
+// or after k_bin end_binning, with k_setup otherwise leave them at zero)
 __device__ __forceinline__ void reset_counters(Counters *ctr)
 {
     ctr->npairs = 0;
@@ -5117,8 +5117,9 @@ struct Spread {
 struct Exec {
     hipStream_t stream = nullptr;
     int cu_count = 256;
-    // blocks at once: depth<stencil>, depth<no stencil>, general, then the
-    // depth kernels at four waves per SIMD (launches of several scenes)
+    // blocks at once: depth<stencil>, depth<no stencil>, general, the depth
+    // kernels at four waves per SIMD (launches of several scenes), general for
+    // GEN_PLAIN, the depth kernels of SIMPLE launches, general for GEN_SIMPLE
     uint32_t resident[9] = {256, 256, 256, 256, 256, 256, 256, 256, 256};
     Counters *ctr = nullptr;                       // device (regions, sums and stat_slots are of its block)
     Counters *ctr_host = nullptr;                  // pinned mirror for readback (report is of its block)
@@ -5156,7 +5157,8 @@ struct Exec {
     std::vector<unsigned long long> stat_host;
     mtgl_dev_stats stats = {};
     bool timing = false;
-    bool ctr_clean = false;                        // per-launch counters at zero (k_expand's block 0 leaves them so)
+    bool ctr_clean = false;                        // per-launch counters at zero (k_expand's block 0 leaves them so,
+                                                   // or after k_bin the first raster kernel's: end_binning)
     uint32_t timing_every = 1;     // time one fragment-stage launch in this many
     uint32_t timing_count = 0;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pending_events;
@@ -5620,47 +5622,6 @@ struct SceneIn {
     mtgl_dev *dev;
     const mtgl_draw *dr;
 };
-
-// Vertex work of a draw.  An indexed draw whose arrays address fewer vertices
-// than it has indices transforms each addressed vertex once: slot k is vertex
-// base + k for k < n - 1, and slot n - 1 stands for every index no array
-// addresses (each array fetch of such an index reads the same defaults).
-// Setup then finds a stream position's record through its index.  Other
-// draws transform one vertex per stream position.
-struct VSlots {
-    uint32_t n;
-    int32_t base;
-    bool unique;
-};
-
-VSlots vertex_slots(const mtgl_dev *d, const mtgl_draw *dr)
-{
-    VSlots r = {dr->count, 0, false};
-    if (dr->index_type == 0 || (dr->n_vstates > 1 && dr->state_index.enabled)) return r;
-    // the indices each array reads in range (the bounds test of fetch) and their hull
-    const uint8_t marker = 0;
-    const mtgl_array *arrs[4] = {&dr->position, &dr->color, &dr->texcoord, &dr->normal};
-    int64_t lo = INT64_MAX, hi = -1;
-    for (int k = 0; k < 4; k++) {
-        if (k > 0 && !arrs[k]->enabled) continue;
-        const DArr a = resolve(d, *arrs[k], &marker, dr->staged_bytes);
-        if (!a.src || a.stride <= 0) continue;
-        const int64_t elem = (int64_t)a.comps * (a.type == GL_FLOAT ? 4 : 1);
-        const int64_t room = a.size - elem - a.offset;   // at + elem <= size
-        if (room < 0) continue;
-        const int64_t ilo = a.offset >= 0 ? 0 : (-a.offset + a.stride - 1) / a.stride;
-        const int64_t ihi = std::min<int64_t>(room / a.stride, 0x7FFFFFFF);
-        if (ilo > ihi) continue;
-        lo = std::min(lo, ilo);
-        hi = std::max(hi, ihi);
-    }
-    const int64_t n = hi < lo ? 1 : hi - lo + 2;
-    if (n > (int64_t)dr->count) return r;
-    r.n = (uint32_t)n;
-    r.base = hi < lo ? 0 : (int32_t)lo;
-    r.unique = true;
-    return r;
-}
 
 // Triangle and tile totals of a set of scenes and the buffers they need.
 struct Sizes {
@@ -6182,8 +6143,9 @@ int tile_sort(Exec &x, Launch &L, bool frozen, uint32_t seq, uint32_t cap, uint3
 // what earlier launches needed (exec_grow); a frozen run, a replay or one being
 // captured into a graph, allocates nothing and uses the capacity of its sizing
 // run.  A launch that needs more, or more clip slots than the pool holds,
-// poisons the Exec with seq (k_bin, or k_expand) and writes nothing: the host learns of it when it next waits for the stream and
-// runs the launch again with larger arrays.
+// poisons the Exec with seq (k_bin, or k_expand) and writes nothing: the host
+// learns of it when it next waits for the stream and runs the launch again with
+// larger arrays.
 int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
 {
     if (L.ns == 0) return L.unsupported ? MTGL_ERR_UNSUPPORTED : MTGL_OK;
@@ -6233,8 +6195,8 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
 
     // ---- K2: set-up, with the vertex transform
     unsigned long long *blk_pairs = as<unsigned long long>(x.blk_pairs);
-    // k_setup and k_expand reset the per-launch counters as they go; a
-    // launch that stopped between them leaves them to k_launch_begin
+    // k_setup and k_expand or end_binning reset the per-launch counters as they
+    // go; a launch that stopped between them leaves them to k_launch_begin
     if (!x.ctr_clean) hipLaunchKernelGGL(k_launch_begin, dim3(1), dim3(64), 0, x.stream, x.ctr);
     x.ctr_clean = false;
     // a wave per corner while the blocks leave SIMDs idle
@@ -7566,7 +7528,8 @@ MTGL_API int mtgl_dev_draw(mtgl_dev *d, const mtgl_draw *dr)
 
 static int launch_pixels(mtgl_dev *d, const mtgl_pixels &px, uint64_t bytes);
 
-// the launch both glDrawPixels entry points share: src holds the image in HBM
+// the launch both glDrawPixels entry points share; src: the image in HBM, or a
+// staged RGBA image in the ring (launch_pixels)
 static int draw_pixels_kernel(mtgl_dev *d, const mtgl_pixels *p, const uint8_t *src, uint64_t n, bool timed)
 {
     Exec &x = d->ex;
