@@ -40,6 +40,7 @@
 #include <algorithm>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -277,7 +278,7 @@ struct RasterParams {
     uint32_t list_cap;             // items one region of the list holds (HEAVY_SPLIT per tile)
     const RegionCounters *regions;
     uint32_t *kept, *meets;        // k_setup's 64 partial counts, for the first kernel of the stage (kept: only after
-                                   // k_bin), else null
+                                   // k_bin; meets: then or when they were counted), else null
     unsigned long long *stats;     // per block: fragments, algorithmic bytes (summed when read)
     Counters *ctr;
 };
@@ -1170,10 +1171,13 @@ __device__ __forceinline__ uint32_t dpp_wave_minmax_u16x2(uint32_t v)
 // each triangle's tile bounds (tbox) and their union per block (blk_box); the
 // tile masks are then k_bin's, and only the launches of the tile sort write a
 // box and a pair count per triangle and the counts per block.  sums: 64
-// partial counts of the kept fan triangles (BIN), then 64 of the squares of
-// bin_side tiles that the blocks' bounds meet, which tell the host how far a
-// block's triangles lie apart (use_bins).
-template <bool MULTI, int NW, bool BIN>
+// partial counts of the kept fan triangles (BIN), then, with COUNT, 64 of the
+// squares of bin_side tiles that the blocks' bounds meet, which tell the host
+// how far a block's triangles lie apart (use_bins).  Replays and launches whose
+// way does not hang on it run without COUNT: the bounds held to the end cost
+// the 512-scene batch's sorted set-up 714 us, 679 without them; a wave per
+// corner takes 40,000 scattered triangles' from 45.5 to 41.8.
+template <bool MULTI, int NW, bool BIN, bool COUNT>
 __global__ void __launch_bounds__(NW * SETUP_BLOCK) k_setup(const SetupParams *Ss, const VertexParams *Vs,
                                                             const uint32_t *block_pre, const uint32_t *block_scene,
                                                             uint32_t nscenes, uint32_t *blk_kept,
@@ -1270,7 +1274,7 @@ __global__ void __launch_bounds__(NW * SETUP_BLOCK) k_setup(const SetupParams *S
         }
     }
     const uint32_t kept = (uint32_t)__builtin_amdgcn_readlane((int)dpp_incl_scan(nout), 63);
-    {
+    if (BIN || COUNT) {
         const uint32_t lo = nout ? (uint32_t)tb.x0 | ((uint32_t)tb.y0 << 16) : TBOX_NONE_X;
         const uint32_t hi = nout ? (uint32_t)tb.x1 | ((uint32_t)tb.y1 << 16) : TBOX_NONE_Y;
         if (BIN && act) {
@@ -1285,10 +1289,12 @@ __global__ void __launch_bounds__(NW * SETUP_BLOCK) k_setup(const SetupParams *S
             if (BIN) blk_box[blockIdx.x] = make_uint2(blo, bhi);
             if (kept) {
                 // (64 addresses: no long queue at any of them)
-                const uint32_t side = P.bin_side;
-                const uint32_t cols = (bhi & 0xFFFFu) / side - (blo & 0xFFFFu) / side + 1u;
-                const uint32_t rows = (bhi >> 16) / side - (blo >> 16) / side + 1u;
-                atomicAdd(sums + 64u + (blockIdx.x & 63u), cols * rows);
+                if (COUNT) {
+                    const uint32_t side = P.bin_side;
+                    const uint32_t cols = (bhi & 0xFFFFu) / side - (blo & 0xFFFFu) / side + 1u;
+                    const uint32_t rows = (bhi >> 16) / side - (blo >> 16) / side + 1u;
+                    atomicAdd(sums + 64u + (blockIdx.x & 63u), cols * rows);
+                }
                 if (BIN) atomicAdd(sums + (blockIdx.x & 63u), kept);
             }
         }
@@ -6206,16 +6212,21 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
                            L.smap, L.ns, as<uint32_t>(x.blk_kept), blk_pairs, as<uint2>(x.blk_box), x.sums, x.regions,
                            L.ns == 1u ? L.rs1 : nullptr, L.ns == 1u ? L.vs1 : nullptr);
     };
-    if (!L.bins) {
-        if (L.multi_vs) setup_kernel(k_setup<true, 1, false>, 1);
-        else setup_kernel(k_setup<false, 1, false>, 1);
-    } else if (L.multi_vs) {
-        if (split) setup_kernel(k_setup<true, 3, true>, 3);
-        else setup_kernel(k_setup<true, 1, true>, 1);
-    } else {
-        if (split) setup_kernel(k_setup<false, 3, true>, 3);
-        else setup_kernel(k_setup<false, 1, true>, 1);
-    }
+    const bool count = !frozen && L.meets_slot < MEETS_SLOTS;
+    auto setup = [&](auto multi, auto bin, auto cnt) {
+        if (split) setup_kernel(k_setup<multi.value, 3, bin.value, cnt.value>, 3);
+        else setup_kernel(k_setup<multi.value, 1, bin.value, cnt.value>, 1);
+    };
+    auto with_count = [&](auto multi, auto bin) {
+        if (count) setup(multi, bin, std::true_type());
+        else setup(multi, bin, std::false_type());
+    };
+    auto with_bins = [&](auto multi) {
+        if (L.bins) with_count(multi, std::true_type());
+        else with_count(multi, std::false_type());
+    };
+    if (L.multi_vs) with_bins(std::true_type());
+    else with_bins(std::false_type());
     HIPC(hipGetLastError());
 
     // ---- K3: every tile's records in submission order and the work list
@@ -6270,8 +6281,8 @@ int run_launch(Exec &x, Launch &L, bool frozen, uint32_t seq)
     rp.regions = x.regions;
     rp.ctr = x.ctr;
     rp.kept = L.bins ? x.sums : nullptr;
-    rp.meets = x.sums + 64;
-    rp.meets_slot = frozen ? MEETS_NONE : L.meets_slot;
+    rp.meets = L.bins || count ? x.sums + 64 : nullptr;
+    rp.meets_slot = count ? L.meets_slot : MEETS_NONE;
     rp.stats = x.stat_slots;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     if (x.timing && !frozen && x.timing_count++ % x.timing_every == 0u) (void)take_event_pair(x, ev0, ev1);
