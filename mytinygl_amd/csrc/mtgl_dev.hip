@@ -6560,6 +6560,7 @@ void exec_grow(Exec &x, const Counters &c, uint32_t ntri)
 
 // (the clip pool and the room of k_bin's regions double each time, 14 and 15 times in all)
 constexpr int MAX_RERUNS = 48;
+constexpr int MAX_REBINS = 3;   // sizing runs of a batch for another way of binning
 
 // Reads x's counters back (the stream must have drained) and clears the
 // poison it carries, returning it (0: none).
@@ -6815,14 +6816,15 @@ int batch_build_inner(mtgl_batch *b, int autotune)
     // sizing runs: every round in order, until none needs larger arrays than
     // the earlier rounds grew them to, and each is binned as its own count of
     // met squares asks for (the replays' rounds stay as this leaves them)
-    for (int attempt = 0;; attempt++) {
+    for (int attempt = 0, rebinned = 0;; attempt++) {
         if ((rc = batch_reserve(b))) return rc;
         if ((rc = batch_run(b, false))) return rc;
         HIPC(hipStreamSynchronize(x.stream));
         uint32_t poison = 0;
         if ((rc = exec_take_poison(x, poison))) return rc;
         saw_meets(x, x.ctr_host->meets);
-        if (!poison && !batch_rebins(b)) break;
+        // (a choice that would not settle must not fail the build: either way is right)
+        if (!poison && (rebinned++ >= MAX_REBINS || !batch_rebins(b))) break;
         if (attempt >= MAX_RERUNS) return MTGL_ERR_OUT_OF_MEMORY;
         if (poison) exec_grow(x, *x.ctr_host, b->rounds[poison - 1].launch.tri_total);
         ring_release(x);
