@@ -230,3 +230,38 @@ def test_every_tile_heavy(mtgl, oracle, fb):
             g.destroy_context(ctx)
             g.release()
     assert plane_diffs(*planes) == {"color": 0, "depth": 0, "stencil": 0}
+
+
+def test_sorted_draw_of_several_vertex_states(mtgl, oracle):
+    """A draw whose material changes between vertices, binned and then sorted
+    (set-up's variants that read the states from memory), lit, scattered, and
+    with triangles past the near and far planes."""
+    W, H, n = 1920, 1080, 7_000
+    pos, col = _triangles(np.random.default_rng(5), W, H, n, 9, False)
+    pos, col = pos.tolist(), col.tolist()
+    out = []
+    for g in (oracle, mtgl):
+        ctx = g.create_context(W, H)
+        try:
+            _ortho(g, W, H)
+            g.glEnable(E["GL_LIGHTING"])
+            g.glEnable(E["GL_LIGHT0"])
+            g.glNormal3f(0.0, 0.0, 1.0)
+            for _ in range(2):
+                g.glClear(ALL)
+                g.glBegin(E["GL_TRIANGLES"])
+                for k, (p, c) in enumerate(zip(pos, col)):
+                    if k % 1000 == 1:
+                        g.glMaterialfv(E["GL_FRONT_AND_BACK"], E["GL_DIFFUSE"], g.fv(*c))
+                    g.glVertex3f(*p)
+                g.glEnd()
+                out.append(g.read_framebuffer(ctx, W, H))
+            if g is mtgl:
+                t = trace(g, ctx)
+                assert t["binned"] >= 1 and t["sorted"] >= 1
+        finally:
+            g.destroy_context(ctx)
+            g.release()
+    for a, b in zip(out[:2], out[2:]):
+        assert plane_diffs(a, b) == {"color": 0, "depth": 0, "stencil": 0}
+    assert (out[0][0] != out[0][0][0, 0]).sum() > W * H // 50
