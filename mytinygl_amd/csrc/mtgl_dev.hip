@@ -7724,6 +7724,7 @@ static int confirm(mtgl_dev *d)
         x.timing = timing;
         d->replaying = false;
         if (rc) return rc;
+        d->last.gen = x.gen;   // (the latest draw ran again last: a capture reads its tiles' new stamps)
     }
     d->ops.clear();
     ring_release(x);

@@ -9,10 +9,13 @@ grows the arrays and runs the logged clears and draws again from that launch
 on.  These frames make launches of a fresh context overflow all three ways
 (the room of k_bin's regions, the tile sort's pairs, the clip pool), between
 other clears and draws, and must equal the oracle's frames."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from conftest import color_histogram, plane_diffs, trace
+from mytinygl_amd import diff as D
 from mytinygl_amd import scenes as S
 from mytinygl_amd.gl import ENUMS as E
 from test_gpu_bins import _ortho, _triangles
@@ -151,3 +154,33 @@ def test_statistics_count_each_launch_once(mtgl, oracle):
             g.release()
     print("oracle", out[0], "device", out[1])
     assert out[0] == out[1]
+
+
+def test_capture_of_a_draw_that_ran_again(mtgl, oracle):
+    """A differentiable capture of a draw that overflowed: the view is the one
+    its second run left, not an empty one."""
+    W = H = 512
+    P = D.diff_params(grid=2, tex_size=16, views=1)
+    P = dict(P, idx=np.ascontiguousarray(np.tile(P["idx"], 300)))   # 2,400 triangles of about 100 tiles
+    tex8, _ = D.quantise(P["tex"])
+    got = []
+    for g in (oracle, mtgl):
+        D._bind(g.lib)
+        h = C.c_void_p()
+        assert g.lib.mtgl_diff_create(len(P["verts"]), 16, 16, C.byref(h)) == 0
+        ctx = g.create_context(W, H)
+        try:
+            assert g.lib.mtgl_diff_arm(g.device(ctx)) == 0
+            D.draw_view(g, P, 0, W, H, tex8)
+            assert g.lib.mtgl_diff_add_view(h.value, g.device(ctx)) == 0
+            px = np.empty(W * H, D.GPX_DTYPE)
+            assert g.lib.mtgl_diff_gbuffer(h.value, 0, px.ctypes.data) == 0
+            got.append(px)
+            if g is mtgl:
+                assert trace(g, ctx)["reruns"] == 1
+        finally:
+            g.lib.mtgl_diff_destroy(h.value)
+            g.destroy_context(ctx)
+            g.release()
+    assert (got[0]["tri"] >= 0).sum() > 10_000
+    assert got[0].tobytes() == got[1].tobytes()
